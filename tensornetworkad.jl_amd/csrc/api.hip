@@ -232,6 +232,7 @@ void run_ctmrg(tnad_ctx* ctx, tnad_tape& t, const double* C0, const double* T0, 
   const int nk = partial ? chi : n;
   double rest = std::numeric_limits<double>::infinity(), rest_err = 0.0;
   double oldrest = rest, oldrest_err = 0.0;
+  EigPlan plan;
   // StopFunction(oldvals, -1, tol, maxit) (src/ctmrg.jl:114): the counter starts at -1 and the test runs on
   // the initial state too, so at most maxit + 1 steps are taken and maxit = 0 still takes one
   int counter = -1;
@@ -278,6 +279,7 @@ void run_ctmrg(tnad_ctx* ctx, tnad_tape& t, const double* C0, const double* T0, 
       tp = t.steps.back().get();
     }
     StepState ss;
+    ss.plan = plan;
     double* X_keep = nullptr;
     const bool warm = o.eig_warm && n > JACOBI_MAX;
     if (warm && !tp) {
@@ -289,6 +291,7 @@ void run_ctmrg(tnad_ctx* ctx, tnad_tape& t, const double* C0, const double* T0, 
     if (warm) X0 = tp ? tp->X.as<double>() : Xprev.as<double>();
     rest = ss.rest;
     rest_err = ss.rest_err;
+    plan = ss.plan;
     std::swap(Ca, Cb);
     std::swap(Ta, Tb);
     iters += 1;

@@ -39,8 +39,17 @@ struct StepOpts {
   double eig_tol_low = 1e-13; // the same for steps at a lower contraction precision
 };
 
+// where the subspace iteration of a similar matrix converged (the previous CTMRG step's corner matrix): the
+// products it took, the kept residual there and its ratio per product.  Only places the first Rayleigh-Ritz
+// step; convergence is always decided by the residual measured there.
+struct EigPlan {
+  int products = 0;
+  double resid = 0.0, rate = 0.0;
+};
+
 struct StepState {
   int k = 0;
+  EigPlan plan;   // in: the previous step's (or none); out: this step's
   int eig_iters = 0;
   double eig_resid = 0.0;
   // n > 192 only: norm of the singular values beyond the chi kept ones, relative to s[1]
@@ -64,12 +73,12 @@ struct EigWork {
 };
 
 // Top-k eigenpairs (by |lambda|) of the symmetric n x n FP64 matrix A.
-// n <= 192: full Jacobi (k = n).  Otherwise block subspace iteration with
-// Rayleigh-Ritz and CholeskyQR orthonormalisation (one pass, CholeskyQR2 or shifted CholeskyQR3 as the
-// block needs), optionally warm-started from X0.
+// n <= 192: the full spectrum by divide and conquer (k = n).  Otherwise block subspace iteration with CholeskyQR
+// orthonormalisation (one pass, CholeskyQR2 or shifted CholeskyQR3 as the block needs) and Rayleigh-Ritz where
+// the residual is expected to have converged, optionally warm-started from X0.
 // Outputs X (n x k), AX = A X, theta (k).  Returns k.
 int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, int maxit, double tol,
-             double* X, double* AX, double* theta, EigStats* st);
+             double* X, double* AX, double* theta, EigStats* st, EigPlan* plan = nullptr);
 
 // Subspace block of a step: n (full spectrum) for n <= 192; else the chi kept columns plus a guard of
 // 1.25 chi (2.25 chi in all), or eig_block when set.  The guard sets the convergence rate

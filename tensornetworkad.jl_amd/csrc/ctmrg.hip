@@ -92,10 +92,10 @@ __global__ __launch_bounds__(256) void ritz_scale_norms_kernel(const double* __r
 // |G - I|_F^2 of a k x k matrix (k <= 256): one workgroup of GD_NT threads, thread (row i, column
 // phase jo) sums rows i over columns jo, jo + GD_NT / 256, ... (coalesced along rows)
 constexpr int GD_NT = 1024;
-// out[0] = |G - I|_F^2; out[1] = *info (the preceding Cholesky's breakdown column, as a double), so the host
-// reads the pass's status with the pivot in one transfer
+// (next to the Cholesky kernel's smallest pivot and breakdown column, so the host reads the pass's status with
+// one transfer)
 __global__ __launch_bounds__(GD_NT) void gram_dev_kernel(const double* __restrict__ G, int k,
-                                                         double* __restrict__ out, const int* __restrict__ info) {
+                                                         double* __restrict__ out) {
   __shared__ double red[GD_NT / 64];
   const int t = threadIdx.x, i = t & 255, jo = t >> 8;
   double acc = 0.0;
@@ -111,7 +111,6 @@ __global__ __launch_bounds__(GD_NT) void gram_dev_kernel(const double* __restric
     double s = 0.0;
     for (int w = 0; w < GD_NT / 64; ++w) s += red[w];
     out[0] = s;
-    out[1] = (double)*info;
   }
 }
 
@@ -302,21 +301,26 @@ static void dbg_finite(Ctx* c, const char* what, const double* dev, size_t n) {
 // Eigensolver: top-k eigenpairs of a symmetric n x n FP64 matrix by |lambda|
 // ==========================================================================
 // norms_ready: w.nrm already holds the column norms of Y (ritz_scale_norms_kernel)
+// light: one pass is enough (the block goes through another product and orthonormalisation before a
+// Rayleigh-Ritz step looks at it, so only its span and a deviation well below 1 matter): X^T X is not formed
 static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& w, unsigned seed,
-                           bool norms_ready = false) {
+                           bool norms_ready = false, bool light = false) {
   hipStream_t s = c->stream;
   // column scaling, random refill of (numerically) null columns
   if (norms_ready) k_fill_scale_cols(Y, n, k, w.nrm.as<double>(), 1e-13, seed, s);
   else k_normalize_cols(Y, n, k, w.nrm.as<double>(), 1e-13, seed, s);
   // A well-conditioned block takes plain CholeskyQR passes: one when the result is orthonormal to
   // working precision (|X^T X - I|_F <= 1e-12, the usual case once the iteration converges), else a
-  // second: X (X^T X)^{-1/2} to second order when |X^T X - I|_F <= 1e-5, CholeskyQR2 above.  That holds when the Cholesky pivots of the Gram matrix stay above 1e-4 (unit
-  // columns: condition number around 1e4, far below u^-1/2).  The first pass and the test run before
-  // the host looks at the pivots, so that one round trip serves both.  Otherwise: shifted CholeskyQR
-  // followed by two plain passes (sCholQR3); columns that the shifted pass finds linearly dependent
-  // on earlier ones (pivot at the shift's level: the block has lower rank than k, e.g. a
-  // rank-deficient corner matrix) are replaced by random directions first, so the block always spans
-  // k dimensions.
+  // second: X (X^T X)^{-1/2} to second order when |X^T X - I|_F <= 1e-5, CholeskyQR2 above.  That holds when the
+  // Cholesky pivots of the Gram matrix stay above 1e-6 (unit columns: condition number below u^-1/2) and the
+  // first pass leaves a deviation below 1e-2.  The first pass and the test run before
+  // the host looks at the pivots, so that one round trip serves both.  A block that fails (condition
+  // number up to ~1e10: the first product with a random block) takes one shifted CholeskyQR pass, which
+  // keeps its small directions (to an accuracy of u over their relative size, all that the iteration needs of
+  // them), and the plain pass again.  If that fails too, the block has lower rank than k (a rank-deficient
+  // corner matrix): columns that a shifted pass finds linearly dependent on earlier ones (pivot at the
+  // shift's level) are replaced by random directions, so the block always spans k dimensions, and what
+  // still fails takes shifted CholeskyQR followed by two plain passes (sCholQR3).
   std::vector<double> piv(k);
   std::vector<int> dead(k);
   const double u = 1.1102230246251565e-16;
@@ -344,51 +348,57 @@ static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& 
     }
     return ndead;
   };
-  // Plain CholeskyQR as described above; when its pivots are too small, the shifted Cholesky finds
-  // the dependent columns, they are refilled, and the plain passes are tried once more (a block whose
-  // only defect was those columns is now well-conditioned).  What still fails takes sCholQR3 below.
-  for (int round = 0; round < 2; ++round) {
-    double* scal = w.scal.as<double>();   // [0] smallest pivot, [1] |X^T X - I|_F^2, [2] breakdown column
+  // Plain CholeskyQR as described above, then the shifted pass (round 0) or the refill of dependent columns
+  // (round 1), each followed by the plain pass again.  What still fails takes sCholQR3 below.
+  for (int round = 0; round < 3; ++round) {
+    double* scal = w.scal.as<double>();   // [0] smallest pivot, [1] breakdown column, [2] |X^T X - I|_F^2
     tc_launch(c, Prec::F64, gemm_desc('T', 'N', k, k, n, n, n, k), Y, Y, w.G.as<double>(), s);
     chol_inv(w.G.as<double>(), k, 0.0, w.Rinv.as<double>(), w.info.as<int>(), nullptr, s, scal);
     tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, k, n, k, n), Y, w.Rinv.as<double>(), X, s);
-    tc_launch(c, Prec::F64, gemm_desc('T', 'N', k, k, n, n, n, k), X, X, w.G.as<double>(), s);
-    hipLaunchKernelGGL(gram_dev_kernel, dim3(1), dim3(GD_NT), 0, s, w.G.as<double>(), k, scal + 1,
-                       w.info.as<int>());
-    TNAD_HIP_TRY(hipGetLastError());
-    double hs[3] = {0.0, 0.0, 0.0};   // smallest pivot, |X^T X - I|_F^2, Cholesky breakdown column
-    c->read_async(hs, scal, 3 * sizeof(double));
+    if (!light) {
+      tc_launch(c, Prec::F64, gemm_desc('T', 'N', k, k, n, n, n, k), X, X, w.H.as<double>(), s);
+      hipLaunchKernelGGL(gram_dev_kernel, dim3(1), dim3(GD_NT), 0, s, w.H.as<double>(), k, scal + 2);
+      TNAD_HIP_TRY(hipGetLastError());
+    }
+    double hs[3] = {0.0, 0.0, 0.0};   // smallest pivot, breakdown column, |X^T X - I|_F^2
+    c->read_async(hs, scal, (light ? 2 : 3) * sizeof(double));
     c->sync();
-    int info = (int)hs[2];
+    int info = (int)hs[1];
+    const double dev = std::sqrt(hs[2]);
     if (std::getenv("TNAD_DEBUG_EIG"))
-      std::fprintf(stderr, "[tnad eig] plain Cholesky info=%d min pivot=%.3e |X^T X - I|_F=%.3e\n", info, hs[0],
-                   std::sqrt(hs[1]));
-    if (info == 0 && hs[0] > 1e-4) {
-      const double dev = std::sqrt(hs[1]);
-      if (dev <= 1e-12) return;
+      std::fprintf(stderr, "[tnad eig] plain Cholesky info=%d min pivot=%.3e |X^T X - I|_F=%.3e\n", info, hs[0], dev);
+    if (info == 0 && hs[0] > 1e-6 && dev <= 1e-2) {
+      if (light || dev <= 1e-12) return;
       if (dev <= 1e-5) {
         // X^T X = I + E with |E|_F <= 1e-5: X F with F = (I + E)^{-1/2} to second order is orthonormal to
         // O(|E|^3) (below 1e-15) and spans the same columns, which is all the iteration keeps; it takes
         // two small products instead of a second Cholesky and its host check
-        tc_launch(c, Prec::F64, gemm_desc('N', 'N', k, k, k, k, k, k), w.G.as<double>(), w.G.as<double>(),
+        tc_launch(c, Prec::F64, gemm_desc('N', 'N', k, k, k, k, k, k), w.H.as<double>(), w.H.as<double>(),
                   w.Rinv.as<double>(), s);
-        hipLaunchKernelGGL(inv_sqrt2_coef_kernel, dim3((k * k + 255) / 256), dim3(256), 0, s, w.G.as<double>(),
+        hipLaunchKernelGGL(inv_sqrt2_coef_kernel, dim3((k * k + 255) / 256), dim3(256), 0, s, w.H.as<double>(),
                            w.Rinv.as<double>(), k, w.Rinv.as<double>());
         TNAD_HIP_TRY(hipGetLastError());
         tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, k, n, k, n), X, w.Rinv.as<double>(), Y, s);
         k_copy(Y, X, (size_t)n * k, s);
         return;
       }
-      chol_inv(w.G.as<double>(), k, 0.0, w.Rinv.as<double>(), w.info.as<int>(), nullptr, s);
+      chol_inv(w.H.as<double>(), k, 0.0, w.Rinv.as<double>(), w.info.as<int>(), nullptr, s);
       c->read_async(&info, w.info.ptr, sizeof(int));
       c->sync();
       if (info != 0)   // breakdown (pivot <= 0): factor the shifted Gram instead
-        chol_inv(w.G.as<double>(), k, shift, w.Rinv.as<double>(), w.info.as<int>(), nullptr, s);
+        chol_inv(w.H.as<double>(), k, shift, w.Rinv.as<double>(), w.info.as<int>(), nullptr, s);
       tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, k, n, k, n), X, w.Rinv.as<double>(), Y, s);
       k_copy(Y, X, (size_t)n * k, s);
       return;
     }
-    if (round == 1) break;
+    if (round == 2) break;
+    if (round == 0) {   // ill-conditioned: the shifted factor of the same Gram matrix, columns back to unit norm
+      chol_inv(w.G.as<double>(), k, shift, w.Rinv.as<double>(), w.info.as<int>(), nullptr, s);
+      tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, k, n, k, n), Y, w.Rinv.as<double>(), X, s);
+      k_copy(X, Y, (size_t)n * k, s);
+      k_normalize_cols(Y, n, k, w.nrm.as<double>(), 1e-13, seed + 104729u, s);
+      continue;
+    }
     const int ndead = find_dead(seed + 7919u, true);
     if (std::getenv("TNAD_DEBUG_EIG"))
       std::fprintf(stderr, "[tnad eig] shifted CholeskyQR: %d dependent columns refilled\n", ndead);
@@ -427,7 +437,7 @@ EigWork::EigWork(Ctx* c, int n, int k)
       nrm(c, (size_t)k * 8), res(c, (size_t)(k + 2) * 8), info(c, (size_t)k * sizeof(int) + 16), scal(c, 16 * 8) {}
 
 int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, int maxit, double tol,
-             double* X, double* AX, double* theta, EigStats* st) {
+             double* X, double* AX, double* theta, EigStats* st, EigPlan* plan) {
   hipStream_t s = c->stream;
   if (n <= JACOBI_MAX) {
     // full spectrum: exact reference semantics (all n singular values / vectors), by divide and conquer
@@ -443,38 +453,57 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
   // status transfer below are sized by want and need want <= k
   if (want < 1 || want > k) throw Error(TNAD_ERR_UNSUPPORTED, "eigensolver: kept block wider than 192");
   EigWork w(c, n, k);
-  // starting block
-  if (X0) {
-    k_copy(X0, w.Y.as<double>(), (size_t)n * k, s);
-  } else {
-    k_random_matrix(w.Y.as<double>(), (size_t)n * k, 0x1234567u, s);
+  // starting block: the previous step's Ritz vectors, or a random one (its columns' norms lie within a few per
+  // cent of each other, and only its span counts: it needs no orthonormalisation)
+  if (X0) k_copy(X0, X, (size_t)n * k, s);
+  else k_random_matrix(X, (size_t)n * k, 0x1234567u, s);
+  if (maxit < 2) {   // the Rayleigh-Ritz step comes at once: it needs an orthonormal block
+    k_copy(X, w.Y.as<double>(), (size_t)n * k, s);
+    orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x9e3779b9u);
   }
-  orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x9e3779b9u);
   std::vector<double> hres(k + 2), hth(k);
   // opt-in trace of the iteration (TNAD_DEBUG_EIG=1), to stderr
   static const bool dbg = [] {
     const char* e = std::getenv("TNAD_DEBUG_EIG");
     return e && *e && *e != '0';
   }();
-  int it = 0;
-  double rel = 0.0, best = HUGE_VAL, best_mark = HUGE_VAL, prev_rel = HUGE_VAL;
-  int best_it = 0, n_exact = 0;
+  // Orthogonal iteration X <- orth(A X), with a Rayleigh-Ritz step only where the kept residual is expected to
+  // have reached tol: the span after p products is the same whether or not Ritz vectors were formed on
+  // the way, and a Rayleigh-Ritz step (0.65 ms of eigensolver at k = 192, two n x k x k products, a host round
+  // trip) costs as much as three or four products with their CholeskyQR passes.  The first one comes after the
+  // product count that the caller's previous, similar matrix needed (plan), else after the second
+  // product; it measures the residual and the rate |theta_k / theta_want| per product, which place the next
+  // one.  At chi = 128, D = 4: ~6 Rayleigh-Ritz steps per eigenproblem before, 1 to 2 now.
+  int it = 0, n_exact = 0, last_rr = 0, best_it = 0;
+  int next_rr = 2;
+  if (plan && plan->products > 0 && plan->rate > 0.0) {
+    int d;   // products to add (or leave out) for this tolerance at that matrix's rate
+    if (plan->resid < 3e-15) d = -std::max(1, plan->products / 4);   // rounding level: reached some products earlier
+    else d = (int)std::ceil(std::max(-16.0, std::min(16.0, std::log(tol / plan->resid) / std::log(plan->rate))));
+    next_rr = std::max(2, plan->products + d);
+  }
+  next_rr = std::min(next_rr, std::max(maxit, 1));
+  double rel = 0.0, best = HUGE_VAL, best_mark = HUGE_VAL, prev_rel = HUGE_VAL, rate = 0.0;
   bool force_exact = false;
-  for (it = 1; it <= maxit; ++it) {
-    // Y = A X ; H = X^T Y ; H = W diag(theta) W^T ; Xr = X W ; Yr = Y W
-    tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, n, n, n, n), A, X, w.Y.as<double>(), s);
+  while (true) {
+    tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, n, n, n, n), A, X, w.Y.as<double>(), s);   // Y = A X
+    ++it;
+    if (it < next_rr) {
+      orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, false, it + 1 < next_rr);
+      continue;
+    }
+    // Rayleigh-Ritz: H = X^T Y ; H = W diag(theta) W^T ; Xr = X W ; Yr = Y W.  One product after the last
+    // Ritz basis (H nearly diagonal) a few rotations of near-degenerate pairs plus second-order perturbation
+    // theory (ritz_select) may stand in for the eigendecomposition of H; otherwise H is decomposed exactly,
+    // by divide and conquer: after products without a Rayleigh-Ritz step between (there the columns mix,
+    // and the perturbation theory's remainder, not the span, set the residual: up to 96 products instead of
+    // 12 on the 800 x 800 splits of TRG at chi = 20), whenever H is not close enough to diagonal, and
+    // whenever the residual stopped falling.  ritz_select's flag gates the exact solver's kernels on the
+    // device: no host round trip.
     tc_launch(c, Prec::F64, gemm_desc('T', 'N', k, k, n, n, n, k), X, w.Y.as<double>(), w.H.as<double>(), s);
     dbg_finite(c, "X", X, (size_t)n * k);
     dbg_finite(c, "H", w.H.as<double>(), (size_t)k * k);
-    // Rayleigh-Ritz: once the block is nearly an invariant subspace (H nearly diagonal in the
-    // previous Ritz basis) a few rotations of near-degenerate pairs plus second-order perturbation
-    // theory (ritz_select) stand in for the eigendecomposition of H; otherwise H is decomposed exactly,
-    // by divide and conquer: on the first cold iteration, whenever H is not close enough to diagonal,
-    // and whenever the residual stopped falling (by 10% per iteration).  ritz_select's flag gates the
-    // exact solver's kernels on the device: no host round trip.  (Exact solves where two or three
-    // Jacobi sweeps used to improve the basis cut the subspace iterations per evaluation from 35 to 30
-    // on the FP64 path at chi = 128, D = 4, and 17 to 14 on the mixed one, 21% and 10% less time.)
-    const bool exact_forced = force_exact || (it == 1 && !X0);
+    const bool exact_forced = force_exact || last_rr == 0 || it - last_rr > 1;
     int* gate = w.info.as<int>();
     if (!exact_forced) ritz_select(w.H.as<double>(), k, k, want, 1e-2, theta, w.W.as<double>(), gate, s);
     syev_dc(w.H.as<double>(), k, k, theta, w.W.as<double>(), w.Vw.as<double>(), s, exact_forced ? nullptr : gate);
@@ -487,8 +516,8 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
                        theta, n, w.res.as<double>(), exact_forced ? nullptr : gate);
     TNAD_HIP_TRY(hipGetLastError());
     c->read_async(hres.data(), w.res.ptr, (size_t)(want + 2) * 8);   // residuals, theta_0, flag
+    c->read_async(hth.data(), theta, (size_t)k * 8);
     c->sync();
-    hth[0] = hres[want];
     const int flag = (int)hres[want + 1];
     const bool exact = flag != 0;   // the exact solver ran (forced, or the selective Rayleigh-Ritz declined)
     n_exact += exact;
@@ -498,23 +527,32 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
     if (dbg)
       std::fprintf(stderr, "[tnad eig] n=%d k=%d want=%d it=%d rel_resid=%.3e theta0=%.6e rr=%s(%d)\n", n, k, want,
                    it, rel, hth[0], exact ? "exact" : "select", exact_forced ? -1 : flag);
-    force_exact = !(rel < 0.9 * prev_rel);
-    prev_rel = rel;
     if (!(rel == rel)) throw Error(TNAD_ERR_NAN, "eigensolver: NaN in Ritz residual");
-    if (rel <= tol || it == maxit) break;
+    // residual ratio per product: observed between two Rayleigh-Ritz steps, else the guard's edge over the
+    // last kept value
+    rate = std::fabs(hth[k - 1]) / std::max(std::fabs(hth[want - 1]), 1e-300);
+    if (last_rr > 0 && prev_rel > 0.0 && rel > 0.0) rate = std::pow(rel / prev_rel, 1.0 / (it - last_rr));
+    rate = std::max(1e-3, std::min(0.9, rate));
+    force_exact = last_rr > 0 && !(rel < 0.9 * prev_rel);
+    prev_rel = rel;
+    last_rr = it;
+    if (rel <= tol || it >= maxit) break;
     // stagnation at the rounding level: no halving of the best residual in 8 iterations
     if (rel < best) { if (rel < 0.5 * best_mark) { best_mark = rel; best_it = it; } best = rel; }
     if (best < 1e3 * tol && it - best_it >= 8) break;
+    const int ahead = (int)std::ceil(std::log(tol / rel) / std::log(rate));
+    next_rr = std::min(maxit, it + std::max(1, std::min(ahead, 16)));
     hipLaunchKernelGGL(ritz_scale_norms_kernel, dim3(k), dim3(256), 0, s, w.Xr.as<double>(), w.Yr.as<double>(),
                        theta, n, w.Y.as<double>(), w.nrm.as<double>());
     TNAD_HIP_TRY(hipGetLastError());
-    orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, true);
+    orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, true, it + 1 < next_rr);
   }
+  if (plan) { plan->products = it; plan->resid = rel; plan->rate = rate; }
   k_copy(w.Xr.as<double>(), X, (size_t)n * k, s);
   k_copy(w.Yr.as<double>(), AX, (size_t)n * k, s);
   hipLaunchKernelGGL(canon_sign_kernel, dim3(k), dim3(NT), 0, s, X, AX, n);
   TNAD_HIP_TRY(hipGetLastError());
-  if (st) { st->iters = std::min(it, maxit); st->k = k; st->resid = rel; st->exact = n_exact; }
+  if (st) { st->iters = it; st->k = k; st->resid = rel; st->exact = n_exact; }
   return k;
 }
 
@@ -575,7 +613,7 @@ void ctmrg_step(Ctx* c, const StepDims& d, const StepOpts& o, const double* a64,
   const bool warm = X0 != nullptr && n > JACOBI_MAX;
   c->mark(4);
   int k = topk_eig(c, M, n, chi, kreq, warm ? X0 : nullptr, warm ? o.eig_warm_iters : o.eig_max_iters,
-                   p == Prec::F64 ? o.eig_tol : o.eig_tol_low, X, AX, theta, &est);
+                   p == Prec::F64 ? o.eig_tol : o.eig_tol_low, X, AX, theta, &est, &state.plan);
   c->mark(5);
   state.k = k;
   if (X_keep) k_copy(X, X_keep, (size_t)n * k, s);

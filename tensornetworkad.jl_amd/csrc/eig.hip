@@ -624,7 +624,10 @@ __global__ __launch_bounds__(CH_G * CH_G) void chol_inv_kernel(const double* __r
   chol_blocks<0>(A, B, m, sh, st, tx, ty, t, piv, Rinv);
   if (t == 0) {
     if (info) *info = st.bad;
-    if (pmin_out) *pmin_out = st.pmin;
+    if (pmin_out) {   // the smallest pivot and the breakdown column, for one host transfer
+      pmin_out[0] = st.pmin;
+      pmin_out[1] = (double)st.bad;
+    }
   }
 }
 

@@ -124,6 +124,58 @@ __global__ void split_vectors_kernel(const double* __restrict__ X, int N, int m,
   }
 }
 
+// The same for pairs from the subspace iteration, which are converged to 1e-13 |theta_0|: relative to a small s
+// that leaves a part 1e-13 s_0 / (2 s) of the (-s, [u; -v]) partner in the vector, which lengthens u and
+// shortens v by as much.  Normalising the halves separately takes it out to first order, and theta over the
+// product of the halves' norms is the singular value (they are 1/sqrt 2 each without it).  One workgroup per
+// column; also writes s_j and sqrt(s_j).  A column whose halves are far from equal (an unconverged guard
+// pair) is only scaled.
+__global__ __launch_bounds__(NT) void split_vectors_unit_kernel(const double* __restrict__ X,
+                                                                const double* __restrict__ theta, int N, int m,
+                                                                const int* __restrict__ cols, double* __restrict__ U,
+                                                                double* __restrict__ V, double* __restrict__ sv,
+                                                                double* __restrict__ sq) {
+  __shared__ double red[2][NT / 64];
+  const int j = blockIdx.x, mp = N - m;
+  const double* x = X + (size_t)N * cols[j];
+  double a = 0.0, b = 0.0;
+  for (int r = threadIdx.x; r < N; r += NT) {
+    const double v = x[r] * x[r];
+    if (r < m) a += v;
+    else b += v;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_down(a, o);
+    b += __shfl_down(b, o);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = a;
+    red[1][threadIdx.x >> 6] = b;
+  }
+  __syncthreads();
+  double nu = 0.0, nv = 0.0;
+  for (int w = 0; w < NT / 64; ++w) {
+    nu += red[0][w];
+    nv += red[1][w];
+  }
+  nu = sqrt(nu);
+  nv = sqrt(nv);
+  double fu = 1.4142135623730951, fv = 1.4142135623730951, s = theta[cols[j]];
+  if (2.0 * nu * nv > 0.5) {
+    fu = 1.0 / nu;
+    fv = 1.0 / nv;
+    s *= 0.5 * fu * fv;
+  }
+  for (int r = threadIdx.x; r < N; r += NT) {
+    if (r < m) U[r + (size_t)m * j] = fu * x[r];
+    else V[(r - m) + (size_t)mp * j] = fv * x[r];
+  }
+  if (threadIdx.x == 0) {
+    sv[j] = s;
+    sq[j] = sqrt(s);
+  }
+}
+
 // u_out[:, j] = U[:, j] sqrt(s_j) (m x k);  v_out[j, :] = sqrt(s_j) V[:, j]^T (rows j < k of an
 // ldv x mp column-major array)
 __global__ void scale_split_kernel(const double* __restrict__ U, const double* __restrict__ V,
@@ -275,7 +327,7 @@ struct SvdTape {
 
 // singular triplets of M from the top eigenpairs of [[0, M], [M^T, 0]]
 static void svd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, int dmax, double tol, double* u_out,
-                      double* v_out, SvdTape& tp) {
+                      double* v_out, SvdTape& tp, EigPlan* plan = nullptr) {
   hipStream_t s = c->stream;
   const int m = d1 * d2, mp = d3 * d4, N = m + mp;
   const int len = std::min(m, mp);
@@ -290,7 +342,7 @@ static void svd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, i
   keig = std::min(keig, N);
   DevBuf X(c, (size_t)N * keig * 8), AX(c, (size_t)N * keig * 8), theta(c, (size_t)keig * 8);
   keig = topk_eig(c, B.as<double>(), N, std::min(want, keig), keig, nullptr, 300, 1e-13, X.as<double>(),
-                  AX.as<double>(), theta.as<double>(), nullptr);
+                  AX.as<double>(), theta.as<double>(), nullptr, plan);
   std::vector<double> th(keig);
   c->read_async(th.data(), theta.ptr, (size_t)keig * 8);
   c->sync();
@@ -320,10 +372,16 @@ static void svd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, i
   k_fill(tp.sq.as<double>(), (size_t)std::max(k, Kc), 0.0, s);
   if (K > 0) {
     c->write_async(cols.ptr, pos.data(), (size_t)K * sizeof(int));
-    c->write_async(tp.sv.ptr, tp.hs.data(), (size_t)K * 8);
-    c->write_async(tp.sq.ptr, hsq.data(), (size_t)K * 8);
-    hipLaunchKernelGGL(split_vectors_kernel, dim3(nb((size_t)N * K)), dim3(NT), 0, s, X.as<double>(), N, m,
-                       cols.as<int>(), K, tp.U.as<double>(), tp.V.as<double>());
+    if (N > JACOBI_MAX) {
+      hipLaunchKernelGGL(split_vectors_unit_kernel, dim3(K), dim3(NT), 0, s, X.as<double>(), theta.as<double>(), N, m,
+                         cols.as<int>(), tp.U.as<double>(), tp.V.as<double>(), tp.sv.as<double>(),
+                         tp.sq.as<double>());
+    } else {   // the whole spectrum at once: pairs accurate to rounding
+      c->write_async(tp.sv.ptr, tp.hs.data(), (size_t)K * 8);
+      c->write_async(tp.sq.ptr, hsq.data(), (size_t)K * 8);
+      hipLaunchKernelGGL(split_vectors_kernel, dim3(nb((size_t)N * K)), dim3(NT), 0, s, X.as<double>(), N, m,
+                         cols.as<int>(), K, tp.U.as<double>(), tp.V.as<double>());
+    }
   }
   // u = U[:, 1:k] sqrt(s), v = sqrt(s) V[:, 1:k]^T; columns j >= K are zero
   k_fill(u_out, (size_t)m * k, 0.0, s);
@@ -438,6 +496,9 @@ void trg_run(Ctx* c, const double* a_host, int q, int chi, int niter, double tol
   std::vector<std::unique_ptr<TrgIter>> tape;
   double lnz = 0.0;
   DevBuf mv(c, 16), mi(c, 16);
+  // the splits of one size are alike from one iteration to the next, and the two of an iteration too
+  EigPlan plan;
+  size_t plan_size = 0;
   for (int it = 1; it <= niter; ++it) {
     const size_t na = (size_t)du * dr * du * dr;
     std::unique_ptr<TrgIter> T(new TrgIter());
@@ -476,8 +537,10 @@ void trg_run(Ctx* c, const double* a_host, int q, int chi, int niter, double tol
     T->ul_t = DevBuf(c, (size_t)kmax1 * du * dr * 8 + 8);
     T->ld_t = DevBuf(c, (size_t)dr * du * kmax2 * 8 + 8);
     T->ru_t = DevBuf(c, (size_t)kmax2 * dr * du * 8 + 8);
-    svd_split(c, p1.as<double>(), du, dr, du, dr, chi, tol, T->dr_t.as<double>(), T->ul_t.as<double>(), T->s1);
-    svd_split(c, p2.as<double>(), dr, du, dr, du, chi, tol, T->ld_t.as<double>(), T->ru_t.as<double>(), T->s2);
+    if (plan_size != na) plan = EigPlan{};
+    plan_size = na;
+    svd_split(c, p1.as<double>(), du, dr, du, dr, chi, tol, T->dr_t.as<double>(), T->ul_t.as<double>(), T->s1, &plan);
+    svd_split(c, p2.as<double>(), dr, du, dr, du, chi, tol, T->ld_t.as<double>(), T->ru_t.as<double>(), T->s2, &plan);
     const int k1 = T->s1.k, k2 = T->s2.k;
     T->k1 = k1; T->k2 = k2;
     // a = ein"npu,por,dom,lmn -> urdl"(dr, ld, ul, ru)                   (src/trg.jl:25)
