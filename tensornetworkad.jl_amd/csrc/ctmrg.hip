@@ -57,35 +57,18 @@ __global__ void resid_norms_kernel(const double* __restrict__ X, const double* _
   if (threadIdx.x == 0) out[j] = sqrt(red[0] + red[1] + red[2] + red[3]);
 }
 
-// Next subspace block from the Rayleigh-Ritz pairs, and its column norms, in one pass:
+// Next subspace block from the Rayleigh-Ritz pairs:
 // Z[:, j] = Yr[:, j] / theta_j = Xr[:, j] + R[:, j] / theta_j (R = Yr - Xr Theta is orthogonal to Xr, so
 // Z^T Z = I + (R Theta^-1)^T (R Theta^-1) >= I stays well conditioned however collinear the residuals are);
-// numerically null Ritz values keep Z[:, j] = Xr[:, j].  One block of 256 threads per column j, the sum of
-// squares taken in the order of the column-norm kernel (thread-strided partial sums, a shuffle tree per
-// wave, the wave sums added in order).
-__global__ __launch_bounds__(256) void ritz_scale_norms_kernel(const double* __restrict__ Xr,
-                                                               const double* __restrict__ Yr,
-                                                               const double* __restrict__ theta, int n,
-                                                               double* __restrict__ Z, double* __restrict__ nrm) {
-  __shared__ double red[4];
+// numerically null Ritz values keep Z[:, j] = Xr[:, j].  One block of 256 threads per column j.
+__global__ __launch_bounds__(256) void ritz_scale_kernel(const double* __restrict__ Xr, const double* __restrict__ Yr,
+                                                         const double* __restrict__ theta, int n,
+                                                         double* __restrict__ Z) {
   const int j = blockIdx.x;
   const double t0 = fabs(theta[0]), th = theta[j];
   const bool use_y = fabs(th) > 1e-14 * t0;
   const size_t o = (size_t)n * j;
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) {
-    const double z = use_y ? Yr[o + i] / th : Xr[o + i];
-    Z[o + i] = z;
-    acc += z * z;
-  }
-  for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double sum = 0.0;
-    for (int w = 0; w < 4; ++w) sum += red[w];
-    nrm[j] = sqrt(sum);
-  }
+  for (int i = threadIdx.x; i < n; i += 256) Z[o + i] = use_y ? Yr[o + i] / th : Xr[o + i];
 }
 
 // *out = sum_ij (G_ij - delta_ij)^2 (one workgroup; G is k x k)
@@ -300,15 +283,12 @@ static void dbg_finite(Ctx* c, const char* what, const double* dev, size_t n) {
 // ==========================================================================
 // Eigensolver: top-k eigenpairs of a symmetric n x n FP64 matrix by |lambda|
 // ==========================================================================
-// norms_ready: w.nrm already holds the column norms of Y (ritz_scale_norms_kernel)
 // light: one pass is enough (the block goes through another product and orthonormalisation before a
 // Rayleigh-Ritz step looks at it, so only its span and a deviation well below 1 matter): X^T X is not formed
-static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& w, unsigned seed,
-                           bool norms_ready = false, bool light = false) {
+static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& w, unsigned seed, bool light = false) {
   hipStream_t s = c->stream;
-  // column scaling, random refill of (numerically) null columns
-  if (norms_ready) k_fill_scale_cols(Y, n, k, w.nrm.as<double>(), 1e-13, seed, s);
-  else k_normalize_cols(Y, n, k, w.nrm.as<double>(), 1e-13, seed, s);
+  // (the columns' scale is taken out of the Gram matrix by the Cholesky kernel: Y itself is only normalised,
+  // with a random refill of null columns, when a pass fails)
   // A well-conditioned block takes plain CholeskyQR passes: one when the result is orthonormal to
   // working precision (|X^T X - I|_F <= 1e-12, the usual case once the iteration converges), else a
   // second: X (X^T X)^{-1/2} to second order when |X^T X - I|_F <= 1e-5, CholeskyQR2 above.  That holds when the
@@ -353,7 +333,7 @@ static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& 
   for (int round = 0; round < 3; ++round) {
     double* scal = w.scal.as<double>();   // [0] smallest pivot, [1] breakdown column, [2] |X^T X - I|_F^2
     tc_launch(c, Prec::F64, gemm_desc('T', 'N', k, k, n, n, n, k), Y, Y, w.G.as<double>(), s);
-    chol_inv(w.G.as<double>(), k, 0.0, w.Rinv.as<double>(), w.info.as<int>(), nullptr, s, scal);
+    chol_inv(w.G.as<double>(), k, 0.0, w.Rinv.as<double>(), w.info.as<int>(), nullptr, s, scal, true);
     tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, k, n, k, n), Y, w.Rinv.as<double>(), X, s);
     if (!light) {
       tc_launch(c, Prec::F64, gemm_desc('T', 'N', k, k, n, n, n, k), X, X, w.H.as<double>(), s);
@@ -393,7 +373,7 @@ static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& 
     }
     if (round == 2) break;
     if (round == 0) {   // ill-conditioned: the shifted factor of the same Gram matrix, columns back to unit norm
-      chol_inv(w.G.as<double>(), k, shift, w.Rinv.as<double>(), w.info.as<int>(), nullptr, s);
+      chol_inv(w.G.as<double>(), k, shift, w.Rinv.as<double>(), w.info.as<int>(), nullptr, s, nullptr, true);
       tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, k, n, k, n), Y, w.Rinv.as<double>(), X, s);
       k_copy(X, Y, (size_t)n * k, s);
       k_normalize_cols(Y, n, k, w.nrm.as<double>(), 1e-13, seed + 104729u, s);
@@ -489,7 +469,7 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
     tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, n, n, n, n), A, X, w.Y.as<double>(), s);   // Y = A X
     ++it;
     if (it < next_rr) {
-      orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, false, it + 1 < next_rr);
+      orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, it + 1 < next_rr);
       continue;
     }
     // Rayleigh-Ritz: H = X^T Y ; H = W diag(theta) W^T ; Xr = X W ; Yr = Y W.  One product after the last
@@ -542,10 +522,10 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
     if (best < 1e3 * tol && it - best_it >= 8) break;
     const int ahead = (int)std::ceil(std::log(tol / rel) / std::log(rate));
     next_rr = std::min(maxit, it + std::max(1, std::min(ahead, 16)));
-    hipLaunchKernelGGL(ritz_scale_norms_kernel, dim3(k), dim3(256), 0, s, w.Xr.as<double>(), w.Yr.as<double>(),
-                       theta, n, w.Y.as<double>(), w.nrm.as<double>());
+    hipLaunchKernelGGL(ritz_scale_kernel, dim3(k), dim3(256), 0, s, w.Xr.as<double>(), w.Yr.as<double>(), theta, n,
+                       w.Y.as<double>());
     TNAD_HIP_TRY(hipGetLastError());
-    orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, true, it + 1 < next_rr);
+    orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, it + 1 < next_rr);
   }
   if (plan) { plan->products = it; plan->resid = rel; plan->rate = rate; }
   k_copy(w.Xr.as<double>(), X, (size_t)n * k, s);

@@ -466,169 +466,251 @@ __global__ __launch_bounds__(JS_NT) void jacobi_sort_kernel(const double* __rest
   for (int row = t; row < m; row += JS_NT) V[row + (long long)rank * m] = sgn * vi[row];
 }
 
-// Cholesky (with diagonal shift) + triangular inverse of an m x m SPD matrix, m <= 192,
-// in one workgroup of 16 x 16 threads (one wavefront per SIMD: the per-step costs that every
-// thread pays, the pivot's reciprocal square root and the scaling of its column entries, are
-// then paid by 4 wavefronts instead of 16; 158 -> 140 us at m = 192).  Thread (ty, tx) holds
-// the 12 x 12 elements (ty + 16a, tx + 16b) in registers (cyclic distribution, so every step
-// keeps all threads busy).  One sweep of m elimination steps forms both L and B = L^-1: step jj
-// broadcasts column jj of the Schur complement and row jj of B (both through LDS, one
-// barrier per step, double-buffered); every thread then updates its part of the trailing
-// Schur complement (A -= l l^T) and of the rows of B below jj (B[i,:] -= L[i,jj] B[jj,:],
-// forward substitution for L B = I), and the owners finish column jj of L and row jj of B.
-// Only L's current column is ever needed, so finished columns of L are dropped, and the
-// rows of B in a 16-row block are final when the block's steps are done: they go straight
-// to the output.  The steps run in twelve 16-column blocks whose block index is a template
-// parameter, so every register access is static and blocks that a step cannot touch
-// (finished columns, the upper triangle) are not even emitted.
-// Output Rinv = L^-T (upper triangular, column-major, zeros below the diagonal) so
-// that X = Y Rinv; piv (nullable) receives diag(L).
-constexpr int CH_G = 16;                  // thread grid edge
-constexpr int CH_R = JACOBI_MAX / CH_G;   // elements per thread per dimension
-static_assert(CH_R * CH_G == JACOBI_MAX, "Cholesky tiling");
+// Cholesky (with diagonal shift, optionally of the matrix scaled to unit diagonal) and triangular inverse of an
+// m x m SPD matrix, m <= 192, in one workgroup of 16 wavefronts, blocked by 16 on the FP64 matrix cores.
+// With G = U^T U by blocks (U upper triangular), B = U^-T = L^-1:
+//   panel J:  U_JJ from A_JJ, W = U_JJ^-T ;  U_JI = W A_JI (I > J) ;  B_JK = W R_JK (K < J), B_JJ = W
+//   update :  A_KI -= U_JK^T U_JI (J < K <= I) ;  R_IK -= U_JI^T B_JK (K <= J < I)
+// A_KI is dead once panel K is done and R_IK (zero before it) is first touched then, so both live in the one
+// accumulator of the pair (K, I): at most seven 16 x 16 accumulators per wavefront, and each pair takes exactly
+// one product per panel.  Every operand of every product is used as the accumulator layout holds it (lane l,
+// register r: row l / 16 + 4 r, column l % 16): the product's B operand B[k][n] and the transposed A operand
+// A^T[k][m] are both indexed that way, so the panels go through LDS as plain [register][lane] arrays without
+// bank conflicts and without a transposition.
+// Wavefront 0 does nothing but the diagonal blocks, one row per lane (repeated in the four groups of 16
+// lanes, which share the columns of W), values of other rows by DPP row broadcasts; it forms U_J,J+1 and the
+// update of A_J+1,J+1 in its own registers and goes straight on to the next block.  The twelve wavefronts on
+// the other three SIMDs own the pairs; they form the rest of panel J while wavefront 0 prepares block J + 1 and
+// update while it factors that.  (Products on wavefront 0's SIMD nearly doubled its chain:
+// 4,800 cycles per block alone, 8,200 beside them.)  The three others of its SIMD write finished rows of B.
+// Bound by the 192-step scalar chain of the diagonal blocks (~330 cycles a step: broadcast, reciprocal square
+// root, scaling, update) and, in the first panels, by the products.  Launches back to back: 53 us at m = 192, 36 at
+// 144, 25 at 96; the kernel before (unblocked, 16 x 16 threads, one barrier and one reciprocal square root per
+// column) took 145 us at m = 192 and 113 at 144.
+// Output Rinv = U^-1 (upper triangular, column-major, zeros below the diagonal), scaled so that X = Y Rinv holds for
+// the unscaled G; piv (nullable) receives the pivots diag(U).
+constexpr int CH_B = 16;                        // block size
+constexpr int CH_NB = JACOBI_MAX / CH_B;        // blocks per dimension
+constexpr int CH_W = 16;                        // wavefronts
+constexpr int CH_P = 12;                        // of them with pairs (not on SIMD 0)
+constexpr int CH_S = (CH_NB * (CH_NB + 1) / 2 + CH_P - 1) / CH_P;   // pairs per wavefront
+static_assert(CH_NB * CH_B == JACOBI_MAX, "Cholesky tiling");
+typedef double chd4 __attribute__((ext_vector_type(4)));
 
 struct CholShared {
-  double* cb;     // 2 x JACOBI_MAX broadcast buffers: column jj of the Schur complement
-  double* rb;     // 2 x JACOBI_MAX broadcast buffers: row jj of B before its scaling
+  double U[CH_NB][4][64];   // U_JI of the current panel, at I
+  double B[CH_NB][4][64];   // B_JK of the current panel, at K
+  double W[2][4][64];       // W of panel J (at J & 1) as an A operand: register k, lane l: W[l % 16][l / 16 + 4 k]
+  double H[2][4][64];       // handed to wavefront 0: A_J,J+1 and A_J+1,J+1, updated with the panels before J
+  double D[CH_B][CH_B + 1]; // the diagonal block on its way to one row per lane
+  double sc[JACOBI_MAX];    // 1 / sqrt(G_ii) (1 without scaling)
+  double pv[JACOBI_MAX];    // the pivots
 };
 
-// the first non-positive pivot (1-based, 0: none) and the smallest pivot so far, kept by thread 0 in
-// registers (every thread sees the same pivots)
-struct CholState {
-  int bad = 0;
-  double pmin = HUGE_VAL;
-};
-
-// 1 / sqrt(d) for a positive normal d: the hardware estimate refined by two Newton steps
+// 1 / sqrt(d) for a positive normal d: the hardware estimate y (2^-24 relative) with e = 1 - d y^2 corrected to
+// third order, y (1 + e / 2 + 3 e^2 / 8): remainder 5/16 e^3 < 2^-70, and four dependent operations where two
+// Newton steps take six.  A d that is not positive gives a NaN or an infinity, and so does what follows from it.
 __device__ __forceinline__ double rsqrt_refined(double d) {
-  double y = __builtin_amdgcn_rsq(d);
-  y = y * (1.5 - 0.5 * d * y * y);
-  y = y * (1.5 - 0.5 * d * y * y);
-  return y;
+  const double y = __builtin_amdgcn_rsq(d);
+  const double e = fma(-(d * y), y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
-// elimination steps jj = 16 BJ .. min(16 BJ + 15, m - 1).  The owner column broadcasts the whole
-// column jj (zeros above the diagonal and in the padding), so the update needs no bounds tests: its
-// only stray products land in row jj above the diagonal (the unused upper triangle) and in column
-// jj, which the owner rewrites.  Likewise row jj of B is zero right of its diagonal, its stray
-// product lands in row jj itself (rewritten by its owner), and rows above jj meet a zero L[i,jj].
-// After the block's steps its rows of B are final and are written to Rinv.
-template <int BJ>
-__device__ __forceinline__ void chol_block(double (&A)[CH_R][CH_R], double (&B)[CH_R][CH_R], int m,
-                                           const CholShared& sh, CholState& st, int tx, int ty, int t,
-                                           double* __restrict__ piv, double* __restrict__ Rinv) {
-  const int j0 = BJ * CH_G, j1 = min(m, j0 + CH_G);
-  for (int jj = j0; jj < j1; ++jj) {
-    double* col = sh.cb + (jj & 1) * JACOBI_MAX;
-    double* row = sh.rb + (jj & 1) * JACOBI_MAX;
-    const int tj = jj - j0;
-    if (tx == tj) {
+// the value of lane N of each group of 16 lanes, in every lane of the group (DPP row_newbcast; one 64-bit move)
+extern "C" __device__ long tnad_update_dpp_i64(long old, long src, int ctrl, int row_mask, int bank_mask,
+                                               bool bound_ctrl) __asm("llvm.amdgcn.update.dpp.i64");
+template <int N> __device__ __forceinline__ double row_lane(double x) {
+  return __longlong_as_double(tnad_update_dpp_i64(0, __double_as_longlong(x), 0x150 + N, 0xF, 0xF, true));
+}
+
+// a[C] -= l l_C for C = C0 .. 15
+template <int C0> __device__ __forceinline__ void chol_rank1(double (&a)[CH_B], double l) {
+  if constexpr (C0 < CH_B) {
+    a[C0] = fma(-l, row_lane<C0>(l), a[C0]);
+    chol_rank1<C0 + 1>(a, l);
+  }
+}
+
+// elimination steps J .. 15 of the 16 x 16 block: lane (q, r) holds row r of the Schur complement (a) and the
+// entries W[r][4 i + q] of the inverse (w).  Row J of W is final at step J: every lane of group q has it then and
+// writes it out (the same value to the same address), as an A operand (Wo) and in the accumulator layout (Bo).
+// Rows up to J go on with meaningless numbers, which no other row reads.
+template <int J>
+__device__ __forceinline__ void chol_diag(double (&a)[CH_B], double (&w)[4], int q, double (&Wo)[4][64],
+                                          double (&Bo)[4][64], double* pv, double& pmin, int& bad, int col0) {
+  const double d = row_lane<J>(a[J]);
+  const double isd = rsqrt_refined(d);
+  const double l = a[J] * isd;
+  chol_rank1<J + 1>(a, l);
 #pragma unroll
-      for (int a = BJ; a < CH_R; ++a) {
-        const int i = ty + CH_G * a;
-        col[i] = (i >= jj && i < m) ? A[a][BJ] : 0.0;
+  for (int i = 0; i < 4; ++i) {
+    double x = 0.0;   // W is lower triangular (column 4 i + q; zero by itself for columns of this i beyond J)
+    if (i <= J / 4) {
+      x = row_lane<J>(w[i]) * isd;
+      w[i] = fma(-l, x, w[i]);
+    }
+    Wo[i][16 * q + J] = x;
+    Bo[J >> 2][16 * (J & 3) + 4 * i + q] = x;
+  }
+  const double sd = d * isd;
+  pmin = fmin(pmin, sd);
+  bad = (d > 0.0 || bad != 0) ? bad : col0 + J + 1;
+  pv[J] = sd;
+  if constexpr (J + 1 < CH_B) chol_diag<J + 1>(a, w, q, Wo, Bo, pv, pmin, bad, col0);
+}
+
+__global__ __launch_bounds__(64 * CH_W) void chol_inv_kernel(const double* __restrict__ G, int m, double shift,
+                                                             int unit, double* __restrict__ Rinv, int* info,
+                                                             double* __restrict__ piv,
+                                                             double* __restrict__ pmin_out) {
+  __shared__ CholShared sh;
+  const int t = threadIdx.x, lane = t & 63, q = lane >> 4, r = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);   // uniform: the pair tests below are scalar
+  const int nb = (m + CH_B - 1) / CH_B;
+  // the wavefront's pairs (K, I), K <= I: every twelfth of the order 00, 01, 11, 02, ... (wavefront 0: the first
+  // diagonal block).  All the raw loads are in flight at once, ahead of the scale factors and their barrier.
+  const bool pairs = (wave & 3) != 0;
+  int pk[CH_S], pi[CH_S];
+  chd4 acc[CH_S];
+#pragma unroll
+  for (int s = 0; s < CH_S; ++s) {
+    const int p = pairs ? (wave / 4) * 3 + (wave & 3) - 1 + CH_P * s : 0;
+    // i (i + 1) / 2 <= p: the root of a number at least 0.5 from the next perfect square's
+    const int i = __builtin_amdgcn_readfirstlane((int)(0.5f * (__builtin_amdgcn_sqrtf(8.0f * p + 1.5f) - 1.0f)));
+    pi[s] = i < nb ? i : -1;                 // -1: no pair (its column is beyond the matrix)
+    pk[s] = p - i * (i + 1) / 2;
+    const double* g = G + min(CH_B * i + r, m - 1);   // clamped addresses; G is symmetric
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[s][k] = g[m * min(CH_B * pk[s] + q + 4 * k, m - 1)];
+    if (!pairs) break;                                // (uniform; wavefront 0 needs the first block only)
+  }
+  if (t < JACOBI_MAX) {
+    double s = 1.0;
+    if (unit && t < m) {
+      const double g = G[t + (size_t)m * t];
+      s = g > 0.0 ? rsqrt_refined(g) : 0.0;   // a null column: its pivot fails
+    }
+    sh.sc[t] = s;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < CH_S; ++s)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int row = CH_B * pk[s] + q + 4 * k, col = CH_B * (pi[s] < 0 ? 0 : pi[s]) + r;
+      // padding beyond m: a diagonal never coupled to the rest (large, so that it never is the smallest pivot)
+      acc[s][k] = (row < m && col < m) ? (acc[s][k] * sh.sc[row] * sh.sc[col] + (row == col ? shift : 0.0))
+                                       : (row == col ? 1e300 : 0.0);
+    }
+
+  if (wave == 0) {
+    double pmin = HUGE_VAL;
+    int bad = 0;
+    chd4 x = acc[0];
+    for (int J = 0; J < nb; ++J) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) sh.D[r][q + 4 * k] = x[k];   // symmetric: entry (q + 4 k, r)
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   // the rows come from other lanes
+      __builtin_amdgcn_wave_barrier();
+      double a[CH_B], w[4];
+#pragma unroll
+      for (int c = 0; c < CH_B; ++c) a[c] = sh.D[r][c];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = r == 4 * i + q ? 1.0 : 0.0;
+      if (J > 0) __syncthreads();   // panel J - 1 is published (by the others)
+      chol_diag<0>(a, w, q, sh.W[J & 1], sh.B[J], sh.pv + CH_B * J, pmin, bad, CH_B * J);
+      __syncthreads();   // W is published, the others have updated with panel J - 1 and handed over
+      if (J + 1 < nb) {
+        chd4 u = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          u = __builtin_amdgcn_mfma_f64_16x16x4f64(sh.W[J & 1][k][lane], sh.H[0][k][lane], u, 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = sh.H[1][k][lane];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x = __builtin_amdgcn_mfma_f64_16x16x4f64(-u[k], u[k], x, 0, 0, 0);
       }
     }
-    if (ty == tj) {
-#pragma unroll
-      for (int b = 0; b <= BJ; ++b) row[tx + CH_G * b] = B[BJ][b];
+    __syncthreads();   // the last row block of B is published
+    if (piv)
+      for (int i = lane; i < m; i += 64) piv[i] = sh.pv[i];
+    if (lane == 0) {
+      if (info) *info = bad;
+      if (pmin_out) {   // the smallest pivot and the breakdown column, for one host transfer
+        pmin_out[0] = pmin;
+        pmin_out[1] = (double)bad;
+      }
+    }
+    return;
+  }
+
+  if (!pairs) {
+    // row block J of B (published, final) to the output: columns 16 J .. of Rinv, Rinv(j, i) = B(i, j)
+    auto write_rows = [&](int J) {
+      for (int c = wave / 4 - 1; c < CH_B; c += CH_W / 4 - 1) {
+        const int i = CH_B * J + c;
+        if (i >= m) break;
+        for (int j = lane; j < m; j += 64)
+          Rinv[j + (size_t)m * i] = j <= i ? sh.B[j >> 4][c >> 2][16 * (c & 3) + (j & 15)] * sh.sc[j] : 0.0;
+      }
+    };
+    for (int J = 0; J < nb; ++J) {
+      if (J > 0) {
+        __syncthreads();
+        write_rows(J - 1);
+      }
+      __syncthreads();
     }
     __syncthreads();
-    // every LDS read of the step first, so that their latency overlaps the pivot's reciprocal square root;
-    // no branch before the products (the pivot bookkeeping is thread 0's, in registers)
-    double d = col[jj];
-    double li[CH_R], lj[CH_R], xr[CH_R];
+    write_rows(nb - 1);
+    return;
+  }
+
+  // panel P from its W: U_PI to U[I] (R_IP starts at zero), B_PK to B[K] (the pair is finished)
+  auto panel = [&](int P) {
 #pragma unroll
-    for (int a = BJ; a < CH_R; ++a) {
-      li[a] = col[ty + CH_G * a];
-      lj[a] = col[tx + CH_G * a];
+    for (int s = 0; s < CH_S; ++s) {
+      const int K = pk[s], I = pi[s];
+      if (I < 0 || K == I || (K != P && I != P)) continue;
+      chd4 c = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) c = __builtin_amdgcn_mfma_f64_16x16x4f64(sh.W[P & 1][k][lane], acc[s][k], c, 0, 0, 0);
+      double(&out)[4][64] = K == P ? sh.U[I] : sh.B[K];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) out[k][lane] = c[k];
+      acc[s] = chd4{0.0, 0.0, 0.0, 0.0};
+    }
+  };
+  for (int J = 0; J < nb; ++J) {
+    if (J > 0) {
+      panel(J - 1);
+      __syncthreads();   // panel J - 1 is published
     }
 #pragma unroll
-    for (int b = 0; b <= BJ; ++b) xr[b] = row[tx + CH_G * b];
-    const bool ok = d > 0.0;
-    st.bad = (!ok && st.bad == 0) ? jj + 1 : st.bad;
-    d = ok ? d : 1e-300;
-    const double isd = rsqrt_refined(d);
-    const double sd = d * isd;
-    st.pmin = fmin(st.pmin, sd);
+    for (int s = 0; s < CH_S; ++s) {
+      const int K = pk[s], I = pi[s];
+      if (I < J || (K == J && I == J)) continue;   // (block J, J is wavefront 0's)
+      if (J > 0) {
+        const double(&A)[4][64] = K >= J ? sh.U[K] : sh.U[I];
+        const double(&B)[4][64] = K >= J ? sh.U[I] : sh.B[K];
+        double x[4], y[4];
 #pragma unroll
-    for (int a = BJ; a < CH_R; ++a) {
-      li[a] *= isd;
-      lj[a] *= isd;
-    }
+        for (int k = 0; k < 4; ++k) {
+          x[k] = -A[k][lane];
+          y[k] = B[k][lane];
+        }
 #pragma unroll
-    for (int b = 0; b <= BJ; ++b) xr[b] *= isd;   // row jj of B, final
-    if (t == 0 && piv) piv[jj] = sd;
-    // trailing lower blocks BJ <= b <= a of the Schur complement
+        for (int k = 0; k < 4; ++k) acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[k], y[k], acc[s], 0, 0, 0);
+      }
+      if (I == J + 1 && K >= J) {
 #pragma unroll
-    for (int a = BJ; a < CH_R; ++a)
-#pragma unroll
-      for (int b = BJ; b <= a; ++b) A[a][b] -= li[a] * lj[b];
-    // rows of B below jj (blocks a >= BJ, columns b <= BJ)
-#pragma unroll
-    for (int a = BJ; a < CH_R; ++a)
-#pragma unroll
-      for (int b = 0; b <= BJ; ++b) B[a][b] -= li[a] * xr[b];
-    if (tx == tj) {
-#pragma unroll
-      for (int a = BJ; a < CH_R; ++a) {
-        const int i = ty + CH_G * a;
-        if (i >= jj) A[a][BJ] = (i == jj) ? sd : li[a];
+        for (int k = 0; k < 4; ++k) sh.H[K - J][k][lane] = acc[s][k];
       }
     }
-    if (ty == tj) {
-#pragma unroll
-      for (int b = 0; b <= BJ; ++b) B[BJ][b] = xr[b];
-    }
+    __syncthreads();   // W of panel J is published
   }
-  // rows i = ty + 16 BJ of B are final: Rinv(j, i) = B(i, j), zero above B's diagonal
-  const int i = ty + CH_G * BJ;
-  if (i < m) {
-#pragma unroll
-    for (int b = 0; b < CH_R; ++b) {
-      const int j = tx + CH_G * b;
-      if (j < m) Rinv[j + (size_t)m * i] = (b <= BJ && j <= i) ? B[BJ][b <= BJ ? b : 0] : 0.0;
-    }
-  }
-}
-
-// the column blocks BJ, BJ + 1, ..., CH_R - 1 in turn
-template <int BJ>
-__device__ __forceinline__ void chol_blocks(double (&A)[CH_R][CH_R], double (&B)[CH_R][CH_R], int m,
-                                            const CholShared& sh, CholState& st, int tx, int ty, int t,
-                                            double* __restrict__ piv, double* __restrict__ Rinv) {
-  chol_block<BJ>(A, B, m, sh, st, tx, ty, t, piv, Rinv);
-  if constexpr (BJ + 1 < CH_R) chol_blocks<BJ + 1>(A, B, m, sh, st, tx, ty, t, piv, Rinv);
-}
-
-__global__ __launch_bounds__(CH_G * CH_G) void chol_inv_kernel(const double* __restrict__ G, int m,
-                                                               double shift, double* __restrict__ Rinv,
-                                                               int* info, double* __restrict__ piv,
-                                                               double* __restrict__ pmin_out) {
-  __shared__ double bufs[4 * JACOBI_MAX];
-  CholShared sh{bufs, bufs + 2 * JACOBI_MAX};
-  CholState st;
-  const int t = threadIdx.x, tx = t % CH_G, ty = t / CH_G;
-  double A[CH_R][CH_R], B[CH_R][CH_R];
-#pragma unroll
-  for (int a = 0; a < CH_R; ++a) {
-#pragma unroll
-    for (int b = 0; b < CH_R; ++b) {
-      const int i = ty + CH_G * a, j = tx + CH_G * b;
-      const double g = G[min(j, m - 1) + (size_t)m * min(i, m - 1)];   // branch-free, clamped address
-      // padding beyond m: identity, never coupled to the rest
-      A[a][b] = (i < m && j < m) ? g + (i == j ? shift : 0.0) : (i == j ? 1.0 : 0.0);
-      B[a][b] = (i == j) ? 1.0 : 0.0;
-    }
-  }
-  chol_blocks<0>(A, B, m, sh, st, tx, ty, t, piv, Rinv);
-  if (t == 0) {
-    if (info) *info = st.bad;
-    if (pmin_out) {   // the smallest pivot and the breakdown column, for one host transfer
-      pmin_out[0] = st.pmin;
-      pmin_out[1] = (double)st.bad;
-    }
-  }
+  panel(nb - 1);
+  __syncthreads();
 }
 
 
@@ -967,9 +1049,9 @@ void ritz_select(const double* H, int ldh, int m, int nh, double thresh, double*
 }
 
 void chol_inv(const double* G, int m, double shift, double* Rinv, int* info, double* piv, hipStream_t s,
-              double* pmin) {
+              double* pmin, bool unit) {
   if (m < 1 || m > JACOBI_MAX) throw Error(TNAD_ERR_ARG, "chol_inv: size out of range");
-  hipLaunchKernelGGL(chol_inv_kernel, dim3(1), dim3(CH_G * CH_G), 0, s, G, m, shift, Rinv, info, piv, pmin);
+  hipLaunchKernelGGL(chol_inv_kernel, dim3(1), dim3(64 * CH_W), 0, s, G, m, shift, unit ? 1 : 0, Rinv, info, piv, pmin);
   TNAD_HIP_TRY(hipGetLastError());
 }
 

@@ -124,10 +124,11 @@ void ritz_select(const double* H, int ldh, int m, int nh, double thresh, double*
 
 // Cholesky of the m x m SPD matrix G (+ shift on the diagonal), returns Linv^T
 // (upper triangular, column-major) so that X = Y * Rinv with Rinv = L^-T.
-// piv (nullable, m doubles) receives the Cholesky pivots diag(L); pmin (nullable, device double) the
-// smallest of them.
+// piv (nullable, m doubles) receives the Cholesky pivots diag(L); pmin (nullable, two device doubles) the
+// smallest of them and the first non-positive one's column (1-based, 0: none).  unit: G is scaled to unit
+// diagonal first (before the shift) and Rinv scaled back, so that Y's columns need no normalisation.
 void chol_inv(const double* G, int m, double shift, double* Rinv, int* info, double* piv, hipStream_t s,
-              double* pmin = nullptr);
+              double* pmin = nullptr, bool unit = false);
 
 // ---------------------------------------------------------------------------
 // Elementwise / reduction kernels (elem.hip)

@@ -28,8 +28,13 @@ def _matrix(kind, n, want, rng):
     return 0.5 * (A + A.T), lam
 
 
-@pytest.mark.parametrize("n,want,k", [(193, 16, 40), (333, 37, 83), (576, 80, 192)])
-@pytest.mark.parametrize("kind", ["graded", "low_rank", "pairs", "multiplets", "slow"])
+# block widths at the edges of the Cholesky kernel's 16-column blocks, down to a single block
+EDGES = [(200, 1, 1), (200, 3, 5), (200, 8, 16), (200, 8, 17), (300, 20, 95), (300, 20, 97), (400, 100, 191)]
+
+
+@pytest.mark.parametrize("n,want,k,kind", [(n, w, k, kind) for n, w, k in [(193, 16, 40), (333, 37, 83), (576, 80, 192)]
+                                           for kind in ("graded", "low_rank", "pairs", "multiplets", "slow")]
+                         + [e + ("graded",) for e in EDGES])
 def test_symeig_truncated_hard_spectra(ctx, n, want, k, kind):
     print(f"case: symeig truncated {kind} n={n} want={want} k={k}", flush=True)
     A, lam = _matrix(kind, n, want, np.random.default_rng(n))
