@@ -142,26 +142,36 @@ __global__ void canon_sign_kernel(double* __restrict__ X, double* __restrict__ Y
   }
 }
 
-// coefficient block of the eigen adjoint among the kept pairs (see eig_adjoint below):
+// coefficient block (rows x chi) of the eigen adjoint (see eig_adjoint below).  Rows i < chi, the kept pairs:
 //   coef = Kt/2 with Kt = R11 Sigma + Sigma R11^T + C1bar,  R11_ij = (F_ij g_ij + F_ji g_ji) s_j,
 // F_ij = (s_j^2 - s_i^2) / ((s_j^2 - s_i^2)^2 + eta),  s = |lambda|.
 // Evaluated without FP contraction: the reference forms S2 = S.^2 first and then
 // S2' .- S2 (src/trg.jl:76-78), so the diagonal difference is exactly zero and the
 // Lorentzian F vanishes there; a fused multiply-add would leave the rounding residual of
 // s^2 (~1e-17) in place of that zero and F would blow up to ~1e23.
+// Rows i >= chi (only with the whole spectrum, rows = n): the pairs of a kept and a discarded vector,
+//   (lambda_j + lambda_i) L(s_j^2 - s_i^2) g_ij,
+// the difference of squares formed as (lambda_j - lambda_i)(lambda_j + lambda_i), so that the quotient stays
+// accurate for a (+s, -s) pair; nothing for a kept value at the rounding level (s_j <= 1e-14 s_0, as in
+// resolvent_pcg).
 __global__ void eigback_coef_kernel(const double* __restrict__ g, const double* __restrict__ lam,
-                                    const double* __restrict__ C1bar, int chi, double eta,
+                                    const double* __restrict__ C1bar, int chi, int rows, double eta,
                                     double* __restrict__ coef) {
 #pragma clang fp contract(off)
   int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= chi * chi) return;
-  int i = e % chi, j = e / chi;
+  if (e >= rows * chi) return;
+  int i = e % rows, j = e / rows;
   double li = lam[i], lj = lam[j];
+  if (i >= chi) {
+    const double p = lj + li, d = (lj - li) * p;
+    coef[e] = fabs(lj) > 1e-14 * fabs(lam[0]) ? p * (d / (d * d + eta)) * g[e] : 0.0;
+    return;
+  }
   double si2 = li * li, sj2 = lj * lj;
   double Fij = (sj2 - si2) / ((sj2 - si2) * (sj2 - si2) + eta);
   double Fji = -Fij;
-  double gij = g[i + (long long)j * chi];
-  double gji = g[j + (long long)i * chi];
+  double gij = g[i + (long long)j * rows];
+  double gji = g[j + (long long)i * rows];
   double sj = fabs(lj), si = fabs(li);
   double sigj = lj < 0 ? -1.0 : 1.0, sigi = li < 0 ? -1.0 : 1.0;
   double R_ij = (Fij * gij + Fji * gji) * sj;   // R11[i,j]
@@ -704,8 +714,9 @@ void ctmrg_step(Ctx* c, const StepDims& d, const StepOpts& o, const double* a64,
 // along u_i, i.e. (lambda_j - A)^-1 = (lambda_j + A)(lambda_j^2 - A^2)^-1 on the
 // complement of the kept vectors: X_c solves (lambda_j^2 - A^2) x_j = P G_j there
 // (resolvent_pcg, preconditioned by the extra Ritz pairs the eigensolver carries).
-// With the whole spectrum known (n <= 192) the preconditioner is the exact
-// inverse and the solve ends after its first step.
+// With the whole spectrum known (n <= 192) those contributions are a coefficient
+// each, in rows chi..n-1 of the coefficient block: W = U Kf over all n vectors, no
+// solve (28 launches and two host round trips fewer per step).
 // ==========================================================================
 void eig_adjoint(Ctx* c, const StepDims& d, const StepTape& tp, const double* G, const double* C1bar,
                  double* cpbar, EigBackStats* st, double* sweep_ref) {
@@ -713,16 +724,17 @@ void eig_adjoint(Ctx* c, const StepDims& d, const StepTape& tp, const double* G,
   const int chi = d.chi, n = d.n, k = tp.k;
   const double* X = tp.X.as<double>();
   const double* lam = tp.theta.as<double>();
-  DevBuf g(c, (size_t)chi * chi * 8), coef(c, (size_t)chi * chi * 8), W(c, (size_t)n * chi * 8);
-  // g = U1^T G  (chi x chi)
-  tc_launch(c, Prec::F64, gemm_desc('T', 'N', chi, chi, n, n, n, chi), X, G, g.as<double>(), s);
-  hipLaunchKernelGGL(eigback_coef_kernel, dim3((chi * chi + NT - 1) / NT), dim3(NT), 0, s, g.as<double>(), lam,
-                     C1bar, chi, 1e-40, coef.as<double>());
+  const int rows = k == n ? n : chi;   // the vectors that enter by coefficients: all of them when all are known
+  DevBuf g(c, (size_t)rows * chi * 8), coef(c, (size_t)rows * chi * 8), W(c, (size_t)n * chi * 8);
+  // g = U^T G  (rows x chi)
+  tc_launch(c, Prec::F64, gemm_desc('T', 'N', rows, chi, n, n, n, rows), X, G, g.as<double>(), s);
+  hipLaunchKernelGGL(eigback_coef_kernel, dim3((rows * chi + NT - 1) / NT), dim3(NT), 0, s, g.as<double>(), lam,
+                     C1bar, chi, rows, 1e-40, coef.as<double>());
   TNAD_HIP_TRY(hipGetLastError());
-  // W = U1 coef  (n x chi . chi x chi)
-  tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, chi, chi, n, chi, n), X, coef.as<double>(), W.as<double>(), s);
+  // W = U coef  (n x rows . rows x chi)
+  tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, chi, rows, n, rows, n), X, coef.as<double>(), W.as<double>(), s);
   int iters = 0;
-  if (n > chi) {
+  if (n > rows) {
     DevBuf sq(c, (size_t)k * 8), Xc(c, (size_t)n * chi * 8), AXc(c, (size_t)n * chi * 8),
         tmp(c, (size_t)n * chi * 8);
     k_square(lam, sq.as<double>(), k, s);
