@@ -292,6 +292,12 @@ void run_ctmrg(tnad_ctx* ctx, tnad_tape& t, const double* C0, const double* T0, 
     rest = ss.rest;
     rest_err = ss.rest_err;
     plan = ss.plan;
+    if (tp) {   // the inputs move into the tape
+      tp->C = std::move(Ca);
+      tp->T = std::move(Ta);
+      Ca = DevBuf(c, nC * 8);
+      Ta = DevBuf(c, nT * 8);
+    }
     std::swap(Ca, Cb);
     std::swap(Ta, Tb);
     iters += 1;

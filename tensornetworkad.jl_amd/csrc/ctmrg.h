@@ -100,7 +100,7 @@ struct StepTape {
   Prec prec;
   int k;
   double eig_tol = 1e-13;   // relative Ritz residual the step's eigensolver was run to
-  DevBuf C, T;          // step inputs (FP64)
+  DevBuf C, T;          // step inputs (FP64), moved in by the caller after the step
   DevBuf X, AX, theta;  // eigenpairs (FP64): X = [z | extra], AX = A X
   DevBuf M;             // cpmat + cpmat^T (FP64)
   PBuf X2, Y2;          // contraction intermediates reused by the adjoint

@@ -191,13 +191,13 @@ __global__ void add_lam_cols_kernel(double* __restrict__ W, const double* __rest
   }
 }
 
-// lbar[abc, x, y] += coef * tr[abc] * delta_xy
+// lbar[abc, x, y] += f * *coef * tr[abc] * delta_xy
 __global__ void add_trace_diag_kernel(double* __restrict__ lbar, const double* __restrict__ tr,
-                                      const double* __restrict__ coef_dev, double coef_host, int m, int s) {
+                                      const double* __restrict__ coef, double f, int m, int s) {
   int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= m * s) return;
   int abc = e % m, x = e / m;
-  double c = coef_dev ? *coef_dev : coef_host;
+  const double c = f * *coef;
   lbar[abc + (size_t)m * (x + s * x)] += c * tr[abc];
 }
 
@@ -227,8 +227,6 @@ __global__ void norm_back_kernel(const double* __restrict__ x, const double* __r
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
     out[i] = ybar[i] / nrm + nbar * x[i] / (nrm + eps0);
 }
-
-__global__ void sqrt_inplace_kernel(double* x) { x[0] = sqrt(x[0]); }
 
 inline unsigned nb(size_t n) {
   size_t b = (n + NT - 1) / NT;
@@ -264,6 +262,14 @@ const PBuf& at_prec(Ctx* c, const PBuf& src, Prec p, PBuf& tmp) {
     k_cast<float>(src.b.as<float>(), tmp.b.as<double>(), src.n, c->stream);
   }
   return tmp;
+}
+
+// src at precision p as a kernel operand: src itself for FP64, else a converted copy held in tmp
+static const void* as_prec(Ctx* c, const double* src, size_t n, Prec p, PBuf& tmp) {
+  if (p == Prec::F64) return src;
+  tmp = PBuf(c, p, n);
+  to_prec(c, src, tmp);
+  return tmp.ptr();
 }
 
 void tc(Ctx* c, Prec p, const TView& A, const void* a, const TView& B, const void* b, const TView& C, void* o,
@@ -550,8 +556,7 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
 // CTMRG step (src/ctmrg.jl:126-153)
 // ==========================================================================
 StepTape::StepTape(Ctx* c, const StepDims& d, Prec p, int k)
-    : prec(p), k(k), C(c, (size_t)d.chi * d.chi * 8), T(c, (size_t)d.chi * d.D * d.chi * 8),
-      X(c, (size_t)d.n * k * 8), AX(c, (size_t)d.n * k * 8), theta(c, (size_t)k * 8),
+    : prec(p), k(k), X(c, (size_t)d.n * k * 8), AX(c, (size_t)d.n * k * 8), theta(c, (size_t)k * 8),
       M(c, (size_t)d.n * d.n * 8), X2(c, p, (size_t)d.n * d.n), Y2(c, p, (size_t)d.n * d.n),
       C2(c, (size_t)d.chi * d.chi * 8), T2(c, (size_t)d.chi * d.D * d.chi * 8), nrm(c, 4 * 8) {}
 
@@ -562,33 +567,26 @@ void ctmrg_step(Ctx* c, const StepDims& d, const StepOpts& o, const double* a64,
   const int chi = d.chi, D = d.D, n = d.n;
   const long long lc = chi, lD = D;
   const Prec p = o.prec;
-  const size_t es = esize(p);
   // operands at contraction precision
-  PBuf Cp(c, p, (size_t)chi * chi), Tp(c, p, (size_t)chi * D * chi);
-  to_prec(c, C, Cp);
-  to_prec(c, T, Tp);
+  PBuf Cq, Tq;
+  const void* Cp = as_prec(c, C, (size_t)chi * chi, p, Cq);
+  const void* Tp = as_prec(c, T, (size_t)chi * D * chi, p, Tq);
   PBuf X1(c, p, (size_t)n * chi);
   PBuf X2tmp;
   PBuf* X2 = tape ? &tape->X2 : nullptr;
   if (!X2) { X2tmp = PBuf(c, p, (size_t)n * n); X2 = &X2tmp; }
   PBuf cp(c, p, (size_t)n * n);
   // cp = ein"ad,iba,dcl,jkcb -> ijlk"(C, T, T, a)          (src/ctmrg.jl:130)
-  tc(c, p, cm("iba", {lc, lD, lc}), Tp.ptr(), cm("ad", {lc, lc}), Cp.ptr(), cm("ibd", {lc, lD, lc}), X1.ptr());
-  tc(c, p, cm("ibd", {lc, lD, lc}), X1.ptr(), cm("dcl", {lc, lD, lc}), Tp.ptr(), cm("ibcl", {lc, lD, lD, lc}),
-     X2->ptr());
+  tc(c, p, cm("iba", {lc, lD, lc}), Tp, cm("ad", {lc, lc}), Cp, cm("ibd", {lc, lD, lc}), X1.ptr());
+  tc(c, p, cm("ibd", {lc, lD, lc}), X1.ptr(), cm("dcl", {lc, lD, lc}), Tp, cm("ibcl", {lc, lD, lD, lc}), X2->ptr());
   tc(c, p, cm("ibcl", {lc, lD, lD, lc}), X2->ptr(), cm("jkcb", {lD, lD, lD, lD}), ap.ptr(),
      cm("ijlk", {lc, lD, lc, lD}), cp.ptr());
   // cpmat = reshape(cp, n, n); cpmat += cpmat'                (src/ctmrg.jl:134-135)
   DevBuf Mtmp;
   double* M = tape ? tape->M.as<double>() : nullptr;
   if (!M) { Mtmp = DevBuf(c, (size_t)n * n * 8); M = Mtmp.as<double>(); }
-  if (p == Prec::F64) {
-    k_sym_add(cp.b.as<double>(), n, M, s);
-  } else {
-    DevBuf cp64(c, (size_t)n * n * 8);
-    k_cast<float>(cp.b.as<float>(), cp64.as<double>(), (size_t)n * n, s);
-    k_sym_add(cp64.as<double>(), n, M, s);
-  }
+  if (p == Prec::F64) k_sym_add(cp.b.as<double>(), n, M, s);
+  else k_sym_add(cp.b.as<float>(), n, M, s);
   // u, s, v = svd(cpmat) -> top-k eigenpairs by |lambda|        (src/ctmrg.jl:136)
   // block size: n (full spectrum) or 2.25 chi guard-extended (eig_block if set), capped at 192
   const int kreq = step_k(d, o);
@@ -618,44 +616,26 @@ void ctmrg_step(Ctx* c, const StepDims& d, const StepOpts& o, const double* a64,
   tc_launch(c, Prec::F64, gemm_desc('T', 'N', chi, chi, n, n, n, chi), z, AX, C2, s);
   // T' = ein"abjcd,abi,dck -> ijk"(tp, z, z), tp = ein"iam,jkla -> ijklm"(T, a)  (src/ctmrg.jl:131,140)
   // evaluated as ((T z) a) z without materialising tp.
-  PBuf zp(c, p, (size_t)n * chi);
-  to_prec(c, z, zp);
+  PBuf zq;
+  const void* zp = as_prec(c, z, (size_t)n * chi, p, zq);
   PBuf Y1(c, p, (size_t)n * n);
   PBuf Y2tmp;
   PBuf* Y2 = tape ? &tape->Y2 : nullptr;
   if (!Y2) { Y2tmp = PBuf(c, p, (size_t)n * n); Y2 = &Y2tmp; }
   PBuf T1p(c, p, (size_t)chi * D * chi);
-  tc(c, p, cm("aed", {lc, lD, lc}), Tp.ptr(), cm("abx", {lc, lD, lc}), zp.ptr(), cm("edbx", {lD, lc, lD, lc}),
-     Y1.ptr());
+  tc(c, p, cm("aed", {lc, lD, lc}), Tp, cm("abx", {lc, lD, lc}), zp, cm("edbx", {lD, lc, lD, lc}), Y1.ptr());
   tc(c, p, cm("edbx", {lD, lc, lD, lc}), Y1.ptr(), cm("bjce", {lD, lD, lD, lD}), ap.ptr(),
      cm("dcxj", {lc, lD, lc, lD}), Y2->ptr());
-  tc(c, p, cm("dcxj", {lc, lD, lc, lD}), Y2->ptr(), cm("dcy", {lc, lD, lc}), zp.ptr(), cm("xjy", {lc, lD, lc}),
-     T1p.ptr());
-  DevBuf T1(c, (size_t)chi * D * chi * 8);
-  from_prec(c, T1p, T1.as<double>());
+  tc(c, p, cm("dcxj", {lc, lD, lc, lD}), Y2->ptr(), cm("dcy", {lc, lD, lc}), zp, cm("xjy", {lc, lD, lc}), T1p.ptr());
   double* T2 = tape ? tape->T2.as<double>() : nullptr;
   DevBuf T2tmp;
   if (!T2) { T2tmp = DevBuf(c, (size_t)chi * D * chi * 8); T2 = T2tmp.as<double>(); }
-  // edge += ein"ijk -> kji"(conj(edge))                          (src/ctmrg.jl:146)
-  k_edge_sym(T1.as<double>(), chi, D, T2, s);
-  // corner /= norm(corner); edge /= norm(edge)                   (src/ctmrg.jl:149-150)
-  DevBuf red(c, 300 * 8), nr(c, 4 * 8);
+  // edge += ein"ijk -> kji"(conj(edge)); corner /= norm(corner); edge /= norm(edge)   (src/ctmrg.jl:146-150)
+  DevBuf red(c, 512 * 8), nr(c, 4 * 8);
   double* nrm = tape ? tape->nrm.as<double>() : nr.as<double>();
-  k_sumsq(C2, (size_t)chi * chi, red.as<double>(), s);
-  k_copy(red.as<double>(), nrm + 0, 1, s);
-  k_sumsq(T2, (size_t)chi * D * chi, red.as<double>(), s);
-  k_copy(red.as<double>(), nrm + 1, 1, s);
-  hipLaunchKernelGGL(sqrt_inplace_kernel, dim3(1), dim3(1), 0, s, nrm + 0);
-  hipLaunchKernelGGL(sqrt_inplace_kernel, dim3(1), dim3(1), 0, s, nrm + 1);
-  k_copy(C2, Cout, (size_t)chi * chi, s);
-  k_scale_by_dev(Cout, (size_t)chi * chi, nrm + 0, s);
-  k_copy(T2, Tout, (size_t)chi * D * chi, s);
-  k_scale_by_dev(Tout, (size_t)chi * D * chi, nrm + 1, s);
-  if (tape) {
-    tape->eig_tol = p == Prec::F64 ? o.eig_tol : o.eig_tol_low;
-    k_copy(C, tape->C.as<double>(), (size_t)chi * chi, s);
-    k_copy(T, tape->T.as<double>(), (size_t)chi * D * chi, s);
-  }
+  if (p == Prec::F64) k_step_end(T1p.b.as<double>(), chi, D, C2, T2, red.as<double>(), nrm, Cout, Tout, s);
+  else k_step_end(T1p.b.as<float>(), chi, D, C2, T2, red.as<double>(), nrm, Cout, Tout, s);
+  if (tape) tape->eig_tol = p == Prec::F64 ? o.eig_tol : o.eig_tol_low;
   // vals = s ./ s[1]   (src/ctmrg.jl:142).  With the whole spectrum computed (n <= 192) all n
   // values; otherwise the k largest (the chi kept values, resolved to the eigensolver tolerance, and the
   // guard block's Ritz values, which are not), with the rest 0.  For n > 192 the step also measures the
@@ -666,22 +646,14 @@ void ctmrg_step(Ctx* c, const StepDims& d, const StepOpts& o, const double* a64,
   const int nv = k;
   std::vector<double> th(nv);
   double sq[2] = {0.0, 0.0};
-  DevBuf E, XT, red1, red2, sqd;
+  DevBuf E, XT, sqd;
   if (n > JACOBI_MAX) {
     XT = DevBuf(c, (size_t)n * chi * 8);
     E = DevBuf(c, (size_t)n * n * 8);
-    red1 = DevBuf(c, 300 * 8);
-    red2 = DevBuf(c, 300 * 8);
     sqd = DevBuf(c, 2 * 8);
-    k_copy(X, XT.as<double>(), (size_t)n * chi, s);
-    k_scale_cols(XT.as<double>(), n, chi, theta, 0, s);
-    k_copy(M, E.as<double>(), (size_t)n * n, s);
-    tc_launch(c, Prec::F64, gemm_desc('N', 'T', n, n, chi, n, n, n, -1.0, 1.0), XT.as<double>(), X,
-              E.as<double>(), s);
-    k_sumsq(E.as<double>(), (size_t)n * n, red1.as<double>(), s);
-    k_sumsq(M, (size_t)n * n, red2.as<double>(), s);
-    k_copy(red1.as<double>(), sqd.as<double>() + 0, 1, s);
-    k_copy(red2.as<double>(), sqd.as<double>() + 1, 1, s);
+    k_scale_cols_to(X, n, chi, theta, XT.as<double>(), s);
+    tc_launch(c, Prec::F64, gemm_desc('N', 'T', n, n, chi, n, n, n), XT.as<double>(), X, E.as<double>(), s);
+    k_diff_sumsq(M, E.as<double>(), (size_t)n * n, red.as<double>(), sqd.as<double>(), s);
     c->read_async(sq, sqd.ptr, 2 * 8);
   }
   c->read_async(th.data(), theta, (size_t)nv * 8);
@@ -699,7 +671,6 @@ void ctmrg_step(Ctx* c, const StepDims& d, const StepOpts& o, const double* a64,
     state.rest_err = (double)n * 2.3e-16 * std::sqrt(sq[1]) / s0 + std::sqrt(2.0 * chi) * est.resid;
     if (!(state.rest == state.rest)) throw Error(TNAD_ERR_NAN, "ctmrgstep: NaN in the discarded spectrum");
   }
-  (void)es;
 }
 
 // ==========================================================================
@@ -788,69 +759,64 @@ void ctmrg_step_back(Ctx* c, const StepDims& d, Prec p, const StepTape& tp, cons
   const int chi = d.chi, D = d.D, n = d.n;
   const long long lc = chi, lD = D;
   const size_t nC = (size_t)chi * chi, nT = (size_t)chi * D * chi, nA = (size_t)D * D * D * D;
-  DevBuf red(c, 300 * 8), dotb(c, 300 * 8);
-  // --- normalisation adjoints (src/autodiff.jl:23-29) --------------------
-  DevBuf C2bar(c, nC * 8), T2bar(c, nT * 8), C1bar(c, nC * 8), T1bar(c, nT * 8);
-  {
-    DevBuf ss(c, 2 * 8), dd(c, 2 * 8);
-    k_sumsq(tp.C2.as<double>(), nC, red.as<double>(), s);
-    k_copy(red.as<double>(), ss.as<double>() + 0, 1, s);
-    k_dot(tp.C2.as<double>(), C3bar, nC, red.as<double>(), s);
-    k_copy(red.as<double>(), dd.as<double>() + 0, 1, s);
-    k_sumsq(tp.T2.as<double>(), nT, red.as<double>(), s);
-    k_copy(red.as<double>(), ss.as<double>() + 1, 1, s);
-    k_dot(tp.T2.as<double>(), T3bar, nT, red.as<double>(), s);
-    k_copy(red.as<double>(), dd.as<double>() + 1, 1, s);
-    hipLaunchKernelGGL(norm_back_kernel, dim3(nb(nC)), dim3(NT), 0, s, tp.C2.as<double>(), C3bar,
-                       ss.as<double>() + 0, dd.as<double>() + 0, C2bar.as<double>(), nC);
-    hipLaunchKernelGGL(norm_back_kernel, dim3(nb(nT)), dim3(NT), 0, s, tp.T2.as<double>(), T3bar,
-                       ss.as<double>() + 1, dd.as<double>() + 1, T2bar.as<double>(), nT);
-    TNAD_HIP_TRY(hipGetLastError());
-  }
-  // C1bar = C2bar + C2bar' ; T1bar = T2bar + permutedims(T2bar, (3,2,1))
-  k_sym_add(C2bar.as<double>(), chi, C1bar.as<double>(), s);
-  k_edge_sym(T2bar.as<double>(), chi, D, T1bar.as<double>(), s);
+  // --- adjoints of the normalisation and the symmetrisation (src/autodiff.jl:23-29) ---------
+  DevBuf red(c, 512 * 8), C1bar(c, nC * 8), T1bar(c, nT * 8);
+  k_step_end_back(tp.C2.as<double>(), C3bar, tp.T2.as<double>(), T3bar, chi, D, tp.nrm.as<double>(), red.as<double>(),
+                  C1bar.as<double>(), T1bar.as<double>(), s);
 
   // tape intermediates stored at the forward step's precision, converted to the sweep's
   PBuf Y2tmp, X2tmp;
   const PBuf& Y2 = at_prec(c, tp.Y2, p, Y2tmp);
   const PBuf& X2 = at_prec(c, tp.X2, p, X2tmp);
   // --- T' chain adjoint (tp never materialised) ----------------------------
-  PBuf T1b(c, p, nT), zp(c, p, (size_t)n * chi), Tp(c, p, nT), Cp(c, p, nC);
-  to_prec(c, T1bar.as<double>(), T1b);
-  to_prec(c, tp.X.as<double>(), zp);   // first n*chi entries = z
-  to_prec(c, tp.T.as<double>(), Tp);
-  to_prec(c, tp.C.as<double>(), Cp);
+  // (an FP64 sweep uses the tape's tensors and accumulates into the results in place)
+  const bool f64 = p == Prec::F64;
+  PBuf T1q, zq, Tq, Cq;
+  const void* T1b = as_prec(c, T1bar.as<double>(), nT, p, T1q);
+  const void* zp = as_prec(c, tp.X.as<double>(), (size_t)n * chi, p, zq);   // first n*chi entries = z
+  const void* Tp = as_prec(c, tp.T.as<double>(), nT, p, Tq);
+  const void* Cp = as_prec(c, tp.C.as<double>(), nC, p, Cq);
   PBuf P1(c, p, (size_t)n * n), Q1(c, p, (size_t)n * n), S1(c, p, (size_t)n * n);
-  PBuf Tbp(c, p, nT), abp(c, p, nA), zbp(c, p, (size_t)n * chi);
+  DevBuf zbar(c, (size_t)n * chi * 8), Tacc, a_acc;
+  PBuf Tbq, abq, zbq;
+  if (!f64) {
+    Tbq = PBuf(c, p, nT);
+    abq = PBuf(c, p, nA);
+    zbq = PBuf(c, p, (size_t)n * chi);
+    Tacc = DevBuf(c, nT * 8);
+    a_acc = DevBuf(c, nA * 8);
+  }
+  void* Tbp = f64 ? (void*)Tbar : Tbq.ptr();
+  void* abp = f64 ? (void*)abar : abq.ptr();
+  void* zbp = f64 ? zbar.ptr : zbq.ptr();
+  const double acc = f64 ? 1.0 : 0.0;   // abar: added by the contraction itself, or from its own buffer below
   // P1[a,b,j,y] = sum_x z[a,b,x] T1bar[x,j,y]
-  tc(c, p, cm("abx", {lc, lD, lc}), zp.ptr(), cm("xjy", {lc, lD, lc}), T1b.ptr(), cm("abjy", {lc, lD, lD, lc}),
+  tc(c, p, cm("abx", {lc, lD, lc}), zp, cm("xjy", {lc, lD, lc}), T1b, cm("abjy", {lc, lD, lD, lc}),
      P1.ptr());
   // Q1[a,e,c,y] = sum_{b,j} P1[a,b,j,y] a[b,j,c,e] ; Tbar[a,e,d] = sum_{c,y} Q1[a,e,c,y] z[d,c,y]
   tc(c, p, cm("abjy", {lc, lD, lD, lc}), P1.ptr(), cm("bjce", {lD, lD, lD, lD}), ap.ptr(),
      cm("aecy", {lc, lD, lD, lc}), Q1.ptr());
-  tc(c, p, cm("aecy", {lc, lD, lD, lc}), Q1.ptr(), cm("dcy", {lc, lD, lc}), zp.ptr(), cm("aed", {lc, lD, lc}),
-     Tbp.ptr());
+  tc(c, p, cm("aecy", {lc, lD, lD, lc}), Q1.ptr(), cm("dcy", {lc, lD, lc}), zp, cm("aed", {lc, lD, lc}),
+     Tbp);
   // S1[a,e,c,y] = sum_d T[a,e,d] z[d,c,y] ; abar[b,j,c,e] = sum_{a,y} P1[a,b,j,y] S1[a,e,c,y]
-  tc(c, p, cm("aed", {lc, lD, lc}), Tp.ptr(), cm("dcy", {lc, lD, lc}), zp.ptr(), cm("aecy", {lc, lD, lD, lc}),
+  tc(c, p, cm("aed", {lc, lD, lc}), Tp, cm("dcy", {lc, lD, lc}), zp, cm("aecy", {lc, lD, lD, lc}),
      S1.ptr());
   tc(c, p, cm("abjy", {lc, lD, lD, lc}), P1.ptr(), cm("aecy", {lc, lD, lD, lc}), S1.ptr(),
-     cm("bjce", {lD, lD, lD, lD}), abp.ptr());
+     cm("bjce", {lD, lD, lD, lD}), abp, 1.0, acc);
   // U1[a,b,j,y] = sum_{e,c} S1[a,e,c,y] a[b,j,c,e] (reuses P1) ; zbar[a,b,x] = sum_{j,y} U1 T1bar[x,j,y]
   tc(c, p, cm("aecy", {lc, lD, lD, lc}), S1.ptr(), cm("bjce", {lD, lD, lD, lD}), ap.ptr(),
      cm("abjy", {lc, lD, lD, lc}), P1.ptr());
-  tc(c, p, cm("abjy", {lc, lD, lD, lc}), P1.ptr(), cm("xjy", {lc, lD, lc}), T1b.ptr(), cm("abx", {lc, lD, lc}),
-     zbp.ptr());
+  tc(c, p, cm("abjy", {lc, lD, lD, lc}), P1.ptr(), cm("xjy", {lc, lD, lc}), T1b, cm("abx", {lc, lD, lc}),
+     zbp);
   // zbar[d,c,y] += sum_{x,j} Y2[d,c,x,j] T1bar[x,j,y]
-  tc(c, p, cm("dcxj", {lc, lD, lc, lD}), Y2.ptr(), cm("xjy", {lc, lD, lc}), T1b.ptr(), cm("dcy", {lc, lD, lc}),
-     zbp.ptr(), 1.0, 1.0);
-  DevBuf zbar(c, (size_t)n * chi * 8);
-  from_prec(c, zbp, zbar.as<double>());
-  DevBuf a_acc(c, nA * 8);
-  from_prec(c, abp, a_acc.as<double>());
-  k_axpby(1.0, a_acc.as<double>(), 1.0, abar, nA, s);
-  DevBuf Tacc(c, nT * 8);
-  from_prec(c, Tbp, Tacc.as<double>());
+  tc(c, p, cm("dcxj", {lc, lD, lc, lD}), Y2.ptr(), cm("xjy", {lc, lD, lc}), T1b, cm("dcy", {lc, lD, lc}),
+     zbp, 1.0, 1.0);
+  if (!f64) {
+    from_prec(c, zbq, zbar.as<double>());
+    from_prec(c, abq, a_acc.as<double>());
+    k_axpby(1.0, a_acc.as<double>(), 1.0, abar, nA, s);
+    from_prec(c, Tbq, Tacc.as<double>());
+  }
 
   // --- C' chain: zbar += (cpmat + cpmat') z C1bar  (FP64; A z kept from the forward)
   tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, chi, chi, n, chi, n, 1.0, 1.0), tp.AX.as<double>(),
@@ -861,31 +827,35 @@ void ctmrg_step_back(Ctx* c, const StepDims& d, Prec p, const StepTape& tp, cons
   eig_adjoint(c, d, tp, zbar.as<double>(), C1bar.as<double>(), cpbar.as<double>(), nullptr, sweep_ref);
 
   // --- cp chain adjoint -----------------------------------------------------
-  PBuf cpb(c, p, (size_t)n * n), X2b(c, p, (size_t)n * n), X1(c, p, (size_t)n * chi), X1b(c, p, (size_t)n * chi);
-  PBuf Cbp(c, p, nC), Tbp2(c, p, nT);
-  to_prec(c, cpbar.as<double>(), cpb);
+  PBuf cpq, X2b(c, p, (size_t)n * n), X1(c, p, (size_t)n * chi), X1b(c, p, (size_t)n * chi);
+  const void* cpb = as_prec(c, cpbar.as<double>(), (size_t)n * n, p, cpq);
+  PBuf Cbq;
+  if (!f64) Cbq = PBuf(c, p, nC);
+  void* Cbp = f64 ? (void*)Cbar : Cbq.ptr();
   // X1 = T C (recomputed)
-  tc(c, p, cm("iba", {lc, lD, lc}), Tp.ptr(), cm("ad", {lc, lc}), Cp.ptr(), cm("ibd", {lc, lD, lc}), X1.ptr());
+  tc(c, p, cm("iba", {lc, lD, lc}), Tp, cm("ad", {lc, lc}), Cp, cm("ibd", {lc, lD, lc}), X1.ptr());
   // X2bar[i,b,c,l] = sum_{j,k} cpbar[i,j,l,k] a[j,k,c,b]
-  tc(c, p, cm("ijlk", {lc, lD, lc, lD}), cpb.ptr(), cm("jkcb", {lD, lD, lD, lD}), ap.ptr(),
-     cm("ibcl", {lc, lD, lD, lc}), X2b.ptr());
+  tc(c, p, cm("ijlk", {lc, lD, lc, lD}), cpb, cm("jkcb", {lD, lD, lD, lD}), ap.ptr(), cm("ibcl", {lc, lD, lD, lc}),
+     X2b.ptr());
   // abar[j,k,c,b] += sum_{i,l} cpbar[i,j,l,k] X2[i,b,c,l]
-  tc(c, p, cm("ijlk", {lc, lD, lc, lD}), cpb.ptr(), cm("ibcl", {lc, lD, lD, lc}), X2.ptr(),
-     cm("jkcb", {lD, lD, lD, lD}), abp.ptr());
-  from_prec(c, abp, a_acc.as<double>());
-  k_axpby(1.0, a_acc.as<double>(), 1.0, abar, nA, s);
+  tc(c, p, cm("ijlk", {lc, lD, lc, lD}), cpb, cm("ibcl", {lc, lD, lD, lc}), X2.ptr(), cm("jkcb", {lD, lD, lD, lD}), abp,
+     1.0, acc);
+  if (!f64) {
+    from_prec(c, abq, a_acc.as<double>());
+    k_axpby(1.0, a_acc.as<double>(), 1.0, abar, nA, s);
+  }
   // X1bar[i,b,d] = sum_{c,l} X2bar[i,b,c,l] T[d,c,l] ; Tbar[d,c,l] += sum_{i,b} X1[i,b,d] X2bar[i,b,c,l]
-  tc(c, p, cm("ibcl", {lc, lD, lD, lc}), X2b.ptr(), cm("dcl", {lc, lD, lc}), Tp.ptr(), cm("ibd", {lc, lD, lc}),
-     X1b.ptr());
-  tc(c, p, cm("ibd", {lc, lD, lc}), X1.ptr(), cm("ibcl", {lc, lD, lD, lc}), X2b.ptr(), cm("dcl", {lc, lD, lc}),
-     Tbp2.ptr());
+  tc(c, p, cm("ibcl", {lc, lD, lD, lc}), X2b.ptr(), cm("dcl", {lc, lD, lc}), Tp, cm("ibd", {lc, lD, lc}), X1b.ptr());
+  tc(c, p, cm("ibd", {lc, lD, lc}), X1.ptr(), cm("ibcl", {lc, lD, lD, lc}), X2b.ptr(), cm("dcl", {lc, lD, lc}), Tbp, 1.0,
+     acc);
   // Cbar[a,d] = sum_{i,b} T[i,b,a] X1bar[i,b,d] ; Tbar[i,b,a] += sum_d X1bar[i,b,d] C[a,d]
-  tc(c, p, cm("iba", {lc, lD, lc}), Tp.ptr(), cm("ibd", {lc, lD, lc}), X1b.ptr(), cm("ad", {lc, lc}), Cbp.ptr());
-  tc(c, p, cm("ibd", {lc, lD, lc}), X1b.ptr(), cm("ad", {lc, lc}), Cp.ptr(), cm("iba", {lc, lD, lc}), Tbp2.ptr(),
-     1.0, 1.0);
-  from_prec(c, Cbp, Cbar);
-  from_prec(c, Tbp2, Tbar);
-  k_axpby(1.0, Tacc.as<double>(), 1.0, Tbar, nT, s);
+  tc(c, p, cm("iba", {lc, lD, lc}), Tp, cm("ibd", {lc, lD, lc}), X1b.ptr(), cm("ad", {lc, lc}), Cbp);
+  tc(c, p, cm("ibd", {lc, lD, lc}), X1b.ptr(), cm("ad", {lc, lc}), Cp, cm("iba", {lc, lD, lc}), Tbp, 1.0, 1.0);
+  if (!f64) {
+    from_prec(c, Cbq, Cbar);
+    from_prec(c, Tbq, Tbar);
+    k_axpby(1.0, Tacc.as<double>(), 1.0, Tbar, nT, s);
+  }
   (void)a64;
 }
 
@@ -907,12 +877,8 @@ void expectation_fwd(Ctx* c, int chi, int D, int ph, const double* h, const doub
   const size_t nap = (size_t)D * D * D * D * ph * ph;
   DevBuf red(c, 300 * 8);
   // ap /= norm(ap)
-  k_sumsq(ap, nap, red.as<double>(), s);
-  k_copy(red.as<double>(), ev.scal.as<double>() + 3, 1, s);   // |ap|^2
-  k_copy(ap, ev.apn.as<double>(), nap, s);
-  k_copy(red.as<double>(), ev.scal.as<double>() + 4, 1, s);
-  hipLaunchKernelGGL(sqrt_inplace_kernel, dim3(1), dim3(1), 0, s, ev.scal.as<double>() + 4);
-  k_scale_by_dev(ev.apn.as<double>(), nap, ev.scal.as<double>() + 4, s);
+  k_dot_to(ap, nullptr, nap, red.as<double>(), ev.scal.as<double>() + 3, s);   // |ap|^2
+  k_scale_rsqrt(ap, nap, ev.scal.as<double>() + 3, ev.apn.as<double>(), s);
   const Prec F = Prec::F64;
   double* E1 = ev.E1.as<double>();
   double* E2 = ev.E2.as<double>();
@@ -936,11 +902,9 @@ void expectation_fwd(Ctx* c, int chi, int D, int ph, const double* h, const doub
   tc(c, F, cm("abcij", {lc, lD, lc, ls, ls}), l, cm("ijkl", {ls, ls, ls, ls}), h, cm("abckl", {lc, lD, lc, ls, ls}),
      Lh.as<double>());
   const size_t nl = (size_t)n * chi * ph * ph, m3 = (size_t)n * chi;
-  k_dot(Lh.as<double>(), l, nl, red.as<double>(), s);
-  k_copy(red.as<double>(), ev.scal.as<double>() + 0, 1, s);   // e
+  k_dot_to(Lh.as<double>(), l, nl, red.as<double>(), ev.scal.as<double>() + 0, s);   // e
   hipLaunchKernelGGL(trace_last2_kernel, dim3((m3 + NT - 1) / NT), dim3(NT), 0, s, l, (int)m3, ph, ev.tr.as<double>());
-  k_sumsq(ev.tr.as<double>(), m3, red.as<double>(), s);
-  k_copy(red.as<double>(), ev.scal.as<double>() + 1, 1, s);   // nn
+  k_dot_to(ev.tr.as<double>(), nullptr, m3, red.as<double>(), ev.scal.as<double>() + 1, s);   // nn
   // scal[5] = e/nn, scal[6] = 1/nn, scal[7] = -e/nn^2
   hipLaunchKernelGGL(energy_scalars_kernel, dim3(1), dim3(1), 0, s, ev.scal.as<double>() + 0,
                      ev.scal.as<double>() + 1, ev.scal.as<double>() + 5);
@@ -969,17 +933,10 @@ void expectation_back(Ctx* c, int chi, int D, int ph, const double* h, const dou
   k_axpby(1.0, tmp.as<double>(), 1.0, lbar.as<double>(), nl, s);
   // scale by ebar (device scalar): lbar *= 1/nn  -> use scale_by_dev with nn
   k_scale_by_dev(lbar.as<double>(), nl, ev.scal.as<double>() + 1, s);
-  {
-    // 2 * nnbar = -2 e / nn^2
-    DevBuf cf(c, 8);
-    std::vector<double> sc(8);
-    c->read_async(sc.data(), ev.scal.ptr, 8 * 8);
-    c->sync();
-    double coef = 2.0 * sc[7];
-    hipLaunchKernelGGL(add_trace_diag_kernel, dim3((m3 * ph + NT - 1) / NT), dim3(NT), 0, s, lbar.as<double>(),
-                       ev.tr.as<double>(), (const double*)nullptr, coef, (int)m3, ph);
-    TNAD_HIP_TRY(hipGetLastError());
-  }
+  // 2 nnbar = -2 e / nn^2, read on the device
+  hipLaunchKernelGGL(add_trace_diag_kernel, dim3((m3 * ph + NT - 1) / NT), dim3(NT), 0, s, lbar.as<double>(),
+                     ev.tr.as<double>(), ev.scal.as<double>() + 7, 2.0, (int)m3, ph);
+  TNAD_HIP_TRY(hipGetLastError());
   double* E1 = ev.E1.as<double>();
   double* E2 = ev.E2.as<double>();
   double* E3 = ev.E3.as<double>();
@@ -1007,8 +964,7 @@ void expectation_back(Ctx* c, int chi, int D, int ph, const double* h, const dou
   tc(c, F, cm("eg", {lc, lc}), C, cm("efk", {lc, lD, lc}), E3b.as<double>(), cm("gfk", {lc, lD, lc}), Tbar, 1.0, 1.0);
   // ap /= norm(ap) adjoint
   DevBuf dd(c, 8);
-  k_dot(ap, apnb.as<double>(), nap, red.as<double>(), s);
-  k_copy(red.as<double>(), dd.as<double>(), 1, s);
+  k_dot_to(ap, apnb.as<double>(), nap, red.as<double>(), dd.as<double>(), s);
   hipLaunchKernelGGL(norm_back_kernel, dim3(nb(nap)), dim3(NT), 0, s, ap, apnb.as<double>(),
                      ev.scal.as<double>() + 3, dd.as<double>(), apbar, nap);
   TNAD_HIP_TRY(hipGetLastError());

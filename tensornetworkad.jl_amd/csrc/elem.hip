@@ -3,6 +3,8 @@
 // deterministic (fixed grid, fixed tree), so repeated runs agree bit for bit.
 #include "tnad_internal.h"
 
+#include <algorithm>
+
 namespace tnad {
 namespace {
 
@@ -15,21 +17,22 @@ inline unsigned nblk(size_t n, int per = NT) {
   return (unsigned)(b ? b : 1);
 }
 
-// Y = X + X^T for an n x n column-major matrix, 32x32 LDS tiles so both the
-// read of X and of X^T are coalesced.
-__global__ void sym_add_kernel(const double* __restrict__ X, int n, double* __restrict__ Y) {
+// Y = X + X^T for an n x n column-major matrix (X at the contractions' precision, the sum in FP64), 32x32 LDS
+// tiles so both the read of X and of X^T are coalesced.
+template <typename T>
+__global__ void sym_add_kernel(const T* __restrict__ X, int n, double* __restrict__ Y) {
   __shared__ double tile[32][33];
   int bx = blockIdx.x * 32, by = blockIdx.y * 32;
   int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 256 threads: ty in 0..7
   // load the transposed block X[by.., bx..] into tile
   for (int r = ty; r < 32; r += 8) {
     int i = by + tx, j = bx + r;          // element X[i, j] with i in rows of block (by), j cols (bx)
-    tile[r][tx] = (i < n && j < n) ? X[i + (long long)j * n] : 0.0;
+    tile[r][tx] = (i < n && j < n) ? (double)X[i + (long long)j * n] : 0.0;
   }
   __syncthreads();
   for (int r = ty; r < 32; r += 8) {
     int i = bx + tx, j = by + r;          // output Y[i, j] = X[i, j] + X[j, i]
-    if (i < n && j < n) Y[i + (long long)j * n] = X[i + (long long)j * n] + tile[tx][r];
+    if (i < n && j < n) Y[i + (long long)j * n] = (double)X[i + (long long)j * n] + tile[tx][r];
   }
 }
 
@@ -50,10 +53,23 @@ __global__ void axpby_kernel(double a, const double* __restrict__ x, double b, d
     y[i] = a * x[i] + (b == 0.0 ? 0.0 : b * y[i]);
 }
 
+__global__ void copy_kernel(const double* __restrict__ x, double* __restrict__ y, size_t n) {
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    y[i] = x[i];
+}
+
 __global__ void scale_by_dev_kernel(double* x, size_t n, const double* nrm) {
   double inv = 1.0 / *nrm;
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
     x[i] *= inv;
+}
+
+// y = x / sqrt(*sumsq)
+__global__ void scale_rsqrt_kernel(const double* __restrict__ x, size_t n, const double* __restrict__ sumsq,
+                                   double* __restrict__ y) {
+  const double inv = 1.0 / sqrt(*sumsq);
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    y[i] = x[i] * inv;
 }
 
 __device__ __forceinline__ double block_sum(double v, double* red) {
@@ -86,14 +102,130 @@ __global__ void final_sum_kernel(const double* __restrict__ part, int np, double
   if (threadIdx.x == 0) *out = s;
 }
 
-__global__ void edge_sym_kernel(const double* __restrict__ T1, int chi, int D, double* __restrict__ T2) {
-  size_t n = (size_t)chi * D * chi;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x) {
-    int i = e % chi;
-    int j = (e / chi) % D;
-    int k = e / ((size_t)chi * D);
-    T2[e] = T1[e] + T1[k + (size_t)chi * j + (size_t)chi * D * i];
+// index of T^{kji} for the element e of T (chi, D, chi)
+__device__ __forceinline__ size_t edge_flip(size_t e, int chi, int D) {
+  const unsigned u = (unsigned)e, i = u % (unsigned)chi, r = u / (unsigned)chi;   // chi D chi < 2^32 (limits)
+  const unsigned j = r % (unsigned)D, k = r / (unsigned)D;
+  return k + (size_t)chi * j + (size_t)chi * D * i;
+}
+
+// the sum over part[0 .. np) by one block, in every thread (np <= blockDim.x)
+__device__ __forceinline__ double sum_parts(const double* part, int np, double* red, double* bc) {
+  const double s = block_sum((int)threadIdx.x < np ? part[threadIdx.x] : 0.0, red);
+  if (threadIdx.x == 0) *bc = s;
+  __syncthreads();
+  return *bc;
+}
+
+// End of a CTMRG step in two launches (src/ctmrg.jl:146-150): T2 = T1 + T1^{kji} (T1 at the contractions'
+// precision) with the partial sums of |T2|^2 (part) and |C2|^2 (part + gridDim.x); then, from those, the two
+// norms (nrm) and the normalised tensors.
+template <typename T>
+__global__ void edge_sym_norms_kernel(const T* __restrict__ T1, int chi, int D, double* __restrict__ T2,
+                                      const double* __restrict__ C2, double* __restrict__ part) {
+  __shared__ double red[16];
+  const size_t nT = (size_t)chi * D * chi, nC = (size_t)chi * chi, step = (size_t)gridDim.x * blockDim.x;
+  const size_t first = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  double at = 0.0, ac = 0.0;
+  for (size_t e = first; e < nT; e += step) {
+    const double v = (double)T1[e] + (double)T1[edge_flip(e, chi, D)];
+    T2[e] = v;
+    at += v * v;
   }
+  for (size_t e = first; e < nC; e += step) ac += C2[e] * C2[e];
+  at = block_sum(at, red);
+  ac = block_sum(ac, red);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = at;
+    part[gridDim.x + blockIdx.x] = ac;
+  }
+}
+__global__ void normalize_pair_kernel(const double* __restrict__ C2, size_t nC, const double* __restrict__ T2, size_t nT,
+                                      const double* __restrict__ part, int np, double* __restrict__ nrm,
+                                      double* __restrict__ C3, double* __restrict__ T3) {
+  __shared__ double red[16];
+  __shared__ double bc[2];
+  const double nt = sqrt(sum_parts(part, np, red, bc)), nc = sqrt(sum_parts(part + np, np, red, bc + 1));
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    nrm[0] = nc;
+    nrm[1] = nt;
+  }
+  const double it = 1.0 / nt, ic = 1.0 / nc;
+  const size_t step = (size_t)gridDim.x * blockDim.x, first = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  for (size_t e = first; e < nT; e += step) T3[e] = T2[e] * it;
+  for (size_t e = first; e < nC; e += step) C3[e] = C2[e] * ic;
+}
+
+// The adjoint of that end of a step in two launches (src/autodiff.jl:23-29): partial sums of <T2, T3bar>
+// (part) and <C2, C3bar> (part + gridDim.x); then C2bar = C3bar / n + nbar C2 / (n + eps(0f0)) with
+// nbar = -<C2, C3bar> / n^2, likewise T2bar, and the adjoints of the symmetrisations, C1bar = C2bar + C2bar^T
+// and T1bar = T2bar + T2bar^{kji}, formed from the inputs without storing C2bar and T2bar.
+__global__ void norm_dots_kernel(const double* __restrict__ C2, const double* __restrict__ C3bar, size_t nC,
+                                 const double* __restrict__ T2, const double* __restrict__ T3bar, size_t nT,
+                                 double* __restrict__ part) {
+  __shared__ double red[16];
+  const size_t step = (size_t)gridDim.x * blockDim.x, first = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  double at = 0.0, ac = 0.0;
+  for (size_t e = first; e < nT; e += step) at += T2[e] * T3bar[e];
+  for (size_t e = first; e < nC; e += step) ac += C2[e] * C3bar[e];
+  at = block_sum(at, red);
+  ac = block_sum(ac, red);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = at;
+    part[gridDim.x + blockIdx.x] = ac;
+  }
+}
+__global__ void norm_sym_back_kernel(const double* __restrict__ C2, const double* __restrict__ C3bar,
+                                     const double* __restrict__ T2, const double* __restrict__ T3bar, int chi, int D,
+                                     const double* __restrict__ nrm, const double* __restrict__ part, int np,
+                                     double* __restrict__ C1bar, double* __restrict__ T1bar) {
+  __shared__ double red[16];
+  __shared__ double bc[2];
+  const double eps0 = 1.401298464324817e-45;
+  const double nc = nrm[0], nt = nrm[1];
+  const double bt = -sum_parts(part, np, red, bc) / (nt * nt), bC = -sum_parts(part + np, np, red, bc + 1) / (nc * nc);
+  const size_t nT = (size_t)chi * D * chi, nC = (size_t)chi * chi;
+  const size_t step = (size_t)gridDim.x * blockDim.x, first = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  auto ft = [&](size_t e) { return T3bar[e] / nt + bt * T2[e] / (nt + eps0); };
+  auto fc = [&](size_t e) { return C3bar[e] / nc + bC * C2[e] / (nc + eps0); };
+  for (size_t e = first; e < nT; e += step) T1bar[e] = ft(e) + ft(edge_flip(e, chi, D));
+  for (size_t e = first; e < nC; e += step) {
+    const unsigned i = (unsigned)e % (unsigned)chi, j = (unsigned)e / (unsigned)chi;
+    C1bar[e] = fc(e) + fc(j + (size_t)chi * i);
+  }
+}
+
+// part[b] = partial sum of (M - P)^2, part[gridDim.x + b] of M^2, in one pass over both; then the two sums
+__global__ void diff_sumsq_kernel(const double* __restrict__ M, const double* __restrict__ P, size_t n,
+                                  double* __restrict__ part) {
+  __shared__ double red[16];
+  double ad = 0.0, am = 0.0;
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+    const double m = M[i], d = m - P[i];
+    ad += d * d;
+    am += m * m;
+  }
+  ad = block_sum(ad, red);
+  am = block_sum(am, red);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = ad;
+    part[gridDim.x + blockIdx.x] = am;
+  }
+}
+__global__ void final_sums_kernel(const double* __restrict__ part, int np, double* out) {   // one block per sum
+  __shared__ double red[16];
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < np; i += blockDim.x) acc += part[(size_t)blockIdx.x * np + i];
+  const double s = block_sum(acc, red);
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
+}
+
+// Y[:, j] = X[:, j] s_j
+__global__ void scale_cols_to_kernel(const double* __restrict__ X, int n, const double* __restrict__ s,
+                                     double* __restrict__ Y) {
+  const double f = s[blockIdx.x];
+  const size_t o = (size_t)blockIdx.x * n;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) Y[o + i] = f * X[o + i];
 }
 
 __global__ void col_norms_kernel(const double* __restrict__ X, int n, double* __restrict__ nrm) {
@@ -336,11 +468,13 @@ __global__ void double_layer_back_kernel(const double* __restrict__ A, int d, in
 
 }  // namespace
 
-void k_sym_add(const double* X, int n, double* Y, hipStream_t s) {
+template <typename T> void k_sym_add(const T* X, int n, double* Y, hipStream_t s) {
   dim3 g((n + 31) / 32, (n + 31) / 32);
-  hipLaunchKernelGGL(sym_add_kernel, g, dim3(256), 0, s, X, n, Y);
+  hipLaunchKernelGGL(sym_add_kernel<T>, g, dim3(256), 0, s, X, n, Y);
   TNAD_HIP_TRY(hipGetLastError());
 }
+template void k_sym_add<double>(const double*, int, double*, hipStream_t);
+template void k_sym_add<float>(const float*, int, double*, hipStream_t);
 template <typename T> void k_cast(const T* src, double* dst, size_t n, hipStream_t s) {
   hipLaunchKernelGGL((cast_kernel<T, double>), dim3(nblk(n)), dim3(NT), 0, s, src, dst, n);
   TNAD_HIP_TRY(hipGetLastError());
@@ -357,7 +491,10 @@ void k_fill(double* x, size_t n, double v, hipStream_t s) {
   TNAD_HIP_TRY(hipGetLastError());
 }
 void k_copy(const double* x, double* y, size_t n, hipStream_t s) {
-  TNAD_HIP_TRY(hipMemcpyAsync(y, x, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+  // (a kernel: the runtime's device-to-device copy costs the host about 10 us per call, a launch 4)
+  if (n == 0) return;
+  hipLaunchKernelGGL(copy_kernel, dim3(std::min(nblk(n), 4096u)), dim3(NT), 0, s, x, y, n);
+  TNAD_HIP_TRY(hipGetLastError());
 }
 void k_axpby(double a, const double* x, double b, double* y, size_t n, hipStream_t s) {
   hipLaunchKernelGGL(axpby_kernel, dim3(nblk(n)), dim3(NT), 0, s, a, x, b, y, n);
@@ -367,16 +504,58 @@ void k_scale_by_dev(double* x, size_t n, const double* nrm, hipStream_t s) {
   hipLaunchKernelGGL(scale_by_dev_kernel, dim3(nblk(n)), dim3(NT), 0, s, x, n, nrm);
   TNAD_HIP_TRY(hipGetLastError());
 }
-// out must point at a buffer of at least RED_BLOCKS + 1 doubles; the result lands in out[0].
-void k_dot(const double* x, const double* y, size_t n, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(dot_partial_kernel, dim3(RED_BLOCKS), dim3(NT), 0, s, x, y, n, out + 1);
-  hipLaunchKernelGGL(final_sum_kernel, dim3(1), dim3(NT), 0, s, out + 1, RED_BLOCKS, out);
+// Reductions: up to RED_ONE elements one workgroup of 1024 threads sums directly (one launch), above RED_BLOCKS
+// partial sums and a final one.
+constexpr size_t RED_ONE = 16384;
+void k_dot_to(const double* x, const double* y, size_t n, double* scratch, double* out, hipStream_t s) {
+  if (n <= RED_ONE) {
+    hipLaunchKernelGGL(dot_partial_kernel, dim3(1), dim3(1024), 0, s, x, y, n, out);
+  } else {
+    hipLaunchKernelGGL(dot_partial_kernel, dim3(RED_BLOCKS), dim3(NT), 0, s, x, y, n, scratch);
+    hipLaunchKernelGGL(final_sum_kernel, dim3(1), dim3(NT), 0, s, scratch, RED_BLOCKS, out);
+  }
   TNAD_HIP_TRY(hipGetLastError());
 }
+// out must point at a buffer of at least RED_BLOCKS + 1 doubles; the result lands in out[0].
+void k_dot(const double* x, const double* y, size_t n, double* out, hipStream_t s) {
+  k_dot_to(x, y, n, out + 1, out, s);
+}
 void k_sumsq(const double* x, size_t n, double* out, hipStream_t s) { k_dot(x, nullptr, n, out, s); }
-void k_edge_sym(const double* T1, int chi, int D, double* T2, hipStream_t s) {
-  size_t n = (size_t)chi * D * chi;
-  hipLaunchKernelGGL(edge_sym_kernel, dim3(nblk(n)), dim3(NT), 0, s, T1, chi, D, T2);
+void k_diff_sumsq(const double* M, const double* P, size_t n, double* scratch, double* out, hipStream_t s) {
+  hipLaunchKernelGGL(diff_sumsq_kernel, dim3(RED_BLOCKS), dim3(1024), 0, s, M, P, n, scratch);
+  hipLaunchKernelGGL(final_sums_kernel, dim3(2), dim3(NT), 0, s, scratch, RED_BLOCKS, out);
+  TNAD_HIP_TRY(hipGetLastError());
+}
+void k_scale_rsqrt(const double* x, size_t n, const double* sumsq, double* y, hipStream_t s) {
+  hipLaunchKernelGGL(scale_rsqrt_kernel, dim3(std::min(nblk(n), 4096u)), dim3(NT), 0, s, x, n, sumsq, y);
+  TNAD_HIP_TRY(hipGetLastError());
+}
+void k_scale_cols_to(const double* X, int n, int k, const double* scale, double* Y, hipStream_t s) {
+  hipLaunchKernelGGL(scale_cols_to_kernel, dim3(k), dim3(NT), 0, s, X, n, scale, Y);
+  TNAD_HIP_TRY(hipGetLastError());
+}
+// blocks of the two-launch pairs: at most NT partial sums, summed again by every block of the second launch
+static unsigned pair_blocks(size_t n) { return std::min(nblk(n), (unsigned)NT); }
+template <typename T>
+void k_step_end(const T* T1, int chi, int D, const double* C2, double* T2, double* scratch, double* nrm, double* C3,
+                double* T3, hipStream_t s) {
+  const size_t nT = (size_t)chi * D * chi, nC = (size_t)chi * chi;
+  const unsigned np = pair_blocks(nT);
+  hipLaunchKernelGGL(edge_sym_norms_kernel<T>, dim3(np), dim3(NT), 0, s, T1, chi, D, T2, C2, scratch);
+  hipLaunchKernelGGL(normalize_pair_kernel, dim3(np), dim3(NT), 0, s, C2, nC, T2, nT, scratch, (int)np, nrm, C3, T3);
+  TNAD_HIP_TRY(hipGetLastError());
+}
+template void k_step_end<double>(const double*, int, int, const double*, double*, double*, double*, double*, double*,
+                                 hipStream_t);
+template void k_step_end<float>(const float*, int, int, const double*, double*, double*, double*, double*, double*,
+                                hipStream_t);
+void k_step_end_back(const double* C2, const double* C3bar, const double* T2, const double* T3bar, int chi, int D,
+                     const double* nrm, double* scratch, double* C1bar, double* T1bar, hipStream_t s) {
+  const size_t nT = (size_t)chi * D * chi, nC = (size_t)chi * chi;
+  const unsigned np = pair_blocks(nT);
+  hipLaunchKernelGGL(norm_dots_kernel, dim3(np), dim3(NT), 0, s, C2, C3bar, nC, T2, T3bar, nT, scratch);
+  hipLaunchKernelGGL(norm_sym_back_kernel, dim3(np), dim3(NT), 0, s, C2, C3bar, T2, T3bar, chi, D, nrm, scratch,
+                     (int)np, C1bar, T1bar);
   TNAD_HIP_TRY(hipGetLastError());
 }
 void k_col_norms(const double* X, int n, int k, double* nrm, hipStream_t s) {

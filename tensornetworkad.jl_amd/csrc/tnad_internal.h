@@ -133,7 +133,7 @@ void chol_inv(const double* G, int m, double shift, double* Rinv, int* info, dou
 // ---------------------------------------------------------------------------
 // Elementwise / reduction kernels (elem.hip)
 // ---------------------------------------------------------------------------
-void k_sym_add(const double* X, int n, double* Y, hipStream_t s);              // Y = X + X^T
+template <typename T> void k_sym_add(const T* X, int n, double* Y, hipStream_t s);   // Y = X + X^T (T: double, float)
 template <typename T> void k_cast(const T* src, double* dst, size_t n, hipStream_t s);
 template <typename T> void k_cast_from(const double* src, T* dst, size_t n, hipStream_t s);
 void k_fill(double* x, size_t n, double v, hipStream_t s);
@@ -142,7 +142,19 @@ void k_axpby(double a, const double* x, double b, double* y, size_t n, hipStream
 void k_scale_by_dev(double* x, size_t n, const double* nrm, hipStream_t s);   // x /= *nrm
 void k_sumsq(const double* x, size_t n, double* out, hipStream_t s);           // *out = sum x^2 (atomic-free 2 pass)
 void k_dot(const double* x, const double* y, size_t n, double* out, hipStream_t s);
-void k_edge_sym(const double* T1, int chi, int D, double* T2, hipStream_t s);  // T2 = T1 + T1^{kji}
+// the same into *out, with scratch for 256 doubles
+void k_dot_to(const double* x, const double* y, size_t n, double* scratch, double* out, hipStream_t s);
+// out[0] = |M - P|_F^2, out[1] = |M|_F^2 (scratch: 512 doubles)
+void k_diff_sumsq(const double* M, const double* P, size_t n, double* scratch, double* out, hipStream_t s);
+void k_scale_rsqrt(const double* x, size_t n, const double* sumsq, double* y, hipStream_t s);   // y = x / sqrt(*sumsq)
+void k_scale_cols_to(const double* X, int n, int k, const double* scale, double* Y, hipStream_t s);   // Y_j = scale_j X_j
+// T2 = T1 + T1^{kji}, nrm = (|C2|, |T2|), C3 = C2 / |C2|, T3 = T2 / |T2| (scratch: 512 doubles; T: double, float)
+template <typename T>
+void k_step_end(const T* T1, int chi, int D, const double* C2, double* T2, double* scratch, double* nrm, double* C3,
+                double* T3, hipStream_t s);
+// its adjoint: cotangents of C3 and T3 -> of the unsymmetrised corner and edge (nrm from k_step_end)
+void k_step_end_back(const double* C2, const double* C3bar, const double* T2, const double* T3bar, int chi, int D,
+                     const double* nrm, double* scratch, double* C1bar, double* T1bar, hipStream_t s);
 void k_col_norms(const double* X, int n, int k, double* nrm, hipStream_t s);
 void k_scale_cols(double* X, int n, int k, const double* scale, int invert, hipStream_t s);
 // Column norms into nrm; every column whose norm is <= rel * max norm refilled with hash-random entries;
