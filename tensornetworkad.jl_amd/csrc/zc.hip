@@ -30,6 +30,7 @@
 
 #include "api_internal.h"
 #include "ctmrg.h"
+#include "dpp.h"
 #include "zc.h"
 
 namespace tnad {
@@ -114,100 +115,114 @@ __device__ __forceinline__ double phase_weight(int r) {
 // Complex eigenvectors of H from the eigenpairs (ev2, V2) of its real embedding (2n of them, sorted by
 // |lambda| descending): candidates in order, each orthogonalised against the vectors taken so far (two
 // passes of classical Gram-Schmidt), taken when at least half of its norm remains, until n are taken;
-// then the phase rule.  One workgroup.  U: planar n x n; lam: n.
-constexpr int ZX_NT = 256;
+// then the phase rule.  U: planar n x n; lam: n.
+// The candidates depend on each other, so this is one workgroup; the vectors taken so far stay in its LDS
+// (148 KB at n = 96, odd pitch), 16 lanes share each coefficient and 8 each row of an update, and every wavefront
+// forms the norms and the phase sum for itself, so a pass costs two barriers; a candidate that has lost its norm
+// after the first pass (the i x partner of a taken vector) skips the second.  Bound by these ~500-cycle phases:
+// 1441 -> 217 us at n = 48 (before: U in global memory, a serial loop of n per coefficient).
+constexpr int ZX_NT = 1024;
+constexpr int ZX_MAX = JACOBI_MAX / 2;
+static size_t zeig_lds(int n) { return (2 * (size_t)n * (n | 1) + 4 * ZX_MAX) * sizeof(double); }
 __global__ __launch_bounds__(ZX_NT) void zeig_extract_kernel(const double* __restrict__ V2,
                                                               const double* __restrict__ ev2, int n,
                                                               double* __restrict__ U, double* __restrict__ lam) {
-  __shared__ double xr[96], xi[96], cr[96], ci[96];
-  __shared__ double red[8];
-  __shared__ int taken_s;
-  const int t = threadIdx.x;
-  const int m = 2 * n;
+  extern __shared__ double zx[];
+  const int t = threadIdx.x, lane = t & 63, m = 2 * n, p = n | 1;
+  double* ur = zx;
+  double* ui = ur + n * p;
+  double* xr = ui + n * p;
+  double* xi = xr + ZX_MAX;
+  double* cr = xi + ZX_MAX;
+  double* ci = cr + ZX_MAX;
   const size_t nn = (size_t)n * n;
-  if (t == 0) taken_s = 0;
-  __syncthreads();
-  for (int cand = 0; cand < m; ++cand) {
-    const int taken = taken_s;
-    if (taken >= n) break;
-    for (int r = t; r < n; r += ZX_NT) {
-      xr[r] = V2[r + (size_t)m * cand];
-      xi[r] = V2[n + r + (size_t)m * cand];
-    }
+  int taken = 0;   // the same in every thread
+  double next = t < m ? V2[t] : 0.0;
+  for (int cand = 0; cand < m && taken < n; ++cand) {
+    if (t < m) (t < n ? xr[t] : xi[t - n]) = next;
+    if (t < m && cand + 1 < m) next = V2[t + (size_t)m * (cand + 1)];
     __syncthreads();
+    double nrm2 = 0.0;
     for (int pass = 0; pass < 2; ++pass) {
       // c_a = u_a^H x
-      for (int a = t; a < taken; a += ZX_NT) {
-        double sr = 0.0, si = 0.0;
-        for (int r = 0; r < n; ++r) {
-          const double ur = U[r + (size_t)n * a], ui = U[nn + r + (size_t)n * a];
-          sr += ur * xr[r] + ui * xi[r];
-          si += ur * xi[r] - ui * xr[r];
+      for (int a = t >> 4; a < taken; a += ZX_NT / 16) {
+        double sum[2] = {0.0, 0.0};
+        for (int r = t & 15; r < n; r += 16) {
+          const double x = ur[a * p + r], y = ui[a * p + r];
+          sum[0] += x * xr[r] + y * xi[r];
+          sum[1] += x * xi[r] - y * xr[r];
         }
-        cr[a] = sr;
-        ci[a] = si;
+        row16_sums<2>(sum);
+        if ((t & 15) == 0) {
+          cr[a] = sum[0];
+          ci[a] = sum[1];
+        }
       }
       __syncthreads();
       // x -= sum_a c_a u_a
-      for (int r = t; r < n; r += ZX_NT) {
-        double vr = xr[r], vi = xi[r];
-        for (int a = 0; a < taken; ++a) {
-          const double ur = U[r + (size_t)n * a], ui = U[nn + r + (size_t)n * a];
-          vr -= cr[a] * ur - ci[a] * ui;
-          vi -= cr[a] * ui + ci[a] * ur;
+      const int r = t >> 3;
+      if (r < n) {
+        double vr = 0.0, vi = 0.0;
+        for (int a = t & 7; a < taken; a += 8) {
+          const double x = ur[a * p + r], y = ui[a * p + r];
+          vr += cr[a] * x - ci[a] * y;
+          vi += cr[a] * y + ci[a] * x;
         }
-        xr[r] = vr;
-        xi[r] = vi;
+        vr += dpp_d<0xB1>(vr);
+        vi += dpp_d<0xB1>(vi);
+        vr += dpp_d<0x4E>(vr);
+        vi += dpp_d<0x4E>(vi);
+        vr += dpp_d<0x141>(vr);
+        vi += dpp_d<0x141>(vi);
+        if ((t & 7) == 0) {
+          xr[r] -= vr;
+          xi[r] -= vi;
+        }
       }
       __syncthreads();
+      nrm2 = 0.0;
+      for (int q = lane; q < n; q += 64) nrm2 += xr[q] * xr[q] + xi[q] * xi[q];
+      nrm2 = wave_sum(nrm2);
+      if (!(nrm2 > 0.25)) break;   // a further pass only shortens it
     }
-    double acc = 0.0;
-    for (int r = t; r < n; r += ZX_NT) acc += xr[r] * xr[r] + xi[r] * xi[r];
-    const double nrm2 = zblock_sum(acc, red);
     if (nrm2 > 0.25) {
       // phase rule
       double qr = 0.0, qi = 0.0;
-      for (int r = t; r < n; r += ZX_NT) {
+      for (int r = lane; r < n; r += 64) {
         const double w = phase_weight(r);
         qr += w * xr[r];
         qi += w * xi[r];
       }
-      qr = zblock_sum(qr, red);
-      qi = zblock_sum(qi, red);
+      qr = wave_sum(qr);
+      qi = wave_sum(qi);
       const double nrm = sqrt(nrm2);
       if (sqrt(qr * qr + qi * qi) <= 1e-6 * nrm) {
-        if (t == 0) {
-          int best = 0;
-          double bv = -1.0;
-          for (int r = 0; r < n; ++r) {
-            const double v = xr[r] * xr[r] + xi[r] * xi[r];
-            if (v > bv) { bv = v; best = r; }
-          }
-          cr[0] = xr[best];
-          ci[0] = xi[best];
+        int best = 0;
+        double bv = -1.0;
+        for (int r = 0; r < n; ++r) {
+          const double v = xr[r] * xr[r] + xi[r] * xi[r];
+          if (v > bv) { bv = v; best = r; }
         }
-        __syncthreads();
-        qr = cr[0];
-        qi = ci[0];
-        __syncthreads();
+        qr = xr[best];
+        qi = xi[best];
       }
       const double qa = sqrt(qr * qr + qi * qi);
       // x <- x conj(q) / (|q| |x|)
       const double pr = qa > 0.0 ? qr / qa : 1.0, pi = qa > 0.0 ? -qi / qa : 0.0;
-      for (int r = t; r < n; r += ZX_NT) {
-        const double vr = xr[r] / nrm, vi = xi[r] / nrm;
-        U[r + (size_t)n * taken] = vr * pr - vi * pi;
-        U[nn + r + (size_t)n * taken] = vr * pi + vi * pr;
+      if (t < n) {
+        const double vr = xr[t] / nrm, vi = xi[t] / nrm;
+        const double yr = vr * pr - vi * pi, yi = vr * pi + vi * pr;
+        ur[taken * p + t] = yr;
+        ui[taken * p + t] = yi;
+        U[t + (size_t)n * taken] = yr;
+        U[nn + t + (size_t)n * taken] = yi;
       }
-      if (t == 0) {
-        lam[taken] = ev2[cand];
-        taken_s = taken + 1;
-      }
+      if (t == 0) lam[taken] = ev2[cand];
+      ++taken;
     }
     __syncthreads();
   }
   // fewer than n taken only through rounding trouble: leave the rest zero
-  const int taken = taken_s;
   for (size_t e = (size_t)taken * n + t; e < nn; e += ZX_NT) {
     U[e] = 0.0;
     U[nn + e] = 0.0;
@@ -648,7 +663,10 @@ void z_heig(Ctx* c, const double* H, int n, double* U, double* lam) {
   hipLaunchKernelGGL(realify_kernel, dim3(nb((size_t)m * m)), dim3(NT), 0, s, H, n, R.as<double>());
   TNAD_HIP_TRY(hipGetLastError());
   syev_dc(R.as<double>(), m, m, ev2.as<double>(), V2.as<double>(), work.as<double>(), s);
-  hipLaunchKernelGGL(zeig_extract_kernel, dim3(1), dim3(ZX_NT), 0, s, V2.as<double>(), ev2.as<double>(), n, U, lam);
+  const size_t lds = zeig_lds(n);
+  TNAD_HIP_TRY(hipFuncSetAttribute((const void*)zeig_extract_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)lds));
+  hipLaunchKernelGGL(zeig_extract_kernel, dim3(1), dim3(ZX_NT), lds, s, V2.as<double>(), ev2.as<double>(), n, U, lam);
   TNAD_HIP_TRY(hipGetLastError());
 }
 
