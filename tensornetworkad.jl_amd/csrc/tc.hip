@@ -53,9 +53,10 @@ constexpr int TC_BK = 16, TC_BK_DEEP = 32, TC_DEEP_BELOW = 256;
 constexpr int TC_BIG_MIN_WG = 1024;  // 128 x 128 tiles only at 4+ workgroups per CU (slower at 1 per CU)
 constexpr int TC_SMALL_BELOW = 128;  // 32 x 32 tiles below this many 64 x 64 workgroups
 
-__device__ __forceinline__ long long off2(int i, int I0, long long s0, long long s1) {
-  int i0 = i % I0;
-  int i1 = i / I0;
+__device__ __forceinline__ int fdiv(int x, const FDiv& f) { return (int)((__umulhi((unsigned)x, f.mul) + (unsigned)x) >> f.sh); }
+
+__device__ __forceinline__ long long off2(int i, int I0, const FDiv& f, long long s0, long long s1) {
+  const int i1 = fdiv(i, f), i0 = i - i1 * I0;
   return (long long)i0 * s0 + (long long)i1 * s1;
 }
 
@@ -64,9 +65,10 @@ __device__ __forceinline__ long long off2(int i, int I0, long long s0, long long
 struct KPos {
   int k0;
   long long off;
-  __device__ __forceinline__ void init(int k, int K0, long long s0, long long s1) {
-    k0 = k % K0;
-    off = (long long)k0 * s0 + (long long)(k / K0) * s1;
+  __device__ __forceinline__ void init(int k, int K0, const FDiv& f, long long s0, long long s1) {
+    const int k1 = fdiv(k, f);
+    k0 = k - k1 * K0;
+    off = (long long)k0 * s0 + (long long)k1 * s1;
   }
   __device__ __forceinline__ void advance(int step, int K0, long long s0, long long delta) {
     k0 += step;
@@ -142,7 +144,7 @@ __global__ __launch_bounds__(NT, PF == 2 ? (sizeof(T) == 8 ? 3 : 4) : 1) void tc
     else         { a_ki[r] = t % BK; a_mi[r] = t / BK + (NT / BK) * r; }
     int m = tile_m + a_mi[r];
     a_mok[r] = m < M;
-    a_moff[r] = a_mok[r] ? off2(m, d.M0, d.am0, d.am1) : 0;
+    a_moff[r] = a_mok[r] ? off2(m, d.M0, d.fm, d.am0, d.am1) : 0;
   }
   // B loader mapping
   const bool b_nfast = (d.bn0 == 1 && d.N0 > 1) || d.bk0 != 1;
@@ -155,7 +157,7 @@ __global__ __launch_bounds__(NT, PF == 2 ? (sizeof(T) == 8 ? 3 : 4) : 1) void tc
     else         { b_ki[r] = t % BK; b_ni[r] = t / BK + (NT / BK) * r; }
     int n = tile_n + b_ni[r];
     b_nok[r] = n < N;
-    b_noff[r] = b_nok[r] ? off2(n, d.N0, d.bn0, d.bn1) : 0;
+    b_noff[r] = b_nok[r] ? off2(n, d.N0, d.fn, d.bn0, d.bn1) : 0;
   }
 
   T ra0[NR], rb0[NR], ra1[NR], rb1[NR];
@@ -163,8 +165,8 @@ __global__ __launch_bounds__(NT, PF == 2 ? (sizeof(T) == 8 ? 3 : 4) : 1) void tc
   const long long a_dk = d.ak1 - (long long)d.K0 * d.ak0, b_dk = d.bk1 - (long long)d.K0 * d.bk0;
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
-    a_kp[r].init(kbeg + a_ki[r], d.K0, d.ak0, d.ak1);
-    b_kp[r].init(kbeg + b_ki[r], d.K0, d.bk0, d.bk1);
+    a_kp[r].init(kbeg + a_ki[r], d.K0, d.fk, d.ak0, d.ak1);
+    b_kp[r].init(kbeg + b_ki[r], d.K0, d.fk, d.bk0, d.bk1);
   }
   // loads the K-tile starting at k0 into (xa, xb), then moves the loaders one tile on (tiles are
   // loaded in order)
@@ -261,7 +263,7 @@ __global__ __launch_bounds__(NT, PF == 2 ? (sizeof(T) == 8 ? 3 : 4) : 1) void tc
   for (int j = 0; j < FB; ++j) {
     int n = tile_n + wn * (TILE / 2) + j * 16 + (lane & 15);
     if (n >= N) continue;
-    long long noff = off2(n, d.N0, d.cn0, d.cn1);
+    long long noff = off2(n, d.N0, d.fn, d.cn0, d.cn1);
 #pragma unroll
     for (int i = 0; i < FB; ++i) {
 #pragma unroll
@@ -272,7 +274,7 @@ __global__ __launch_bounds__(NT, PF == 2 ? (sizeof(T) == 8 ? 3 : 4) : 1) void tc
           Wz[m + (size_t)M * n] = (T)acc[i][j][r];
           continue;
         }
-        long long o = noff + off2(m, d.M0, d.cm0, d.cm1);
+        long long o = noff + off2(m, d.M0, d.fm, d.cm0, d.cm1);
         T v = alpha * (T)acc[i][j][r];
         if (d.beta != 0.0) v += beta * C[o];
         C[o] = v;
@@ -344,10 +346,10 @@ __global__ __launch_bounds__(NT, TILE == 128 ? 1 : (sizeof(T) == 8 ? 3 : 4)) voi
     const int m = tile_m + a_m[r], n = tile_n + b_n[r];
     a_ok[r] = m < M;
     b_ok[r] = n < N;
-    a_off[r] = a_ok[r] ? off2(m, d.M0, d.am0, d.am1) : 0;
-    b_off[r] = b_ok[r] ? off2(n, d.N0, d.bn0, d.bn1) : 0;
-    a_kp[r].init(kbeg + a_k[r], d.K0, d.ak0, d.ak1);
-    b_kp[r].init(kbeg + b_k[r], d.K0, d.bk0, d.bk1);
+    a_off[r] = a_ok[r] ? off2(m, d.M0, d.fm, d.am0, d.am1) : 0;
+    b_off[r] = b_ok[r] ? off2(n, d.N0, d.fn, d.bn0, d.bn1) : 0;
+    a_kp[r].init(kbeg + a_k[r], d.K0, d.fk, d.ak0, d.ak1);
+    b_kp[r].init(kbeg + b_k[r], d.K0, d.fk, d.bk0, d.bk1);
   }
   // loads of one K-tile (live: a K-tile inside [kbeg, K)).  A slot outside the output tile, or any slot of a
   // dead tile, reads the operand's first vector instead, so the loop body stays free of branches: such
@@ -431,7 +433,7 @@ __global__ __launch_bounds__(NT, TILE == 128 ? 1 : (sizeof(T) == 8 ? 3 : 4)) voi
   for (int j = 0; j < FB; ++j) {
     int n = tile_n + wn * (TILE / 2) + j * 16 + (lane & 15);
     if (n >= N) continue;
-    long long noff = off2(n, d.N0, d.cn0, d.cn1);
+    long long noff = off2(n, d.N0, d.fn, d.cn0, d.cn1);
 #pragma unroll
     for (int i = 0; i < FB; ++i) {
 #pragma unroll
@@ -442,12 +444,118 @@ __global__ __launch_bounds__(NT, TILE == 128 ? 1 : (sizeof(T) == 8 ? 3 : 4)) voi
           Wz[m + (size_t)M * n] = (T)acc[i][j][r];
           continue;
         }
-        long long o = noff + off2(m, d.M0, d.cm0, d.cm1);
+        long long o = noff + off2(m, d.M0, d.fm, d.cm0, d.cm1);
         T v = alpha * (T)acc[i][j][r];
         if (d.beta != 0.0) v += beta * C[o];
         C[o] = v;
       }
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Complex FP64 kernel for small outputs: both planes of both operands staged together, 32 x 32 output tile per
+// workgroup, each of the 4 waves one 16 x 16 block with three accumulators (Ar Br, Ai Bi, Ar Bi + Ai Br), K-tile 16,
+// double-buffered LDS (49 KB).  A complex contraction of the sizes the complex path runs (corner matrix up to
+// 96 x 96) is bound by launch and latency, not by its products: as four real launches, two of them reading back
+// the output, it took 4 x 5.3 us.
+// ---------------------------------------------------------------------------
+constexpr int ZT = 32, ZBK = 16;
+__global__ __launch_bounds__(NT) void ztc_kernel(TcDesc d, const double* __restrict__ A, long long pA, double sa,
+                                                 const double* __restrict__ B, long long pB, double sb,
+                                                 double* __restrict__ C, long long pC) {
+  constexpr int PAD = 16, NR = ZT * ZBK / NT;   // loads per thread, operand and plane per K-tile (2)
+  __shared__ double As[2][2][ZBK][ZT + PAD];    // [buffer][plane]
+  __shared__ double Bs[2][2][ZBK][ZT + PAD];
+  const int M = d.M0 * d.M1, N = d.N0 * d.N1, K = d.K0 * d.K1;
+  const int tile_m = blockIdx.x * ZT, tile_n = blockIdx.y * ZT;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave & 1, wn = wave >> 1;
+  const bool a_mfast = (d.am0 == 1 && d.M0 > 1) || d.ak0 != 1;
+  const bool b_nfast = (d.bn0 == 1 && d.N0 > 1) || d.bk0 != 1;
+  int a_mi[NR], a_ki[NR], b_ni[NR], b_ki[NR];
+  long long a_off[NR], b_off[NR];
+  bool a_ok[NR], b_ok[NR];
+  KPos a_kp[NR], b_kp[NR];
+  const long long a_dk = d.ak1 - (long long)d.K0 * d.ak0, b_dk = d.bk1 - (long long)d.K0 * d.bk0;
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    if (a_mfast) { a_mi[r] = t % ZT; a_ki[r] = t / ZT + (NT / ZT) * r; }
+    else         { a_ki[r] = t % ZBK; a_mi[r] = t / ZBK + (NT / ZBK) * r; }
+    if (b_nfast) { b_ni[r] = t % ZT; b_ki[r] = t / ZT + (NT / ZT) * r; }
+    else         { b_ki[r] = t % ZBK; b_ni[r] = t / ZBK + (NT / ZBK) * r; }
+    const int m = tile_m + a_mi[r], n = tile_n + b_ni[r];
+    a_ok[r] = m < M;
+    b_ok[r] = n < N;
+    a_off[r] = a_ok[r] ? off2(m, d.M0, d.fm, d.am0, d.am1) : 0;
+    b_off[r] = b_ok[r] ? off2(n, d.N0, d.fn, d.bn0, d.bn1) : 0;
+    a_kp[r].init(a_ki[r], d.K0, d.fk, d.ak0, d.ak1);
+    b_kp[r].init(b_ki[r], d.K0, d.fk, d.bk0, d.bk1);
+  }
+  double ra[2][NR], rb[2][NR];
+  auto gload = [&](int k0) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      ra[0][r] = ra[1][r] = rb[0][r] = rb[1][r] = 0.0;
+      if (a_ok[r] && k0 + a_ki[r] < K) {
+        const long long o = a_off[r] + a_kp[r].off;
+        ra[0][r] = A[o];
+        ra[1][r] = sa * A[o + pA];
+      }
+      if (b_ok[r] && k0 + b_ki[r] < K) {
+        const long long o = b_off[r] + b_kp[r].off;
+        rb[0][r] = B[o];
+        rb[1][r] = sb * B[o + pB];
+      }
+      a_kp[r].advance(ZBK, d.K0, d.ak0, a_dk);
+      b_kp[r].advance(ZBK, d.K0, d.bk0, b_dk);
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        As[buf][q][a_ki[r]][a_mi[r]] = ra[q][r];
+        Bs[buf][q][b_ki[r]][b_ni[r]] = rb[q][r];
+      }
+  };
+  d4 rr = {0, 0, 0, 0}, ii = {0, 0, 0, 0}, ri = {0, 0, 0, 0};
+  gload(0);
+  stage(0);
+  if (ZBK < K) gload(ZBK);
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += ZBK, buf ^= 1) {
+#pragma unroll
+    for (int kk = 0; kk < ZBK; kk += 4) {
+      const int row = kk + (lane >> 4), ca = wm * 16 + (lane & 15), cb = wn * 16 + (lane & 15);
+      const double ar = As[buf][0][row][ca], ai = As[buf][1][row][ca], br = Bs[buf][0][row][cb], bi = Bs[buf][1][row][cb];
+      rr = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, rr, 0, 0, 0);
+      ii = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bi, ii, 0, 0, 0);
+      ri = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, ri, 0, 0, 0);
+      ri = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, ri, 0, 0, 0);
+    }
+    if (k0 + ZBK < K) {
+      stage(buf ^ 1);
+      if (k0 + 2 * ZBK < K) gload(k0 + 2 * ZBK);
+    }
+    __syncthreads();
+  }
+  const int n = tile_n + wn * 16 + (lane & 15);
+  if (n >= N) return;
+  const long long noff = off2(n, d.N0, d.fn, d.cn0, d.cn1);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int m = tile_m + wm * 16 + MfmaOp<double>::row(lane, r);
+    if (m >= M) continue;
+    const long long o = noff + off2(m, d.M0, d.fm, d.cm0, d.cm1);
+    double vr = d.alpha * (rr[r] - ii[r]), vi = d.alpha * ri[r];
+    if (d.beta != 0.0) {
+      vr += d.beta * C[o];
+      vi += d.beta * C[o + pC];
+    }
+    C[o] = vr;
+    C[o + pC] = vi;
   }
 }
 
@@ -463,12 +571,12 @@ __global__ __launch_bounds__(NT) void tc_splitk_reduce(TcDesc d, const T* __rest
   const int M = d.M0 * d.M1, N = d.N0 * d.N1;
   const size_t MN = (size_t)M * N;
   for (int n = blockIdx.y; n < N; n += gridDim.y) {
-    const long long on = off2(n, d.N0, d.cn0, d.cn1);
+    const long long on = off2(n, d.N0, d.fn, d.cn0, d.cn1);
     for (int m = blockIdx.x * NT + threadIdx.x; m < M; m += gridDim.x * NT) {
       const size_t e = (size_t)m + (size_t)M * n;
       double acc = 0.0;
       for (int s = 0; s < nsplit; ++s) acc += (double)Wsp[e + (size_t)s * MN];
-      const long long o = (d.M1 == 1 ? (long long)m * d.cm0 : off2(m, d.M0, d.cm0, d.cm1)) + on;
+      const long long o = (d.M1 == 1 ? (long long)m * d.cm0 : off2(m, d.M0, d.fm, d.cm0, d.cm1)) + on;
       double v = d.alpha * acc;
       if (d.beta != 0.0) v += d.beta * (double)C[o];
       C[o] = (T)v;
@@ -520,7 +628,7 @@ __global__ __launch_bounds__(NT) void tc_kernel_bf16(TcDesc d, const float* __re
     else         { a_ki[r] = t & 31; a_mi[r] = (t >> 5) + 8 * r; }
     int m = tile_m + a_mi[r];
     a_mok[r] = m < M;
-    a_moff[r] = a_mok[r] ? off2(m, d.M0, d.am0, d.am1) : 0;
+    a_moff[r] = a_mok[r] ? off2(m, d.M0, d.fm, d.am0, d.am1) : 0;
   }
   const bool b_nfast = (d.bn0 == 1 && d.N0 > 1) || d.bk0 != 1;
   int b_ni[8], b_ki[8];
@@ -532,15 +640,15 @@ __global__ __launch_bounds__(NT) void tc_kernel_bf16(TcDesc d, const float* __re
     else         { b_ki[r] = t & 31; b_ni[r] = (t >> 5) + 8 * r; }
     int n = tile_n + b_ni[r];
     b_nok[r] = n < N;
-    b_noff[r] = b_nok[r] ? off2(n, d.N0, d.bn0, d.bn1) : 0;
+    b_noff[r] = b_nok[r] ? off2(n, d.N0, d.fn, d.bn0, d.bn1) : 0;
   }
   float ra[8], rb[8];
   KPos a_kp[8], b_kp[8];
   const long long a_dk = d.ak1 - (long long)d.K0 * d.ak0, b_dk = d.bk1 - (long long)d.K0 * d.bk0;
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
-    a_kp[r].init(kbeg + a_ki[r], d.K0, d.ak0, d.ak1);
-    b_kp[r].init(kbeg + b_ki[r], d.K0, d.bk0, d.bk1);
+    a_kp[r].init(kbeg + a_ki[r], d.K0, d.fk, d.ak0, d.ak1);
+    b_kp[r].init(kbeg + b_ki[r], d.K0, d.fk, d.bk0, d.bk1);
   }
   // loads the K-tile starting at k0, then moves the loaders one tile on
   auto gload = [&](int k0) {
@@ -597,7 +705,7 @@ __global__ __launch_bounds__(NT) void tc_kernel_bf16(TcDesc d, const float* __re
   for (int j = 0; j < 2; ++j) {
     int n = tile_n + wn * 32 + j * 16 + (lane & 15);
     if (n >= N) continue;
-    long long noff = off2(n, d.N0, d.cn0, d.cn1);
+    long long noff = off2(n, d.N0, d.fn, d.cn0, d.cn1);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
 #pragma unroll
@@ -608,7 +716,7 @@ __global__ __launch_bounds__(NT) void tc_kernel_bf16(TcDesc d, const float* __re
           Wz[m + (size_t)M * n] = acc[i][j][r];
           continue;
         }
-        long long o = noff + off2(m, d.M0, d.cm0, d.cm1);
+        long long o = noff + off2(m, d.M0, d.fm, d.cm0, d.cm1);
         float v = alpha * acc[i][j][r];
         if (d.beta != 0.0) v += beta * C[o];
         C[o] = v;
@@ -665,10 +773,10 @@ __global__ __launch_bounds__(NT, 4) void tc_kernel_vec_bf16(TcDesc d, const floa
     const int m = tile_m + a_m[r], n = tile_n + b_n[r];
     a_ok[r] = m < M;
     b_ok[r] = n < N;
-    a_off[r] = a_ok[r] ? off2(m, d.M0, d.am0, d.am1) : 0;
-    b_off[r] = b_ok[r] ? off2(n, d.N0, d.bn0, d.bn1) : 0;
-    a_kp[r].init(kbeg + a_k[r], d.K0, d.ak0, d.ak1);
-    b_kp[r].init(kbeg + b_k[r], d.K0, d.bk0, d.bk1);
+    a_off[r] = a_ok[r] ? off2(m, d.M0, d.fm, d.am0, d.am1) : 0;
+    b_off[r] = b_ok[r] ? off2(n, d.N0, d.fn, d.bn0, d.bn1) : 0;
+    a_kp[r].init(kbeg + a_k[r], d.K0, d.fk, d.ak0, d.ak1);
+    b_kp[r].init(kbeg + b_k[r], d.K0, d.fk, d.bk0, d.bk1);
   }
   auto gload = [&](f4 (&xa)[NVEC], f4 (&xb)[NVEC], bool live) {
 #pragma unroll
@@ -743,7 +851,7 @@ __global__ __launch_bounds__(NT, 4) void tc_kernel_vec_bf16(TcDesc d, const floa
   for (int j = 0; j < FB; ++j) {
     int n = tile_n + wn * (TILE / 2) + j * 16 + (lane & 15);
     if (n >= N) continue;
-    long long noff = off2(n, d.N0, d.cn0, d.cn1);
+    long long noff = off2(n, d.N0, d.fn, d.cn0, d.cn1);
 #pragma unroll
     for (int i = 0; i < FB; ++i) {
 #pragma unroll
@@ -754,7 +862,7 @@ __global__ __launch_bounds__(NT, 4) void tc_kernel_vec_bf16(TcDesc d, const floa
           Wz[m + (size_t)M * n] = acc[i][j][r];
           continue;
         }
-        long long o = noff + off2(m, d.M0, d.cm0, d.cm1);
+        long long o = noff + off2(m, d.M0, d.fm, d.cm0, d.cm1);
         float v = alpha * acc[i][j][r];
         if (d.beta != 0.0) v += beta * C[o];
         C[o] = v;
@@ -863,6 +971,9 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
   // slices of at least 128 K elements (a multiple of both kernels' K-tile)
   const long long tiles = (long long)grid.x * grid.y;
   TcDesc dd = d;
+  dd.fm = FDiv((unsigned)d.M0);
+  dd.fn = FDiv((unsigned)d.N0);
+  dd.fk = FDiv((unsigned)d.K0);
   int nsplit = 1;
   if (d.batch == 1 && tiles < (small ? 512 : 128) && K >= 256) {
     long long want = std::min<long long>((512 + tiles - 1) / tiles, (K + 127) / 128);
@@ -947,6 +1058,44 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
                          (float*)C);
     TNAD_HIP_TRY(hipGetLastError());
   }
+}
+
+// The complex kernel up to ZTC_TILES 32 x 32 tiles and K up to ZTC_K; four real launches above, where the 64 x 64 tiles, the
+// 16-byte loads and the split along K of tc_launch pay.
+constexpr long long ZTC_TILES = 1024, ZTC_K = 512;
+void ztc_launch(Ctx* c, const TcDesc& d, const double* A, size_t planeA, bool conjA, const double* B, size_t planeB,
+                bool conjB, double* C, size_t planeC, hipStream_t s) {
+  const double sa = conjA ? -1.0 : 1.0, sb = conjB ? -1.0 : 1.0;
+  const long long M = (long long)d.M0 * d.M1, N = (long long)d.N0 * d.N1, K = (long long)d.K0 * d.K1;
+  const long long tiles = ((M + ZT - 1) / ZT) * ((N + ZT - 1) / ZT);
+  if (d.batch != 1 || tiles > ZTC_TILES || K > ZTC_K || M <= 0 || N <= 0 || K <= 0) {
+    // (Ar + i sa Ai)(Br + i sb Bi) = (Ar Br - sa sb Ai Bi) + i (sb Ar Bi + sa Ai Br)
+    const double *Ai = A + planeA, *Bi = B + planeB;
+    double* Ci = C + planeC;
+    TcDesc x = d;
+    tc_launch(c, Prec::F64, x, A, B, C, s);
+    x.alpha = d.alpha * sb;
+    tc_launch(c, Prec::F64, x, A, Bi, Ci, s);
+    x.beta = 1.0;
+    x.alpha = -d.alpha * sa * sb;
+    tc_launch(c, Prec::F64, x, Ai, Bi, C, s);
+    x.alpha = d.alpha * sa;
+    tc_launch(c, Prec::F64, x, Ai, B, Ci, s);
+    return;
+  }
+  const size_t ea = extent_bytes(d.M0, d.am0, d.M1, d.am1, d.K0, d.ak0, d.K1, d.ak1, 1, 0, 8),
+               eb = extent_bytes(d.K0, d.bk0, d.K1, d.bk1, d.N0, d.bn0, d.N1, d.bn1, 1, 0, 8),
+               ec = extent_bytes(d.M0, d.cm0, d.M1, d.cm1, d.N0, d.cn0, d.N1, d.cn1, 1, 0, 8);
+  c->check_range(A, planeA * 8 + ea, "ztc A");
+  c->check_range(B, planeB * 8 + eb, "ztc B");
+  c->check_range(C, planeC * 8 + ec, "ztc C");
+  TcDesc x = d;
+  x.fm = FDiv((unsigned)d.M0);
+  x.fn = FDiv((unsigned)d.N0);
+  x.fk = FDiv((unsigned)d.K0);
+  hipLaunchKernelGGL(ztc_kernel, dim3((unsigned)((M + ZT - 1) / ZT), (unsigned)((N + ZT - 1) / ZT)), dim3(NT), 0, s, x, A,
+                     (long long)planeA, sa, B, (long long)planeB, sb, C, (long long)planeC);
+  TNAD_HIP_TRY(hipGetLastError());
 }
 
 }  // namespace tnad

@@ -52,6 +52,18 @@ struct DevBuf {
 // Each of m, n, k is a pair of sub-indices (x0 fastest) with arbitrary element
 // strides, so every einsum of the hot path is one launch with no permute pass.
 // ---------------------------------------------------------------------------
+// x / d and x % d for 0 <= x < 2^30 by a multiplication (the kernels' index splits; an integer division by a
+// variable takes about 25 instructions): q = (mulhi(x, mul) + x) >> sh with sh = ceil(log2 d),
+// mul = floor(2^32 (2^sh - d) / d) + 1
+struct FDiv {
+  unsigned mul = 1, sh = 0;   // d = 1
+  FDiv() = default;
+  explicit FDiv(unsigned d) {
+    while ((1ull << sh) < d) ++sh;
+    mul = (unsigned)(((((unsigned long long)1 << sh) - d) << 32) / d + 1);
+  }
+};
+
 struct TcDesc {
   int M0 = 1, M1 = 1, N0 = 1, N1 = 1, K0 = 1, K1 = 1;
   long long am0 = 0, am1 = 0, ak0 = 0, ak1 = 0;
@@ -61,6 +73,7 @@ struct TcDesc {
   long long abat = 0, bbat = 0, cbat = 0;
   double alpha = 1.0, beta = 0.0;
   int kchunk = 0;   // set by tc_launch: K elements per split-K slice (0: no split)
+  FDiv fm, fn, fk;  // set by tc_launch: division by M0, N0, K0
 };
 
 // Plain column-major GEMM helper: C(MxN) = alpha op(A) op(B) + beta C
@@ -74,6 +87,10 @@ struct Ctx;
 // Every operand's full strided extent is checked against the context's live device
 // blocks before the launch (a size or precision mismatch throws instead of faulting).
 void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, void* C, hipStream_t s);
+// The same on complex FP64 operands in planar form (imaginary plane planeA / planeB / planeC elements after the real
+// one), either operand conjugated: one launch of a complex kernel for small outputs, four real launches above.
+void ztc_launch(Ctx* c, const TcDesc& d, const double* A, size_t planeA, bool conjA, const double* B, size_t planeB,
+                bool conjB, double* C, size_t planeC, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Small dense kernels (eig.hip)

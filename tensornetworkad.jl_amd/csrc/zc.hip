@@ -625,14 +625,7 @@ static size_t count_of(const std::vector<long long>& d) {
 
 void zein_v(Ctx* c, const TView& vA, const double* A, size_t planeA, bool conjA, const TView& vB, const double* B,
             size_t planeB, bool conjB, const TView& vC, double* Cout, size_t planeC, double alpha, double beta) {
-  const double sa = conjA ? -1.0 : 1.0, sb = conjB ? -1.0 : 1.0;
-  const double *Ar = A, *Ai = A + planeA, *Br = B, *Bi = B + planeB;
-  double *Cr = Cout, *Ci = Cout + planeC;
-  // (Ar + i sa Ai)(Br + i sb Bi) = (Ar Br - sa sb Ai Bi) + i (sb Ar Bi + sa Ai Br)
-  tc(c, Prec::F64, vA, Ar, vB, Br, vC, Cr, alpha, beta);
-  tc(c, Prec::F64, vA, Ai, vB, Bi, vC, Cr, -alpha * sa * sb, 1.0);
-  tc(c, Prec::F64, vA, Ar, vB, Bi, vC, Ci, alpha * sb, beta);
-  tc(c, Prec::F64, vA, Ai, vB, Br, vC, Ci, alpha * sa, 1.0);
+  ztc_launch(c, contract_desc(vA, vB, vC, alpha, beta), A, planeA, conjA, B, planeB, conjB, Cout, planeC, c->stream);
 }
 
 void zein(Ctx* c, const std::string& spec, const ZDims& dm, const double* A, bool conjA, const double* B, bool conjB,
