@@ -47,9 +47,7 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 constexpr int TD_GX = 16, TD_GY = 32;       // thread grid: 32 rows x 16 columns of threads (512)
 constexpr int TD_NT = TD_GX * TD_GY;
 static_assert(TD_GX == 8 || TD_GX == 16 || TD_GX == 32, "row sums span half, one or two DPP rows");
-constexpr int TD_RB = JACOBI_MAX / TD_GX;   // column elements per thread (12)
-constexpr int TD_RA = JACOBI_MAX / TD_GY;   // row elements per thread (4)
-static_assert(TD_RB * TD_GX == JACOBI_MAX && TD_RA * TD_GY == JACOBI_MAX, "tridiagonalisation tiling");
+static_assert(JACOBI_MAX % TD_GX == 0 && JACOBI_MAX % TD_GY == 0, "tridiagonalisation tiling");
 
 struct TrdShared {
   double col[2][JACOBI_MAX];   // column j + 1 as it stands before step j's update (double-buffered by parity)
@@ -116,8 +114,8 @@ __device__ __forceinline__ void trd_reflect(const double (&c)[3], int j, int m, 
 // publish it as it stands; after the second barrier every thread updates its elements while wavefront 0
 // forms column j + 1 after the update from the published column, v, p and (p . v) alone, then the next
 // reflector from it, so two barriers per step.
-template <int BJ>
-__device__ __forceinline__ void trd_block(double (&A)[TD_RA][TD_RB], int m, TrdShared& sh, int tx, int ty,
+template <int RA, int RB, int BJ>
+__device__ __forceinline__ void trd_block(double (&A)[RA][RB], int m, TrdShared& sh, int tx, int ty,
                                           int lane, int tid, double* __restrict__ Vh, double* __restrict__ tauo,
                                           double* __restrict__ eo) {
   constexpr int A0 = (BJ * TD_GX + 1) / TD_GY;   // row blocks a < A0 end at or above row BJ TD_GX
@@ -131,33 +129,33 @@ __device__ __forceinline__ void trd_block(double (&A)[TD_RA][TD_RB], int m, TrdS
     const double tv = sh.tv[buf];
     // p = tau A v on the rows below j (finished row blocks are skipped and never stored); column by column,
     // so only the matrix, the row sums and one v entry are live
-    double ps[TD_RA] = {};
+    double ps[RA] = {};
 #pragma unroll
-    for (int b = BJ; b < TD_RB; ++b) {
+    for (int b = BJ; b < RB; ++b) {
       const double vcb = vv[tx + TD_GX * b];
 #pragma unroll
-      for (int a = A0; a < TD_RA; ++a) {
+      for (int a = A0; a < RA; ++a) {
         if (TD_GY * a + TD_GY - 1 <= j) continue;   // uniform: every row of the block is finished
         ps[a] = fma(A[a][b], vcb, ps[a]);
       }
     }
     // row sums over the TD_GX lanes of each row: pairs, quads, half rows (8 lanes), rows (16), row pairs (32)
 #pragma unroll
-    for (int a = A0; a < TD_RA; ++a) ps[a] += dpp_d<0xB1>(ps[a]);
+    for (int a = A0; a < RA; ++a) ps[a] += dpp_d<0xB1>(ps[a]);
 #pragma unroll
-    for (int a = A0; a < TD_RA; ++a) ps[a] += dpp_d<0x4E>(ps[a]);
+    for (int a = A0; a < RA; ++a) ps[a] += dpp_d<0x4E>(ps[a]);
 #pragma unroll
-    for (int a = A0; a < TD_RA; ++a) ps[a] += dpp_d<0x141>(ps[a]);
+    for (int a = A0; a < RA; ++a) ps[a] += dpp_d<0x141>(ps[a]);
     if constexpr (TD_GX >= 16) {
 #pragma unroll
-      for (int a = A0; a < TD_RA; ++a) ps[a] += dpp_d<0x140>(ps[a]);
+      for (int a = A0; a < RA; ++a) ps[a] += dpp_d<0x140>(ps[a]);
     }
     if constexpr (TD_GX == 32) {   // row_bcast15 adds row 0 into row 1, row 2 into row 3
 #pragma unroll
-      for (int a = A0; a < TD_RA; ++a) ps[a] += dpp_d<0x142, 0xA>(ps[a]);
+      for (int a = A0; a < RA; ++a) ps[a] += dpp_d<0x142, 0xA>(ps[a]);
     }
 #pragma unroll
-    for (int a = A0; a < TD_RA; ++a) {
+    for (int a = A0; a < RA; ++a) {
       if (TD_GY * a + TD_GY - 1 <= j) continue;
       const int r = ty + TD_GY * a;
       if (tx == (TD_GX == 32 ? 16 : 0)) pv[r] = (r > j && r < m) ? tv * ps[a] : 0.0;   // a lane that holds the row total
@@ -168,12 +166,12 @@ __device__ __forceinline__ void trd_block(double (&A)[TD_RA][TD_RB], int m, TrdS
       if (j + 1 < j0 + TD_GX) {
         if (tx == j + 1 - j0) {
 #pragma unroll
-          for (int a = A0; a < TD_RA; ++a) cn[ty + TD_GY * a] = A[a][BJ];
+          for (int a = A0; a < RA; ++a) cn[ty + TD_GY * a] = A[a][BJ];
         }
-      } else if constexpr (BJ + 1 < TD_RB) {   // a buffer of its own: one store merged from the two
+      } else if constexpr (BJ + 1 < RB) {   // a buffer of its own: one store merged from the two
         if (tx == 0) {                          // branches would index A dynamically (A in scratch memory)
 #pragma unroll
-          for (int a = A0; a < TD_RA; ++a) sh.colb[ty + TD_GY * a] = A[a][BJ + 1];
+          for (int a = A0; a < RA; ++a) sh.colb[ty + TD_GY * a] = A[a][BJ + 1];
         }
       }
     }
@@ -197,19 +195,19 @@ __device__ __forceinline__ void trd_block(double (&A)[TD_RA][TD_RB], int m, TrdS
     }
     // the thread's rows of v and w, then the update column by column (p is written this step only for
     // rows in unskipped blocks: columns at or left of j take w = 0)
-    double vr[TD_RA], wr[TD_RA];
+    double vr[RA], wr[RA];
 #pragma unroll
-    for (int a = A0; a < TD_RA; ++a) {
+    for (int a = A0; a < RA; ++a) {
       const int r = ty + TD_GY * a;
       vr[a] = vv[r];
       wr[a] = TD_GY * a + TD_GY - 1 <= j ? 0.0 : pv[r] - kc * vr[a];
     }
 #pragma unroll
-    for (int b = BJ; b < TD_RB; ++b) {
+    for (int b = BJ; b < RB; ++b) {
       const int c = tx + TD_GX * b;
       const double vcb = vv[c], x = pv[c] - kc * vcb, wcb = c > j ? x : 0.0;
 #pragma unroll
-      for (int a = A0; a < TD_RA; ++a) {
+      for (int a = A0; a < RA; ++a) {
         if (TD_GY * a + TD_GY - 1 <= j) continue;
         A[a][b] = fma(-wr[a], vcb, fma(-vr[a], wcb, A[a][b]));
       }
@@ -217,17 +215,20 @@ __device__ __forceinline__ void trd_block(double (&A)[TD_RA][TD_RB], int m, TrdS
   }
 }
 
-// the column blocks BJ, BJ + 1, ..., TD_RB - 1 in turn
-template <int BJ>
-__device__ __forceinline__ void trd_blocks(double (&A)[TD_RA][TD_RB], int m, TrdShared& sh, int tx, int ty,
+// the column blocks BJ, BJ + 1, ..., RB - 1 in turn
+template <int RA, int RB, int BJ>
+__device__ __forceinline__ void trd_blocks(double (&A)[RA][RB], int m, TrdShared& sh, int tx, int ty,
                                            int lane, int tid, double* __restrict__ Vh, double* __restrict__ tauo,
                                            double* __restrict__ eo) {
-  trd_block<BJ>(A, m, sh, tx, ty, lane, tid, Vh, tauo, eo);
-  if constexpr (BJ + 1 < TD_RB) trd_blocks<BJ + 1>(A, m, sh, tx, ty, lane, tid, Vh, tauo, eo);
+  trd_block<RA, RB, BJ>(A, m, sh, tx, ty, lane, tid, Vh, tauo, eo);
+  if constexpr (BJ + 1 < RB) trd_blocks<RA, RB, BJ + 1>(A, m, sh, tx, ty, lane, tid, Vh, tauo, eo);
 }
 
 // H (m x m, ld ldh; the upper triangle is read) -> diagonal dout (m), off-diagonal eout (m - 1),
-// reflectors Vh (m x m, column j = v_j) and tauo (m - 2).
+// reflectors Vh (m x m, column j = v_j) and tauo (m - 2).  RA x RB: elements per thread, the smallest of the
+// instances in trd_launch that covers m: the padding of a larger one is multiplied and updated like the rest (the
+// values are the same for each).
+template <int RA, int RB>
 __global__ __launch_bounds__(TD_NT) void trd_kernel(const double* __restrict__ H, int ldh, int m,
                                                     double* __restrict__ dout, double* __restrict__ eout,
                                                     double* __restrict__ Vh, double* __restrict__ tauo,
@@ -235,11 +236,11 @@ __global__ __launch_bounds__(TD_NT) void trd_kernel(const double* __restrict__ H
   if (gate && *gate == 0) return;
   __shared__ TrdShared sh;
   const int tid = threadIdx.x, ty = tid / TD_GX, tx = tid % TD_GX, lane = tid & 63;
-  double A[TD_RA][TD_RB];
+  double A[RA][RB];
 #pragma unroll
-  for (int a = 0; a < TD_RA; ++a)
+  for (int a = 0; a < RA; ++a)
 #pragma unroll
-    for (int b = 0; b < TD_RB; ++b) {
+    for (int b = 0; b < RB; ++b) {
       const int r = ty + TD_GY * a, c = tx + TD_GX * b;
       const bool in = r < m && c < m;
       const double x = H[in ? min(r, c) + (size_t)max(r, c) * ldh : 0];   // branch-free, clamped address
@@ -248,7 +249,7 @@ __global__ __launch_bounds__(TD_NT) void trd_kernel(const double* __restrict__ H
   if (m > 2) {   // the first reflector, from column 0 (published, then formed by wavefront 0)
     if (tx == 0) {
 #pragma unroll
-      for (int a = 0; a < TD_RA; ++a) sh.col[1][ty + TD_GY * a] = A[a][0];
+      for (int a = 0; a < RA; ++a) sh.col[1][ty + TD_GY * a] = A[a][0];
     }
     __syncthreads();
     if (tid < 64) {
@@ -258,11 +259,11 @@ __global__ __launch_bounds__(TD_NT) void trd_kernel(const double* __restrict__ H
       trd_reflect(c, 0, m, lane, sh, Vh, tauo, eout);
     }
   }
-  trd_blocks<0>(A, m, sh, tx, ty, lane, tid, Vh, tauo, eout);
+  trd_blocks<RA, RB, 0>(A, m, sh, tx, ty, lane, tid, Vh, tauo, eout);
 #pragma unroll
-  for (int a = 0; a < TD_RA; ++a)
+  for (int a = 0; a < RA; ++a)
 #pragma unroll
-    for (int b = 0; b < TD_RB; ++b) {
+    for (int b = 0; b < RB; ++b) {
       const int r = ty + TD_GY * a, c = tx + TD_GX * b;
       if (r == c && r < m) dout[r] = A[a][b];
       if (r == m - 1 && c == m - 2) eout[m - 2] = A[a][b];
@@ -1160,6 +1161,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
     if (lane + 64 * k < m) zc[lane + 64 * k] = z[k];
 }
 
+// Instances for m up to 48, 96, 144, 192 (us at m = 20 / 48 / 80 / 128 with the last one for all: 48 / 102 / 159 / 229;
+// with these: 25 / 54 / 105 / 191)
+void trd_launch(const double* H, int ldh, int m, double* d, double* e, double* Vh, double* tau, const int* gate,
+                hipStream_t s) {
+  if (m <= 48) hipLaunchKernelGGL((trd_kernel<2, 3>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, gate);
+  else if (m <= 96) hipLaunchKernelGGL((trd_kernel<3, 6>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, gate);
+  else if (m <= 144) hipLaunchKernelGGL((trd_kernel<5, 9>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, gate);
+  else hipLaunchKernelGGL((trd_kernel<6, 12>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, gate);
+  TNAD_HIP_TRY(hipGetLastError());
+}
+
 // the work buffer: Vh, Qa, Qb, U (m x m each), d, e, tau, lambda (m each), the reflector block products
 struct DcWork {
   double *Vh, *Qa, *Qb, *U, *dv, *ev, *tau, *lam, *gram;
@@ -1231,8 +1243,7 @@ void syev_dc(const double* H, int ldh, int m, double* evals, double* V, double* 
              const int* gate) {
   if (m < 1 || m > JACOBI_MAX) throw Error(TNAD_ERR_ARG, "syev_dc: size out of range");
   const DcWork w = dc_work(work, m);
-  hipLaunchKernelGGL(trd_kernel, dim3(1), dim3(TD_NT), 0, s, H, ldh, m, w.dv, w.ev, w.Vh, w.tau, gate);
-  TNAD_HIP_TRY(hipGetLastError());
+  trd_launch(H, ldh, m, w.dv, w.ev, w.Vh, w.tau, gate, s);
   dc_solve(w, m, gate, s);
   dc_vectors(w, m, gate, s);
   sort_eigenpairs(w.lam, w.Qa, m, evals, V, gate, s);
@@ -1248,7 +1259,7 @@ void syev_dc_time(const double* H, int m, int reps, double* work, hipStream_t s,
   float acc[3] = {0.f, 0.f, 0.f};
   for (int r = 0; r <= reps; ++r) {   // the first run warms up
     TNAD_HIP_TRY(hipEventRecord(e[0], s));
-    hipLaunchKernelGGL(trd_kernel, dim3(1), dim3(TD_NT), 0, s, H, m, m, w.dv, w.ev, w.Vh, w.tau, (const int*)nullptr);
+    trd_launch(H, m, m, w.dv, w.ev, w.Vh, w.tau, nullptr, s);
     TNAD_HIP_TRY(hipEventRecord(e[1], s));
     dc_solve(w, m, nullptr, s);
     TNAD_HIP_TRY(hipEventRecord(e[2], s));
