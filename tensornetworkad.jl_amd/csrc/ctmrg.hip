@@ -710,9 +710,9 @@ void eig_adjoint(Ctx* c, const StepDims& d, const StepTape& tp, const double* G,
         tmp(c, (size_t)n * chi * 8);
     k_square(lam, sq.as<double>(), k, s);
     const double* M = tp.M.as<double>();
-    auto applyA2 = [&](const double* V, double* out) {
-      tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, chi, n, n, n, n), M, V, tmp.as<double>(), s);
-      tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, chi, n, n, n, n), M, tmp.as<double>(), out, s);
+    auto applyA2 = [&](const double* V, double* out, int nc) {
+      tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, nc, n, n, n, n), M, V, tmp.as<double>(), s);
+      tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, nc, n, n, n, n), M, tmp.as<double>(), out, s);
     };
     // A step computed with low-precision contractions resolved its eigenpairs only to the relative
     // residual its contractions can support (1e-8 and above), so this adjoint is no more accurate

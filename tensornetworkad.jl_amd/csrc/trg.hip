@@ -446,9 +446,9 @@ static void svd_split_back(Ctx* c, const SvdTape& tp, const double* ubar, const 
                        tp.sv.as<double>());
     TNAD_HIP_TRY(hipGetLastError());
     tc_launch(c, Prec::F64, gemm_desc('N', 'N', m, kk, mp, m, mp, m, 1.0, 1.0), M, dV.as<double>(), bl.as<double>(), s);
-    auto applyMMt = [&](const double* Vb, double* out) {
-      tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp, kk, m, m, m, mp), M, Vb, T1.as<double>(), s);
-      tc_launch(c, Prec::F64, gemm_desc('N', 'N', m, kk, mp, m, mp, m), M, T1.as<double>(), out, s);
+    auto applyMMt = [&](const double* Vb, double* out, int nc) {
+      tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp, nc, m, m, m, mp), M, Vb, T1.as<double>(), s);
+      tc_launch(c, Prec::F64, gemm_desc('N', 'N', m, nc, mp, m, mp, m), M, T1.as<double>(), out, s);
     };
     resolvent_pcg(c, m, kk, K, U, sig, tz, applyMMt, bl.as<double>(), X.as<double>(), 1e-13, 200);
     // Mbar += X V_kk^T
@@ -462,9 +462,9 @@ static void svd_split_back(Ctx* c, const SvdTape& tp, const double* ubar, const 
                        tp.sv.as<double>());
     TNAD_HIP_TRY(hipGetLastError());
     tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp, kk, m, m, m, mp, 1.0, 1.0), M, dU.as<double>(), br.as<double>(), s);
-    auto applyMtM = [&](const double* Vb, double* out) {
-      tc_launch(c, Prec::F64, gemm_desc('N', 'N', m, kk, mp, m, mp, m), M, Vb, T1.as<double>(), s);
-      tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp, kk, m, m, m, mp), M, T1.as<double>(), out, s);
+    auto applyMtM = [&](const double* Vb, double* out, int nc) {
+      tc_launch(c, Prec::F64, gemm_desc('N', 'N', m, nc, mp, m, mp, m), M, Vb, T1.as<double>(), s);
+      tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp, nc, m, m, m, mp), M, T1.as<double>(), out, s);
     };
     resolvent_pcg(c, mp, kk, K, V, sig, tz, applyMtM, br.as<double>(), Y.as<double>(), 1e-13, 200);
     // Mbar += U_kk Y^T

@@ -573,13 +573,13 @@ static void zsvd_split_back(Ctx* c, const ZSvdTape& tp, const double* ubar, cons
                        b2.as<double>(), 0);
     TNAD_HIP_TRY(hipGetLastError());
     const int m2 = 2 * m, mp2 = 2 * mp;
-    auto apply = [&](const double* Vb, double* out) {
+    auto apply = [&](const double* Vb, double* out, int nc) {
       if (left) {   // R R^T
-        tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp2, r2, m2, m2, m2, mp2), RM.as<double>(), Vb, T1.as<double>(), s);
-        tc_launch(c, Prec::F64, gemm_desc('N', 'N', m2, r2, mp2, m2, mp2, m2), RM.as<double>(), T1.as<double>(), out, s);
+        tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp2, nc, m2, m2, m2, mp2), RM.as<double>(), Vb, T1.as<double>(), s);
+        tc_launch(c, Prec::F64, gemm_desc('N', 'N', m2, nc, mp2, m2, mp2, m2), RM.as<double>(), T1.as<double>(), out, s);
       } else {      // R^T R
-        tc_launch(c, Prec::F64, gemm_desc('N', 'N', m2, r2, mp2, m2, mp2, m2), RM.as<double>(), Vb, T1.as<double>(), s);
-        tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp2, r2, m2, m2, m2, mp2), RM.as<double>(), T1.as<double>(), out, s);
+        tc_launch(c, Prec::F64, gemm_desc('N', 'N', m2, nc, mp2, m2, mp2, m2), RM.as<double>(), Vb, T1.as<double>(), s);
+        tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp2, nc, m2, m2, m2, mp2), RM.as<double>(), T1.as<double>(), out, s);
       }
     };
     resolvent_pcg(c, R2, r2, k2, W2.as<double>(), sig2.as<double>(), tz2.as<double>(), apply, b2.as<double>(),
