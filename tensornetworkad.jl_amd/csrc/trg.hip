@@ -109,28 +109,12 @@ __global__ void augment_kernel(const double* __restrict__ M, int m, int mp, doub
   }
 }
 
-// U[:, j] = sqrt(2) X[0:m, col_j], V[:, j] = sqrt(2) X[m:, col_j]  (col_j < 0: zero column)
-__global__ void split_vectors_kernel(const double* __restrict__ X, int N, int m, const int* __restrict__ cols,
-                                     int kk, double* __restrict__ U, double* __restrict__ V) {
-  const int mp = N - m;
-  size_t tot = (size_t)N * kk;
-  const double r2 = 1.4142135623730951;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < tot; e += (size_t)gridDim.x * blockDim.x) {
-    int r = e % N, j = e / N;
-    int cidx = cols[j];
-    double v = cidx >= 0 ? r2 * X[r + (size_t)N * cidx] : 0.0;
-    if (r < m) U[r + (size_t)m * j] = v;
-    else V[(r - m) + (size_t)mp * j] = v;
-  }
-}
-
-// The same for pairs from the subspace iteration, which are converged to 1e-13 |theta_0|: relative to a small s
-// that leaves a part 1e-13 s_0 / (2 s) of the (-s, [u; -v]) partner in the vector, which lengthens u and
-// shortens v by as much.  Normalising the halves separately takes it out to first order, and theta over the
-// product of the halves' norms is the singular value (they are 1/sqrt 2 each without it).  One workgroup per
-// column; also writes s_j and sqrt(s_j).  A column whose halves are far from equal (an unconverged guard
-// pair) is only scaled.
-__global__ __launch_bounds__(NT) void split_vectors_unit_kernel(const double* __restrict__ X,
+// Singular triplets from the eigenpairs (theta, [u; v] / sqrt 2) of the augmented matrix: one workgroup per column
+// cols[j].  A pair carries a part eps s_0 / (2 s) of its (-s, [u; -v]) partner, eps being 1e-16 from the full spectrum and up
+// to 1e-13 from the subspace iteration, which lengthens u and shortens v by as much.  Normalising the halves separately
+// takes it out, and theta over the product of the halves' norms is the singular value (they are 1/sqrt 2 each without
+// it).  Also writes s_j and sqrt(s_j).  A column whose halves are far from equal (an unconverged guard pair) is only scaled.
+__global__ __launch_bounds__(NT) void split_vectors_kernel(const double* __restrict__ X,
                                                                 const double* __restrict__ theta, int N, int m,
                                                                 const int* __restrict__ cols, double* __restrict__ U,
                                                                 double* __restrict__ V, double* __restrict__ sv,
@@ -362,8 +346,6 @@ static void svd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, i
   tp.k = k;
   tp.K = K;
   const int Kc = std::max(K, 1);
-  std::vector<double> hsq(Kc, 0.0);
-  for (int j = 0; j < K; ++j) hsq[j] = std::sqrt(tp.hs[j]);
   DevBuf cols(c, (size_t)Kc * sizeof(int) + 16);
   tp.sv = DevBuf(c, (size_t)Kc * 8);
   tp.sq = DevBuf(c, (size_t)std::max(k, Kc) * 8);
@@ -372,15 +354,25 @@ static void svd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, i
   k_fill(tp.sq.as<double>(), (size_t)std::max(k, Kc), 0.0, s);
   if (K > 0) {
     c->write_async(cols.ptr, pos.data(), (size_t)K * sizeof(int));
-    if (N > JACOBI_MAX) {
-      hipLaunchKernelGGL(split_vectors_unit_kernel, dim3(K), dim3(NT), 0, s, X.as<double>(), theta.as<double>(), N, m,
-                         cols.as<int>(), tp.U.as<double>(), tp.V.as<double>(), tp.sv.as<double>(),
-                         tp.sq.as<double>());
-    } else {   // the whole spectrum at once: pairs accurate to rounding
-      c->write_async(tp.sv.ptr, tp.hs.data(), (size_t)K * 8);
-      c->write_async(tp.sq.ptr, hsq.data(), (size_t)K * 8);
-      hipLaunchKernelGGL(split_vectors_kernel, dim3(nb((size_t)N * K)), dim3(NT), 0, s, X.as<double>(), N, m,
-                         cols.as<int>(), K, tp.U.as<double>(), tp.V.as<double>());
+    hipLaunchKernelGGL(split_vectors_kernel, dim3(K), dim3(NT), 0, s, X.as<double>(), theta.as<double>(), N, m,
+                       cols.as<int>(), tp.U.as<double>(), tp.V.as<double>(), tp.sv.as<double>(), tp.sq.as<double>());
+    TNAD_HIP_TRY(hipGetLastError());
+    // Small kept values also mix with each other's partners, by eps s_0 / (s_i + s_j): u and v as wholes then lose their
+    // orthogonality, which the adjoint relies on.  Two Newton-Schulz steps X <- X (3 I - X^T X) / 2 bring the kept
+    // columns back to it.
+    const int kv = std::min(k, K);
+    if (kv > 0 && tp.hs[kv - 1] < 1e-6 * tp.hs[0]) {
+      DevBuf G(c, (size_t)kv * kv * 8), T(c, (size_t)std::max(m, mp) * kv * 8);
+      for (int half = 0; half < 2; ++half) {
+        double* Q = half ? tp.V.as<double>() : tp.U.as<double>();
+        const int rows = half ? mp : m;
+        for (int it = 0; it < 2; ++it) {
+          tc_launch(c, Prec::F64, gemm_desc('T', 'N', kv, kv, rows, rows, rows, kv), Q, Q, G.as<double>(), s);
+          k_copy(Q, T.as<double>(), (size_t)rows * kv, s);
+          tc_launch(c, Prec::F64, gemm_desc('N', 'N', rows, kv, kv, rows, kv, rows, -0.5, 1.5), T.as<double>(),
+                    G.as<double>(), Q, s);
+        }
+      }
     }
   }
   // u = U[:, 1:k] sqrt(s), v = sqrt(s) V[:, 1:k]^T; columns j >= K are zero
