@@ -454,6 +454,214 @@ __global__ __launch_bounds__(NT, TILE == 128 ? 1 : (sizeof(T) == 8 ? 3 : 4)) voi
 }
 
 // ---------------------------------------------------------------------------
+// FP64 kernel for outputs of few tiles: no K loop barrier and no second launch for the split of K.  Every wave of a
+// workgroup computes the whole 16 MB x 16 NB output tile over its own share of K (16-element steps w, w + W, ...),
+// and the W partial tiles are added in wave order in LDS at the end.
+// An FP64 MFMA takes 64 cycles, so operands need no sharing between waves; what bounds such a kernel is the address
+// unit, which serves a load 16 lanes at a time, one cache line per cycle.  MFMA lane l holds row l % 16 of its operand, so
+// how an operand is read depends on which index is contiguous:
+//   0: m (n), or neither: 8 bytes per lane, 16 consecutive rows per 16 lanes (70 bytes per ns and CU from L2)
+//   1: m (n) with even extent: 16 bytes per lane, rows 2 c and 2 c + 1 going to two blocks (136 bytes per ns)
+//   2: k: 8 lanes read the 16 k of a row and the wave transposes through its own LDS rows (136; read straight into the
+//      operand layout, 16 lanes touch 16 lines: 37)
+// ---------------------------------------------------------------------------
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));   // 16-byte loads at 8-byte alignment
+constexpr int SLAB_KP = 18;   // LDS row pitch (doubles) of the transposition: eight rows' 16-byte accesses meet no bank twice
+
+// One operand: NBLK blocks of 16 rows (its m or n index), read by mode MODE.
+template <int NBLK, int MODE> struct SlabOperand {
+  static_assert(MODE != 1 || NBLK % 2 == 0, "row pairs");
+  static constexpr int LDS = MODE == 2 ? NBLK * 16 * SLAB_KP : 0;   // doubles per wave
+  const char* base;
+  unsigned row[MODE == 2 ? 2 * NBLK : NBLK];   // byte offsets of the rows this lane loads
+  unsigned trow[NBLK];                         // and of its operand rows (K remainder)
+  unsigned s0, s1;                             // byte strides of the K sub-indices
+  double v[NBLK][4];                           // raw loads of one K step (mode 2: two rows' pairs; modes 0, 1: the operand)
+
+  // row (within the tile) of operand position c of block i
+  static __device__ __forceinline__ int tile_row(int i, int c) { return MODE == 1 ? 32 * (i >> 1) + 2 * c + (i & 1) : 16 * i + c; }
+  __device__ __forceinline__ void init(const double* p, int tile, int X, int X0, const FDiv& fx, long long x0, long long x1,
+                                       long long k0, long long k1, int lane) {
+    base = reinterpret_cast<const char*>(p);
+    s0 = 8u * (unsigned)k0;
+    s1 = 8u * (unsigned)k1;
+    auto off = [&](int r) { return 8u * (unsigned)off2(min(tile + r, X - 1), X0, fx, x0, x1); };
+#pragma unroll
+    for (int i = 0; i < NBLK; ++i) trow[i] = off(tile_row(i, lane & 15));
+    if (MODE == 2) {
+#pragma unroll
+      for (int i = 0; i < 2 * NBLK; ++i) row[i] = off(8 * i + (lane >> 3));
+    } else if (MODE == 1) {
+#pragma unroll
+      for (int i = 0; i < NBLK; i += 2) row[i] = 8u * (unsigned)off2(min(tile + 16 * i + 2 * (lane & 15), X - 2), X0, fx, x0, x1);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NBLK; ++i) row[i] = trow[i];
+    }
+  }
+  __device__ __forceinline__ unsigned koff(int k, const TcDesc& d) const {
+    if (d.K1 == 1) return (unsigned)k * s0;
+    const int q = fdiv(k, d.fk);
+    return (unsigned)(k - q * d.K0) * s0 + (unsigned)q * s1;
+  }
+  // K step kb .. kb + 15, all inside K: MFMA e of lane group g takes k = kb + 4 g + e
+  __device__ __forceinline__ void load(int kb, int lane, const TcDesc& d) {
+    if (MODE == 2) {
+      const unsigned o = koff(kb + 2 * (lane & 7), d);
+#pragma unroll
+      for (int i = 0; i < 2 * NBLK; ++i) {
+        const d2u x = *reinterpret_cast<const d2u*>(base + (row[i] + o));
+        v[i >> 1][2 * (i & 1)] = x[0];
+        v[i >> 1][2 * (i & 1) + 1] = x[1];
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned o = koff(kb + 4 * (lane >> 4) + e, d);
+        if (MODE == 1) {
+#pragma unroll
+          for (int i = 0; i < NBLK; i += 2) {
+            const d2u x = *reinterpret_cast<const d2u*>(base + (row[i] + o));
+            v[i][e] = x[0];
+            v[i + 1][e] = x[1];
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < NBLK; ++i) v[i][e] = *reinterpret_cast<const double*>(base + (row[i] + o));
+        }
+      }
+    }
+  }
+  // the last, partial K step, straight into operand layout: elements past K read the last one and count as zero
+  __device__ __forceinline__ void load_tail(int kb, int lane, const TcDesc& d, int K) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int k = kb + 4 * (lane >> 4) + e;
+      const unsigned o = koff(min(k, K - 1), d);
+#pragma unroll
+      for (int i = 0; i < NBLK; ++i) {
+        const double x = *reinterpret_cast<const double*>(base + (trow[i] + o));
+        v[i][e] = k < K ? x : 0.0;
+      }
+    }
+  }
+  // the operand registers x from a whole step's loads; lds: this wave's own LDS rows
+  __device__ __forceinline__ void operand(double (&x)[NBLK][4], double* lds, int lane) const {
+    if (MODE == 2) {
+#pragma unroll
+      for (int i = 0; i < 2 * NBLK; ++i)
+        *reinterpret_cast<d2*>(&lds[(8 * i + (lane >> 3)) * SLAB_KP + 2 * (lane & 7)]) =
+            d2{v[i >> 1][2 * (i & 1)], v[i >> 1][2 * (i & 1) + 1]};
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int i = 0; i < NBLK; ++i) {
+        const d2* q = reinterpret_cast<const d2*>(&lds[(16 * i + (lane & 15)) * SLAB_KP + 4 * (lane >> 4)]);
+        const d2 y0 = q[0], y1 = q[1];
+        x[i][0] = y0[0]; x[i][1] = y0[1]; x[i][2] = y1[0]; x[i][3] = y1[1];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    } else {
+#pragma unroll
+      for (int i = 0; i < NBLK; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[i][e] = v[i][e];
+    }
+  }
+};
+
+constexpr int SLAB_W = 8;   // waves: two per SIMD, one's loads and LDS traffic under the other's MFMAs (4: 10-30% slower, 16: no faster)
+template <int MB, int NB, int AM, int BMD>
+__global__ __launch_bounds__(64 * SLAB_W) void tc_slab_kernel(TcDesc d, const double* __restrict__ A,
+                                                              const double* __restrict__ B, double* __restrict__ C) {
+  constexpr int W = SLAB_W;
+  typedef SlabOperand<MB, AM> OpA;
+  typedef SlabOperand<NB, BMD> OpB;
+  constexpr int RP = 4 * 68;   // doubles per 16 x 16 block of a partial tile: entry (row q + 4 r, column n) at 68 r + 17 q + n
+  constexpr int WL = OpA::LDS + OpB::LDS;
+  __shared__ __attribute__((aligned(16))) double sh[W * (WL > MB * NB * RP ? WL : MB * NB * RP)];
+  const int M = d.M0 * d.M1, N = d.N0 * d.N1, K = d.K0 * d.K1;
+  // workgroups go round robin to the 8 XCDs: each XCD takes a contiguous range of the tiles (n fastest), so that its L2
+  // holds its own rows of A and all of B (1440 x 1440 . 1440 x 135: 24.7 -> 18.5 us)
+  const unsigned tiles = gridDim.x * gridDim.y, id = blockIdx.x + gridDim.x * blockIdx.y, xcd = id % 8;
+  const unsigned tile = xcd * (tiles / 8) + min(xcd, tiles % 8) + id / 8;
+  const int tile_m = (int)(tile / gridDim.y) * 16 * MB, tile_n = (int)(tile % gridDim.y) * 16 * NB;
+  C += (long long)blockIdx.z * d.cbat;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  OpA a;
+  OpB b;
+  a.init(A + (long long)blockIdx.z * d.abat, tile_m, M, d.M0, d.fm, d.am0, d.am1, d.ak0, d.ak1, lane);
+  b.init(B + (long long)blockIdx.z * d.bbat, tile_n, N, d.N0, d.fn, d.bn0, d.bn1, d.bk0, d.bk1, lane);
+  double* wl = sh + wave * WL;
+
+  d4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = d4{0, 0, 0, 0};
+  double xa[MB][4], xb[NB][4];
+  auto mul = [&] {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = MfmaOp<double>::run(xa[i][e], xb[j][e], acc[i][j]);
+  };
+  // whole steps, the loads of the next one in flight while this one is multiplied
+  const int Kw = K & ~15;
+  int kb = 16 * wave;
+  if (kb < Kw) {
+    a.load(kb, lane, d);
+    b.load(kb, lane, d);
+  }
+  for (; kb < Kw; kb += 16 * W) {
+    a.operand(xa, wl, lane);
+    b.operand(xb, wl + OpA::LDS, lane);
+    if (kb + 16 * W < Kw) {
+      a.load(kb + 16 * W, lane, d);
+      b.load(kb + 16 * W, lane, d);
+    }
+    mul();
+  }
+  if (kb == Kw && Kw < K) {   // the wave whose turn it is takes the remainder
+    a.load_tail(kb, lane, d, K);
+    b.load_tail(kb, lane, d, K);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i) xa[i][e] = a.v[i][e];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) xb[j][e] = b.v[j][e];
+    }
+    mul();
+  }
+  if (WL > 0) __syncthreads();   // the partial tiles take the place of the transposition rows
+  double* red = sh + wave * MB * NB * RP;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[(i * NB + j) * RP + 68 * r + 17 * (lane >> 4) + (lane & 15)] = acc[i][j][r];
+  __syncthreads();
+  for (int e = threadIdx.x; e < 256 * MB * NB; e += 64 * W) {
+    const int ml = e % (16 * MB), nl = e / (16 * MB);
+    const int m = tile_m + ml, n = tile_n + nl;
+    if (m >= M || n >= N) continue;
+    const int i = AM == 1 ? 2 * (ml >> 5) + (ml & 1) : ml >> 4, mc = AM == 1 ? (ml & 31) >> 1 : ml & 15;
+    const int j = BMD == 1 ? 2 * (nl >> 5) + (nl & 1) : nl >> 4, ncol = BMD == 1 ? (nl & 31) >> 1 : nl & 15;
+    const double* p = sh + (i * NB + j) * RP + 68 * (mc >> 2) + 17 * (mc & 3) + ncol;
+    double v = p[0];
+#pragma unroll
+    for (int w = 1; w < W; ++w) v += p[w * MB * NB * RP];
+    v *= d.alpha;
+    const long long o = off2(m, d.M0, d.fm, d.cm0, d.cm1) + off2(n, d.N0, d.fn, d.cn0, d.cn1);
+    if (d.beta != 0.0) v += d.beta * C[o];
+    C[o] = v;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Complex FP64 kernel for small outputs: both planes of both operands staged together, 32 x 32 output tile per
 // workgroup, each of the 4 waves one 16 x 16 block with three accumulators (Ar Br, Ai Bi, Ar Bi + Ai Br), K-tile 16,
 // double-buffered LDS (49 KB).  A complex contraction of the sizes the complex path runs (corner matrix up to
@@ -941,12 +1149,84 @@ static bool launch_vec(const TcDesc& dd, dim3 grid, const void* A, const void* B
   return true;
 }
 
+// How tc_slab_kernel reads an operand (X0, x0: extent and stride of its first m or n sub-index; even: the tile has an
+// even number of its blocks).
+static int slab_mode(const TcDesc& d, int X0, long long x0, long long k0, bool even) {
+  if (tc_vec_disabled()) return 0;
+  if (k0 == 1 && d.K0 > 1 && (d.K1 == 1 || d.K0 % 2 == 0)) return 2;   // 16-byte loads stay inside one K0 run
+  return even && x0 == 1 && X0 % 2 == 0 ? 1 : 0;
+}
+
+template <int MB, int NB, int AM>
+static void launch_slab_b(int bm, dim3 grid, const TcDesc& d, const double* A, const double* B, double* C, hipStream_t s) {
+  const dim3 block(64 * SLAB_W);
+  if (bm == 2) hipLaunchKernelGGL((tc_slab_kernel<MB, NB, AM, 2>), grid, block, 0, s, d, A, B, C);
+  else if (bm == 1) hipLaunchKernelGGL((tc_slab_kernel<MB, NB, AM, NB % 2 == 0 ? 1 : 0>), grid, block, 0, s, d, A, B, C);
+  else hipLaunchKernelGGL((tc_slab_kernel<MB, NB, AM, 0>), grid, block, 0, s, d, A, B, C);
+}
+template <int MB, int NB>
+static void launch_slab(const TcDesc& d, const double* A, const double* B, double* C, hipStream_t s) {
+  const long long M = (long long)d.M0 * d.M1, N = (long long)d.N0 * d.N1;
+  const dim3 grid((unsigned)((M + 16 * MB - 1) / (16 * MB)), (unsigned)((N + 16 * NB - 1) / (16 * NB)), (unsigned)d.batch);
+  const int am = slab_mode(d, d.M0, d.am0, d.ak0, MB % 2 == 0), bm = slab_mode(d, d.N0, d.bn0, d.bk0, NB % 2 == 0);
+  if (am == 2) launch_slab_b<MB, NB, 2>(bm, grid, d, A, B, C, s);
+  else if (am == 1) launch_slab_b<MB, NB, MB % 2 == 0 ? 1 : 0>(bm, grid, d, A, B, C, s);
+  else launch_slab_b<MB, NB, 0>(bm, grid, d, A, B, C, s);
+}
+
+// The FP64 products tc_slab_kernel takes: up to 512 32 x 32 output tiles (two per CU) at any K up to 8192, and up to 2048 of
+// them once K reaches 256.  Larger outputs amortise the 64 x 64 and 128 x 128 tiles, where waves share operands (us, this
+// kernel / those: 576 x 576 x 64 5.0 / 6.5, 1024 x 1024 x 64 10.1 / 8.9, 1024 x 1024 x 256 15.8 / 18.6, 4096 x 512 x 512 47
+// / 51, 2048 x 2048 x 256 57 / 49); for a longer K a few tiles leave the chip idle, which the split along the grid fills
+// (96 x 96 x 8192 28 / 32, 16 x 16 x 16384 46 / 41).  Operands are addressed with 32-bit byte offsets.
+static bool slab_applies(const TcDesc& d, size_t bytes_a, size_t bytes_b) {
+  const long long M = (long long)d.M0 * d.M1, N = (long long)d.N0 * d.N1, K = (long long)d.K0 * d.K1;
+  const long long n = (M + 31) / 32 * ((N + 31) / 32) * d.batch;
+  return (n <= 512 || (n <= 2048 && K >= 256)) && K <= 8192 && bytes_a < (1ull << 32) &&
+         bytes_b < (1ull << 32);
+}
+
+// Its tile: the one with the least estimated time, rounds over the 256 CUs times the cost of a tile (measured with every
+// CU busy: ns per 16-element K step, 500 ns per round for the start and the sum over the waves, 200 ns per block and
+// dimension for the launch).  One tile size for all would cost up to 2x: 2048 x 17 x 2048 11 us as 1 x 1 block, 30 as 2 x 3;
+// 2048 x 192 x 2048 45 and 35.
+static void slab(const TcDesc& d, const double* A, const double* B, double* C, hipStream_t s) {
+  struct Tile {
+    int mb, nb;
+    double step_ns;
+  };
+  static constexpr Tile tiles[] = {{1, 1, 65.0}, {2, 1, 92.0}, {1, 3, 131.0}, {2, 2, 158.0}, {2, 3, 234.0}};
+  const long long M = (long long)d.M0 * d.M1, N = (long long)d.N0 * d.N1, K = (long long)d.K0 * d.K1;
+  const double steps = (double)((K + 16 * SLAB_W - 1) / (16 * SLAB_W) * SLAB_W);
+  int best = 0;
+  double tb = 0.0;
+  for (int i = 0; i < 5; ++i) {
+    const long long mt = 16 * tiles[i].mb, nt = 16 * tiles[i].nb;
+    const long long n = (M + mt - 1) / mt * ((N + nt - 1) / nt) * d.batch;
+    const double t = (double)((n + 255) / 256) * (steps * tiles[i].step_ns + 500.0) + 200.0 * (tiles[i].mb + tiles[i].nb);
+    if (i == 0 || t < tb) {
+      best = i;
+      tb = t;
+    }
+  }
+  switch (best) {
+    case 0: launch_slab<1, 1>(d, A, B, C, s); break;
+    case 1: launch_slab<2, 1>(d, A, B, C, s); break;
+    case 2: launch_slab<1, 3>(d, A, B, C, s); break;
+    case 3: launch_slab<2, 2>(d, A, B, C, s); break;
+    default: launch_slab<2, 3>(d, A, B, C, s); break;
+  }
+}
+
 void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, void* C, hipStream_t s) {
   const long long M = (long long)d.M0 * d.M1, N = (long long)d.N0 * d.N1;
+  size_t bytes_a, bytes_b;
   {
     const size_t es = p == Prec::F64 ? 8 : 4;
-    c->check_range(A, extent_bytes(d.M0, d.am0, d.M1, d.am1, d.K0, d.ak0, d.K1, d.ak1, d.batch, d.abat, es), "tc A");
-    c->check_range(B, extent_bytes(d.K0, d.bk0, d.K1, d.bk1, d.N0, d.bn0, d.N1, d.bn1, d.batch, d.bbat, es), "tc B");
+    bytes_a = extent_bytes(d.M0, d.am0, d.M1, d.am1, d.K0, d.ak0, d.K1, d.ak1, d.batch, d.abat, es);
+    bytes_b = extent_bytes(d.K0, d.bk0, d.K1, d.bk1, d.N0, d.bn0, d.N1, d.bn1, d.batch, d.bbat, es);
+    c->check_range(A, bytes_a, "tc A");
+    c->check_range(B, bytes_b, "tc B");
     c->check_range(C, extent_bytes(d.M0, d.cm0, d.M1, d.cm1, d.N0, d.cn0, d.N1, d.cn1, d.batch, d.cbat, es), "tc C");
   }
   if (M <= 0 || N <= 0 || d.batch <= 0) return;
@@ -958,22 +1238,28 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
     throw Error(TNAD_ERR_ARG, "tc_launch: extents out of range");
   dim3 grid((unsigned)((M + BM - 1) / BM), (unsigned)((N + BN - 1) / BN), (unsigned)d.batch);
   if (grid.y > 65535) throw Error(TNAD_ERR_ARG, "tc_launch: N too large");
+  TcDesc dd = d;
+  dd.fm = FDiv((unsigned)d.M0);
+  dd.fn = FDiv((unsigned)d.N0);
+  dd.fk = FDiv((unsigned)d.K0);
+  if (p == Prec::F64 && slab_applies(d, bytes_a, bytes_b)) {
+    slab(dd, (const double*)A, (const double*)B, (double*)C, s);
+    TNAD_HIP_TRY(hipGetLastError());
+    return;
+  }
   const long long K = (long long)d.K0 * d.K1;
   const long long tiles64 = (long long)grid.x * grid.y;
   // 32 x 32 tiles (4x the workgroups) when 64 x 64 tiles would leave most CUs idle: short K, or an
   // output of at most 16 tiles with K up to 4096 (the k x k Gram products of the eigensolver, cut along
   // K below as well; for longer K the 64 x 64 tile's higher MFMA rate per slice wins)
   const dim3 grid32((unsigned)((M + 31) / 32), (unsigned)((N + 31) / 32), (unsigned)d.batch);
-  const bool small = (long long)grid.x * grid.y * grid.z < TC_SMALL_BELOW && grid32.y <= 65535 &&
+  // (FP64 calls of these sizes went to tc_slab_kernel above)
+  const bool small = p != Prec::F64 && (long long)grid.x * grid.y * grid.z < TC_SMALL_BELOW && grid32.y <= 65535 &&
                      (K < 256 || (tiles64 <= 16 && K <= 4096));
   if (small) grid = grid32;
   // split-K when the output tiles cannot fill the chip and K is long: about 512 workgroups,
   // slices of at least 128 K elements (a multiple of both kernels' K-tile)
   const long long tiles = (long long)grid.x * grid.y;
-  TcDesc dd = d;
-  dd.fm = FDiv((unsigned)d.M0);
-  dd.fn = FDiv((unsigned)d.N0);
-  dd.fk = FDiv((unsigned)d.K0);
   int nsplit = 1;
   if (d.batch == 1 && tiles < (small ? 512 : 128) && K >= 256) {
     long long want = std::min<long long>((512 + tiles - 1) / tiles, (K + 127) / 128);
@@ -1002,8 +1288,7 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
   if (!tc_vec_disabled()) {
     if (p == Prec::F64)
       vec = vbig ? launch_vec<double, 128, 16>(dd, grid_big, A, B, C, W, s)
-                 : small ? launch_vec<double, 32, 32>(dd, grid, A, B, C, W, s)
-                         : !big && launch_vec<double, 64, 16>(dd, grid, A, B, C, W, s);
+                 : !big && launch_vec<double, 64, 16>(dd, grid, A, B, C, W, s);
     else if (p == Prec::F32)
       vec = vbig ? launch_vec<float, 128, 16>(dd, grid_big, A, B, C, W, s)
                  : small ? launch_vec<float, 32, 32>(dd, grid, A, B, C, W, s)
@@ -1013,10 +1298,7 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
   }
   if (!vec) switch (p) {
     case Prec::F64:
-      if (small)
-        hipLaunchKernelGGL((tc_kernel<double, TC_BK, 32>), grid, dim3(NT), 0, s, dd, (const double*)A,
-                           (const double*)B, (double*)C, (double*)W);
-      else if (big)
+      if (big)
         hipLaunchKernelGGL((tc_kernel<double, TC_BK, 128>), grid_big, dim3(NT), 0, s, dd, (const double*)A,
                            (const double*)B, (double*)C, (double*)W);
       else if (deep)
