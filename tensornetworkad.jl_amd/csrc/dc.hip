@@ -13,8 +13,8 @@
 //    skipped.
 //    The reflectors (v with v[j+1] = 1, zeros above) and their tau are written for the back
 //    transformation.
-//  * dc_kernel : divide and conquer on the tridiagonal matrix T (Cuppen's method), one workgroup.  T is
-//    torn recursively into halves down to 1 x 1 leaves, T = diag(T1, T2) + |b| u u^T with
+//  * dc_kernel : divide and conquer on the tridiagonal matrix T (Cuppen's method), a workgroup for each half of T.  A
+//    half is torn recursively down to leaves of one or two rows (solved directly), T = diag(T1, T2) + |b| u u^T with
 //    u = e_last + sign(b) e_first, and the tree is merged bottom-up, all merges of a level at once:
 //    the children's eigenpairs give D + rho z z^T, z = Q^T u / sqrt 2, rho = 2 |b|; entries with
 //    rho |z_i| below 8 eps max(|D|, rho |z|) deflate, and so does one of two entries whose Givens
@@ -25,11 +25,16 @@
 //    safeguarded by bisection on a bracket; z is then recomputed from the roots (Gu-Eisenstat, Lowner's
 //    formula), which makes the eigenvectors (zhat_i / (d_i - lambda_j))_i orthogonal to working
 //    accuracy; the merged eigenvectors are the children's (block-diagonal) eigenvector matrix times
-//    that K x K matrix (deflated columns are copied).  The eigenvector matrices of a level live in
-//    two m x m ping-pong buffers in global memory (L2-resident), a level's K x K matrices in a third.
-//    The top merge stops short of its product: it leaves the children's eigenvectors Z in Qb and its
-//    m x m merge matrix M (the K x K matrix scattered to the rows of its columns of Z, a 1 for each
-//    deflated column) in U, since H (Z M) = (H Z) M lets the product run over the whole chip.
+//    that K x K matrix (deflated columns are copied), on the matrix cores.
+//    A level is a chain of latencies, not of work: at m = 96, in one workgroup from single rows up, 325 k cycles, 127 k of
+//    them in the roots (four lanes per root, terms reread from LDS in every iteration) and 80 k in products of narrow
+//    merges, one output per thread.  Eight or sixteen lanes per root hold their terms in registers and add by DPP; the
+//    vectors are formed where their norms are; every product goes to the matrix cores; up to 72 rows per half the
+//    eigenvector matrices stay in LDS.  Divide and conquer with its top merge's roots, us at m = 48 / 80 / 96 / 128 / 192:
+//    105 / 141 / 162 / 185 / 310 before, 59 / 90 / 93 / 99 / 182 now.
+//  * dc_top_kernel, dc_sec_kernel, dc_zh_kernel : the merge of the two halves as far as its roots; it stops short of its
+//    product: it leaves the children's eigenvectors Z in Qb and its kept poles, roots and recomputed z, since
+//    H (Z M) = (H Z) M lets the product with the merge matrix M run over the whole chip.
 //  * trd_back_kernel : Z <- H_0 H_1 ... H_(m-3) Z, one wavefront per column of Z (no barriers), four
 //    reflectors per wavefront reduction.
 //  * dc_final_kernel : W = Z M, a 16 x 16 tile of W per workgroup on the FP64 matrix cores.
@@ -83,7 +88,7 @@ __device__ __forceinline__ void trd_reflect(const double (&c)[3], int j, int m, 
   const double a0 = lane_of(c[0], jr & 63), a1 = lane_of(c[1], jr & 63), a2 = lane_of(c[2], jr & 63);
   const double al = sl == 0 ? a0 : (sl == 1 ? a1 : a2);
   double be = al, tv = 0.0, sc = 0.0;
-  if (sg > 0.0) {
+  if (sg > 1e-300) {   // below, beta d leaves the range of a double (a rank-one matrix gets there by rounding noise of noise)
     const double nr = sqrt(al * al + sg);
     be = al >= 0.0 ? -nr : nr;
     const double d = al - be;             // |d| >= |al|: no cancellation
@@ -274,85 +279,89 @@ __global__ __launch_bounds__(TD_NT) void trd_kernel(const double* __restrict__ H
 // divide and conquer
 // ---------------------------------------------------------------------------------------------------
 constexpr int DC_NT = 1024;
-constexpr int DC_M = JACOBI_MAX;
-constexpr int DC_SEC = 256;   // threads from DC_SEC on work four lanes per root / per entry
-constexpr int DC_BIG = 32;    // levels whose widest merge reaches this use the matrix-core product
-constexpr int DC_ONE_LANE = 16;   // levels whose merges are at most this wide solve one root per lane
+constexpr int DC_SEC = 256;   // threads from DC_SEC on work L lanes per root / per entry
 
-struct DcShared {
-  double lam[DC_M];                 // eigenvalue of column g of the current eigenvector matrix
-  double ds[DC_M], zs[DC_M];        // merged node: d and z sorted ascending by d
-  int src[DC_M];                    // column of the sorted entry
-  int nlo[DC_M];                    // lo of the merge node of index g at this level (-1: none)
-  double dK[DC_M], zK[DC_M];        // kept entries (slots lo .. lo + K - 1)
-  double z2[DC_M];                  // rho zK^2
-  int kc[DC_M], ktype[DC_M];        // their columns; 0: top half only, 1: both halves, 2: bottom half only
-  double dvl[DC_M];                 // deflated eigenvalues (slots lo + K .. hi - 1)
-  int dcol[DC_M];                   // their columns
-  int org[DC_M];                    // pole (absolute slot) the root of slot lo + j is measured from
-  double tau[DC_M];                 // root = dK[org] + tau
-  double zh[DC_M], rn[DC_M];        // recomputed z; 1 / |u_j|
-  int upos[DC_M], kcp[DC_M];        // row of kept entry i in the K x K matrix (first its index within
-                                    // its type); column of row p
-  double rc[DC_M], rs[DC_M];        // deflation rotations of a node (slots lo ..)
-  int ra[DC_M], rb[DC_M];
-  int nK[DC_M], nT1[DC_M], nT12[DC_M], nRot[DC_M];   // per node at slot lo
-  double nRho[DC_M];
-  unsigned long long nmd[DC_M], nmz[DC_M];           // per node: bits of max |d|, max |z| (non-negative)
+// state of the merges of one level, NM: rows of the (sub)matrix at most
+template <int NM> struct DcShared {
+  double lam[NM];                 // eigenvalue of column g of the current eigenvector matrix
+  double ds[NM], zs[NM];          // merged node: d and z sorted ascending by d
+  int src[NM];                    // column of the sorted entry
+  int nlo[NM];                    // lo of the merge node of index g at this level (-1: none)
+  double dK[NM], zK[NM];          // kept entries (slots lo .. lo + K - 1)
+  double z2[NM];                  // rho zK^2
+  int kc[NM], ktype[NM];          // their columns; 0: top half only, 1: both halves, 2: bottom half only
+  double dvl[NM];                 // deflated eigenvalues (slots lo + K .. hi - 1)
+  int dcol[NM];                   // their columns
+  int org[NM];                    // pole (absolute slot) the root of slot lo + j is measured from
+  double tau[NM];                 // root = dK[org] + tau
+  double zh[NM];                  // recomputed z
+  int upos[NM], kcp[NM];          // row of kept entry i in the K x K matrix (first its index within
+                                  // its type); column of row p
+  double rc[NM], rs[NM];          // deflation rotations of a node (slots lo ..)
+  int ra[NM], rb[NM];
+  int nK[NM], nT1[NM], nT12[NM], nRot[NM];   // per node at slot lo
+  double nRho[NM];
+  unsigned long long nmd[NM], nmz[NM];       // per node: bits of max |d|, max |z| (non-negative)
+  double floor;                   // least deflation threshold of any node
 };
 
-// node of index g at depth dd (recursive halving of [0, m), the lower half the smaller); false when it
-// is a leaf (a single index, then lo = g, hi = g + 1)
+// node of index g at depth dd (recursive halving of [0, m), the lower half the smaller); false when it is a leaf (one
+// or two rows)
 __device__ __forceinline__ bool dc_node(int g, int dd, int m, int& lo, int& hi) {
   lo = 0;
   hi = m;
   for (int l = 0; l < dd; ++l) {
-    if (hi - lo <= 1) return false;
+    if (hi - lo <= 2) return false;
     const int mid = lo + ((hi - lo) >> 1);
     if (g < mid) hi = mid;
     else lo = mid;
   }
-  return hi - lo >= 2;
+  return dd == 0 || hi - lo > 2;
 }
 
+// levels of merges: halvings until no node has more than two rows
 __device__ __forceinline__ int dc_depth(int m) {
   int d = 0;
-  while ((1 << d) < m) ++d;
+  while ((2 << d) < m) ++d;
   return d;
 }
 
-// sums / products over the L lanes (L = 1 or 4, aligned) that share a root (butterflies: the same
-// bits in all of them)
+// sums / products over the L aligned lanes that share a root (butterflies: the same bits in all of them)
 template <int L>
 __device__ __forceinline__ double sumL(double x) {
-  if constexpr (L == 4) {
-    x += __shfl_xor(x, 1);
-    x += __shfl_xor(x, 2);
-  } else if constexpr (L == 64) {
-    x = wave_sum(x);
-  }
+  if constexpr (L == 64) return wave_sum(x);
+  x += dpp_d<0xB1>(x);
+  x += dpp_d<0x4E>(x);
+  if constexpr (L >= 8) x += dpp_d<0x141>(x);
+  if constexpr (L >= 16) x += dpp_d<0x140>(x);
   return x;
 }
 
 template <int L>
 __device__ __forceinline__ double prodL(double x) {
-  if constexpr (L == 4) {
-    x *= __shfl_xor(x, 1);
-    x *= __shfl_xor(x, 2);
-  } else if constexpr (L == 64) {
+  if constexpr (L == 64) {
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) x *= __shfl_xor(x, o);
+    return x;
   }
+  x *= dpp_d<0xB1>(x);
+  x *= dpp_d<0x4E>(x);
+  if constexpr (L >= 8) x *= dpp_d<0x141>(x);
+  if constexpr (L >= 16) x *= dpp_d<0x140>(x);
   return x;
 }
 
-// root j (0 <= j < K) of 1 + rho sum_i zk_i^2 / (dk_i - lambda) = 0, dk ascending, four lanes (q = 0..3)
-// sharing the sums.  Returns the pole o (index into dk) and lambda - dk[o].
 // 1 / x from the hardware estimate and two Newton steps (x finite and nonzero)
 __device__ __forceinline__ double rcp_nr(double x) {
   double r = __builtin_amdgcn_rcp(x);
   r = fma(r, fma(-x, r, 1.0), r);
   return fma(r, fma(-x, r, 1.0), r);
+}
+
+// a / b to the accuracy of a division (b finite and nonzero)
+__device__ __forceinline__ double div_nr(double a, double b) {
+  const double r = rcp_nr(b), q = a * r;
+  return fma(fma(-b, q, a), r, q);
 }
 
 // root e in (le, he) of c (djl - e)(djr - e) + s1 (djr - e) + s2 (djl - e) = 0 (the secular function
@@ -366,7 +375,12 @@ __device__ __forceinline__ bool dc_quad(double c, double djl, double djr, double
     e = -qc * rcp_nr(qb);
     return e > le && e < he;
   }
-  const double sq = sqrt(fmax(qb * qb - 4.0 * qa * qc, 0.0));
+  const double D = qb * qb - 4.0 * qa * qc;
+  double sq = 0.0;
+  if (D > 1e-290) {
+    const double y = __builtin_amdgcn_rsq(D);
+    sq = D * fma(0.5 * y, fma(-D * y, y, 1.0), y);
+  }
   const double qq = -0.5 * (qb + copysign(sq, qb));
   e = qq * rcp_nr(qa);
   if (e > le && e < he) return true;
@@ -375,64 +389,60 @@ __device__ __forceinline__ bool dc_quad(double c, double djl, double djr, double
   return e > le && e < he;
 }
 
-template <int L>
-__device__ void dc_secular(const double* dk, const double* z2, int K, int j, int q, int& o, double& t) {
-  // fn(i, d_i, rho z_i^2) for every term of this lane
-  auto terms = [&](auto&& fn) {
-    for (int i = q; i < K; i += L) fn(i, dk[i], z2[i]);
-  };
+// root j (0 <= j < K) of 1 + rho sum_i zk_i^2 / (dk_i - lambda) = 0, dk ascending, L lanes (q = 0 .. L - 1) sharing the
+// sums: lane q holds the terms q, q + L, ... (at most T) in registers.  Returns the pole o (index into dk) and
+// lambda - dk[o].
+template <int L, int T>
+__device__ __forceinline__ void dc_secular(const double* dk, const double* z2, int K, int j, int q, int& o, double& t) {
+  double d[T], w[T];   // a term that is not there: weight 0 at a distant pole
+#pragma unroll
+  for (int u = 0; u < T; ++u) {
+    const int i = q + L * u, ic = min(i, K - 1);
+    const double di = dk[ic], wi = z2[ic];
+    d[u] = i < K ? di : 1e300;
+    w[u] = i < K ? wi : 0.0;
+  }
   double lo_t, hi_t;
   if (j < K - 1) {
-    const double mdp = 0.5 * (dk[j] + dk[j + 1]);
+    const double dj = dk[j], dn = dk[j + 1], wj = z2[j], wn = z2[j + 1];
+    // the sign of the function midway picks the nearer pole; the midpoint is kept as an offset from d_j (rounded, it is off
+    // by eps |d|, which between two close poles with equal weights decides the sign and puts the root outside the bracket)
+    const double gap = dn - dj, hg = 0.5 * gap;
     double f = 0.0;
-    terms([&](int, double d, double w) { f += w * rcp_nr(d - mdp); });
+#pragma unroll
+    for (int u = 0; u < T; ++u) f += w[u] * rcp_nr((d[u] - dj) - hg);
     f = 1.0 + sumL<L>(f);
     o = f > 0.0 ? j : j + 1;
-    const double gap = dk[j + 1] - dk[j];
-    if (o == j) { lo_t = 0.0; hi_t = 0.5 * gap; }
-    else { lo_t = -0.5 * gap; hi_t = 0.0; }
+    if (o == j) { lo_t = 0.0; hi_t = hg; }
+    else { lo_t = -hg; hi_t = 0.0; }
     // first iterate: the two nearest poles exactly, the rest of the sum frozen at the midpoint
-    const double djl = dk[j] - dk[o], djr = dk[j + 1] - dk[o];
-    const double cc = f - z2[j] / (dk[j] - mdp) - z2[j + 1] / (dk[j + 1] - mdp);
+    const double djl = o == j ? 0.0 : -gap, djr = o == j ? gap : 0.0;
+    const double rh = rcp_nr(hg), cc = f + wj * rh - wn * rh;
     double e;
-    t = dc_quad(cc, djl, djr, z2[j], z2[j + 1], lo_t, hi_t, e) ? e : 0.5 * (lo_t + hi_t);
+    t = dc_quad(cc, djl, djr, wj, wn, lo_t, hi_t, e) ? e : 0.5 * (lo_t + hi_t);
   } else {
     double zz = 0.0;
-    terms([&](int, double, double w) { zz += w; });
+#pragma unroll
+    for (int u = 0; u < T; ++u) zz += w[u];
     o = j;
     lo_t = 0.0;
     hi_t = sumL<L>(zz);
     t = 0.5 * (lo_t + hi_t);
   }
   const double dorg = dk[o], dj = dk[j] - dorg, dj1 = j < K - 1 ? dk[j + 1] - dorg : 0.0;
+#pragma unroll
+  for (int u = 0; u < T; ++u) d[u] -= dorg;
   for (int it = 0; it < 80; ++it) {
-    // two terms per pass into separate sums, so the two reciprocal chains overlap
-    double f = 0.0, af = 0.0, psp = 0.0, php = 0.0, f2 = 0.0, af2 = 0.0, psp2 = 0.0, php2 = 0.0;
-    int i = q;
-    for (; i + L < K; i += 2 * L) {
-      const double r0 = rcp_nr((dk[i] - dorg) - t), r1 = rcp_nr((dk[i + L] - dorg) - t);
-      const double w0 = z2[i] * r0, w1 = z2[i + L] * r1;
-      f += w0;
-      f2 += w1;
-      af += fabs(w0);
-      af2 += fabs(w1);
-      if (i <= j) psp += w0 * r0;
-      else php += w0 * r0;
-      if (i + L <= j) psp2 += w1 * r1;
-      else php2 += w1 * r1;
+    double f = 0.0, af = 0.0, psp = 0.0, php = 0.0;
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const double r = rcp_nr(d[u] - t), x = w[u] * r, y = x * r;
+      f += x;
+      af += fabs(x);
+      const bool left = q + L * u <= j;
+      psp += left ? y : 0.0;
+      php += left ? 0.0 : y;
     }
-    if (i < K) {
-      const double r = rcp_nr((dk[i] - dorg) - t);
-      const double w = z2[i] * r;
-      f += w;
-      af += fabs(w);
-      if (i <= j) psp += w * r;
-      else php += w * r;
-    }
-    f += f2;
-    af += af2;
-    psp += psp2;
-    php += php2;
     f = 1.0 + sumL<L>(f);
     af = sumL<L>(af);
     psp = sumL<L>(psp);
@@ -448,13 +458,13 @@ __device__ void dc_secular(const double* dk, const double* z2, int K, int j, int
     if (j < K - 1) {
       const double djr = dj1 - t;
       const double s2 = djr * djr * php;
-      const double c = f - s1 * rcp_nr(djl) - s2 * rcp_nr(djr);
+      const double c = f - djl * psp - djr * php;
       double e;
       if (dc_quad(c, djl, djr, s1, s2, lo_t - t, hi_t - t, e)) { tn = t + e; ok = true; }
     } else {
-      const double c = f - s1 / djl;
+      const double c = f - djl * psp;
       if (c != 0.0) {
-        const double e = djl + s1 / c;
+        const double e = djl + s1 * rcp_nr(c);
         if (e > lo_t - t && e < hi_t - t) { tn = t + e; ok = true; }
       }
     }
@@ -473,14 +483,18 @@ struct DcScan {
   int sp = 0;
 };
 
-// deflation threshold of the node at lo: 8 eps max(max |d|, rho max |z|)
-__device__ __forceinline__ double dc_tol(const DcShared& sh, int lo, double rho) {
+// deflation threshold of the node at lo: 8 eps max(max |d|, rho max |z|), and no less than 1e-40 of the whole matrix (far
+// below what the tridiagonalisation left): a rank-deficient matrix leaves nodes of rounding noise of noise, 1e-115 and
+// smaller, where the squares in the secular function and the norms would leave the range of a double
+template <class SH>
+__device__ __forceinline__ double dc_tol(const SH& sh, int lo, double rho) {
   const double dmx = __longlong_as_double((long long)sh.nmd[lo]), zmx = __longlong_as_double((long long)sh.nmz[lo]);
-  return 8.0 * DBL_EPSILON * fmax(dmx, rho * zmx);
+  return fmax(8.0 * DBL_EPSILON * fmax(dmx, rho * zmx), sh.floor);
 }
 
 // keep entry (d, z, column src, rotated?) as kept entry number st.K
-__device__ __forceinline__ void dc_keep(DcShared& sh, int lo, int mid, double rho, double d, double z, int src,
+template <class SH>
+__device__ __forceinline__ void dc_keep(SH& sh, int lo, int mid, double rho, double d, double z, int src,
                                         bool rot, DcScan& st) {
   const int ty = rot ? 1 : (src < mid ? 0 : 2);
   sh.dK[lo + st.K] = d;
@@ -498,7 +512,8 @@ __device__ __forceinline__ void dc_keep(DcShared& sh, int lo, int mid, double rh
 // sequential scan of the sorted entries from .. hi - 1 (one lane): small z deflates; a close pending /
 // new pair is rotated (Givens on the two columns, recorded for the rows of Q) so that the pending entry
 // deflates
-__device__ __forceinline__ void dc_scan_seq(DcShared& sh, int lo, int hi, int mid, double rho, double tol, int from, DcScan& st) {
+template <class SH>
+__device__ __forceinline__ void dc_scan_seq(SH& sh, int lo, int hi, int mid, double rho, double tol, int from, DcScan& st) {
   double dnx = sh.ds[from], znx = sh.zs[from];
   int snx = sh.src[from];
   for (int nj = from; nj < hi; ++nj) {
@@ -546,7 +561,8 @@ __device__ __forceinline__ void dc_scan_seq(DcShared& sh, int lo, int hi, int mi
   }
 }
 
-__device__ __forceinline__ void dc_scan_finish(DcShared& sh, int lo, int mid, double rho, DcScan& st) {
+template <class SH>
+__device__ __forceinline__ void dc_scan_finish(SH& sh, int lo, int mid, double rho, DcScan& st) {
   if (st.have) dc_keep(sh, lo, mid, rho, st.dp, st.zp, st.sp, st.prot, st);
   sh.nK[lo] = st.K;
   sh.nT1[lo] = st.c0;
@@ -559,7 +575,8 @@ __device__ __forceinline__ void dc_scan_finish(DcShared& sh, int lo, int mid, do
 // no entry of a chunk lies within 2 tol of its predecessor (then nothing rotates: every entry that is not
 // deflated is kept, in order); from the first chunk with such a pair on, lane 0 scans sequentially
 // from the state the chunks before it left (the same state the sequential scan would have reached)
-__device__ __forceinline__ void dc_scan_wave(DcShared& sh, const double* __restrict__ ev, int lo, int hi, int lane) {
+template <class SH>
+__device__ __forceinline__ void dc_scan_wave(SH& sh, const double* __restrict__ ev, int lo, int hi, int lane) {
   const int mid = lo + ((hi - lo) >> 1);
   const double rho = 2.0 * fabs(ev[mid - 1]);
   const double tol = dc_tol(sh, lo, rho);
@@ -625,70 +642,76 @@ __device__ __forceinline__ void dc_scan_wave(DcShared& sh, const double* __restr
   }
 }
 
-// the roots of every merge of a level (threads DC_SEC.., L lanes per root), then z from the roots
-// (Lowner's formula) and the order of the kept columns, then the norms of the vectors u_j and the new
-// eigenvalues; three barriers
-template <int L>
-__device__ void dc_roots(DcShared& sh, int m, int tid) {
+// the roots of every merge of a level (threads DC_SEC.., L lanes per root, at most T terms each), then z from the roots
+// (Lowner's formula) and the order of the kept columns, then the normalised vectors u_j into U (K x K per node, transposed:
+// entry (row upos_i, column j) at U[lo + j + (lo + upos_i) LU]) and the new eigenvalues; three barriers
+template <int L, int T, int NM>
+__device__ __forceinline__ void dc_roots(DcShared<NM>& sh, double* U, int LU, int m, int tid) {
   const int g = (tid - DC_SEC) / L, q = (tid - DC_SEC) % L;
   const bool mine = tid >= DC_SEC && g < m && sh.nlo[g] >= 0;
-  if (mine) {
-    const int lo = sh.nlo[g], j = g - lo, K = sh.nK[lo];
-    if (j < K) {
-      int o;
-      double t;
-      dc_secular<L>(sh.dK + lo, sh.z2 + lo, K, j, q, o, t);
-      if (q == 0) {
-        sh.org[lo + j] = lo + o;
-        sh.tau[lo + j] = t;
-      }
+  const int lo = mine ? sh.nlo[g] : 0, j = g - lo, K = mine ? sh.nK[lo] : 0;
+  const bool root = mine && j < K;
+  int o = 0;
+  double t = 0.0;
+  if (root) {
+    dc_secular<L, T>(sh.dK + lo, sh.z2 + lo, K, j, q, o, t);
+    if (q == 0) {
+      sh.org[lo + j] = lo + o;
+      sh.tau[lo + j] = t;
     }
   }
   __syncthreads();
-  if (mine) {
-    const int lo = sh.nlo[g], i = g - lo, K = sh.nK[lo];
-    if (i < K) {
-      const double* dk = sh.dK + lo;
-      const double di = dk[i], rho = sh.nRho[lo];
-      double p = 1.0;
-      for (int jj = q; jj < K; jj += L) {
-        const double lmd = (sh.dK[sh.org[lo + jj]] - di) + sh.tau[lo + jj];
-        const double den = jj == K - 1 ? rho : (jj < i ? dk[jj] - di : dk[jj + 1] - di);
-        p *= lmd / den;
-      }
-      p = prodL<L>(p);
-      if (q == 0) {
-        sh.zh[lo + i] = copysign(sqrt(fmax(p, 0.0)), sh.zK[lo + i]);
-        const int ty = sh.ktype[lo + i];
-        const int pos = sh.upos[lo + i] + (ty == 0 ? 0 : (ty == 1 ? sh.nT1[lo] : sh.nT12[lo]));
-        sh.upos[lo + i] = pos;
-        sh.kcp[lo + pos] = sh.kc[lo + i];
-      }
+  if (root) {
+    const double* dk = sh.dK + lo;
+    const double di = dk[j], rho = sh.nRho[lo];
+    double p = 1.0;
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const int i = q + L * u, ic = min(i, K - 1);
+      const double lmd = (sh.dK[sh.org[lo + ic]] - di) + sh.tau[lo + ic];
+      const double den = ic == K - 1 ? rho : dk[ic < j ? ic : ic + 1] - di;
+      const double x = div_nr(lmd, den);
+      p *= i < K ? x : 1.0;
+    }
+    p = prodL<L>(p);
+    if (q == 0) {
+      sh.zh[lo + j] = copysign(sqrt(fmax(p, 0.0)), sh.zK[lo + j]);
+      const int ty = sh.ktype[lo + j];
+      const int pos = sh.upos[lo + j] + (ty == 0 ? 0 : (ty == 1 ? sh.nT1[lo] : sh.nT12[lo]));
+      sh.upos[lo + j] = pos;
+      sh.kcp[lo + pos] = sh.kc[lo + j];
     }
   }
   __syncthreads();
-  if (mine) {
-    const int lo = sh.nlo[g], j = g - lo, K = sh.nK[lo];
-    if (j < K) {
-      const double dorg = sh.dK[sh.org[lo + j]], tj = sh.tau[lo + j];
-      double s = 0.0;
-      for (int i = q; i < K; i += L) {
-        const double u = sh.zh[lo + i] / ((sh.dK[lo + i] - dorg) - tj);
-        s += u * u;
-      }
-      s = sumL<L>(s);
-      if (q == 0) {
-        sh.rn[lo + j] = 1.0 / sqrt(s);
-        sh.lam[lo + j] = dorg + tj;
-      }
-    } else if (q == 0) {
-      sh.lam[g] = sh.dvl[g];
+  if (root) {
+    const double dorg = sh.dK[lo + o];
+    double s = 0.0, v[T];
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const int i = q + L * u, ic = min(i, K - 1);
+      const double x = div_nr(sh.zh[lo + ic], (sh.dK[lo + ic] - dorg) - t);
+      v[u] = i < K ? x : 0.0;
+      s = fma(v[u], v[u], s);
     }
+    s = sumL<L>(s);
+    const double rn = 1.0 / sqrt(s);
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const int i = q + L * u;
+      if (i < K) U[(lo + j) + (size_t)(lo + sh.upos[lo + i]) * LU] = v[u] * rn;
+    }
+    if (q == 0) sh.lam[lo + j] = dorg + t;
+  } else if (mine && q == 0) {
+    sh.lam[g] = sh.dvl[g];
+  }
+  if (tid < m) {
+    sh.nmd[tid] = 0;
+    sh.nmz[tid] = 0;
   }
   __syncthreads();
 }
 
-// the top merge as dc_kernel leaves it (after its deflation and rotations) for dc_sec_kernel, dc_zh_kernel
+// the top merge as dc_top_kernel leaves it (after its deflation and rotations) for dc_sec_kernel, dc_zh_kernel
 // and dc_final_kernel: the K kept poles (ascending), their z and rho z^2, their columns of Z, the deflated
 // columns (slots K..m-1), and per root its pole, offset and recomputed z
 struct DcTop {
@@ -697,38 +720,63 @@ struct DcTop {
   double* rho;
 };
 
-// one level of merges: Qin holds the children's eigenvectors (block diagonal), Qout receives the
-// merged ones; U (m x m) holds each merge's K x K eigenvector matrix of D + rho z z^T, transposed, in
-// its diagonal block, rows ordered top-half columns, rotated columns, bottom-half columns.
-__device__ void dc_level(DcShared& sh, const double* __restrict__ ev, int m, int dd, double* __restrict__ Qin,
-                         double* __restrict__ Qout, double* __restrict__ U, const DcTop& top,
-                         double* __restrict__ lam_out, int tid) {
-  // children's eigenpairs -> z, sorted d of every merge node
-  if (tid < m) {
-    const int g = tid;
+// children's eigenpairs -> z, sorted d of every merge node of depth dd (DC_ZL lanes per index share its rank)
+constexpr int DC_ZL = 4;
+template <int NM>
+__device__ __forceinline__ void dc_gather(DcShared<NM>& sh, const double* __restrict__ ev, int m, int dd, const double* Qin,
+                                          int LD, int tid) {
+  const int g = tid / DC_ZL, q = tid % DC_ZL;
+  if (g < m) {
     int lo, hi;
     if (!dc_node(g, dd, m, lo, hi)) {
-      sh.nlo[g] = -1;
-      Qout[g + (size_t)g * m] = 1.0;   // a leaf passes through
+      if (q == 0) sh.nlo[g] = -1;
     } else {
-      sh.nlo[g] = lo;
       const int mid = lo + ((hi - lo) >> 1);
       const double be = ev[mid - 1];
-      double z = g < mid ? Qin[(mid - 1) + (size_t)g * m] : (be < 0.0 ? -Qin[mid + (size_t)g * m] : Qin[mid + (size_t)g * m]);
-      z *= 0.70710678118654752440;
-      const double lg = sh.lam[g];
+      const double x = Qin[(g < mid ? mid - 1 : mid) + (size_t)g * LD];
+      const double z = 0.70710678118654752440 * (g >= mid && be < 0.0 ? -x : x);
+      // (a NaN counts as the largest value, so the ranks are a permutation whatever the input)
+      const double lg = fmin(sh.lam[g], DBL_MAX);
       int rank = 0;
-      for (int h = lo; h < hi; ++h) {
-        const double lh = sh.lam[h];
+#pragma unroll 4
+      for (int h = lo + q; h < hi; h += DC_ZL) {
+        const double lh = fmin(sh.lam[h], DBL_MAX);
         rank += (lh < lg) || (lh == lg && h < g);
       }
-      sh.ds[lo + rank] = lg;
-      sh.zs[lo + rank] = z;
-      sh.src[lo + rank] = g;
-      atomicMax(&sh.nmd[lo], (unsigned long long)__double_as_longlong(fabs(lg)));
-      atomicMax(&sh.nmz[lo], (unsigned long long)__double_as_longlong(fabs(z)));
+      rank += __builtin_amdgcn_update_dpp(0, rank, 0xB1, 0xF, 0xF, true);
+      rank += __builtin_amdgcn_update_dpp(0, rank, 0x4E, 0xF, 0xF, true);
+      if (q == 0) {
+        sh.nlo[g] = lo;
+        sh.ds[lo + rank] = sh.lam[g];
+        sh.zs[lo + rank] = z;
+        sh.src[lo + rank] = g;
+        atomicMax(&sh.nmd[lo], (unsigned long long)__double_as_longlong(fabs(lg)));
+        atomicMax(&sh.nmz[lo], (unsigned long long)__double_as_longlong(fabs(z)));
+      }
     }
   }
+}
+
+// the deflation rotations of its node on row r of Qin
+template <int NM>
+__device__ __forceinline__ void dc_rotate(const DcShared<NM>& sh, double* Qin, int LD, int m, int r) {
+  if (r < m && sh.nlo[r] >= 0) {
+    const int lo = sh.nlo[r], nr = sh.nRot[lo];
+    for (int t = 0; t < nr; ++t) {
+      const size_t ia = r + (size_t)sh.ra[lo + t] * LD, ib = r + (size_t)sh.rb[lo + t] * LD;
+      const double x = Qin[ia], y = Qin[ib], c = sh.rc[lo + t], s = sh.rs[lo + t];
+      Qin[ia] = c * x + s * y;
+      Qin[ib] = -s * x + c * y;
+    }
+  }
+}
+
+// one level of merges: Qin holds the children's eigenvectors (block diagonal), Qout receives the
+// merged ones (ld LO).
+template <int L, int NM>
+__device__ __forceinline__ void dc_level(DcShared<NM>& sh, const double* __restrict__ ev, int m, int dd, double* Qin, int LD,
+                                         double* Qout, int LO, double* U, int LU, int tid) {
+  dc_gather(sh, ev, m, dd, Qin, LD, tid);
   __syncthreads();
   // deflation: a wavefront per merge node while a level has at most 16 of them (ballots decide whole chunks
   // of 64 entries at once until a close pair needs the sequential scan), else one thread per node
@@ -741,7 +789,7 @@ __device__ void dc_level(DcShared& sh, const double* __restrict__ ev, int m, int
         if ((wave >> l) & 1) lo = md;
         else hi = md;
       }
-      if (hi - lo >= 2) dc_scan_wave(sh, ev, lo, hi, lane);
+      if (hi - lo > 2) dc_scan_wave(sh, ev, lo, hi, lane);
     }
   } else if (tid < m && sh.nlo[tid] == tid) {
     int lo2, hi;
@@ -753,96 +801,32 @@ __device__ void dc_level(DcShared& sh, const double* __restrict__ ev, int m, int
     dc_scan_finish(sh, tid, mid, rho, st);
   }
   __syncthreads();
-  // deflation rotations on the rows of Qin (row-parallel); the secular roots, z from the roots, norms
-  if (tid < DC_SEC) {
-    const int r = tid;
-    if (r < m && sh.nlo[r] >= 0) {
-      const int lo = sh.nlo[r], nr = sh.nRot[lo];
-      for (int t = 0; t < nr; ++t) {
-        const size_t ia = r + (size_t)sh.ra[lo + t] * m, ib = r + (size_t)sh.rb[lo + t] * m;
-        const double x = Qin[ia], y = Qin[ib], c = sh.rc[lo + t], s = sh.rs[lo + t];
-        Qin[ia] = c * x + s * y;
-        Qin[ib] = -s * x + c * y;
-      }
-    }
-  }
-  if (dd == 0) {   // the top merge goes on over the whole chip (dc_sec_kernel, dc_zh_kernel, dc_final_kernel)
-    const int K = sh.nK[0];
-    if (tid < m) {
-      if (tid < K) {
-        top.dK[tid] = sh.dK[tid];
-        top.zK[tid] = sh.zK[tid];
-        top.z2[tid] = sh.z2[tid];
-        top.kc[tid] = sh.kc[tid];
-      } else {
-        top.dcol[tid] = sh.dcol[tid];
-        lam_out[tid] = sh.dvl[tid];
-      }
-    }
-    if (tid == 0) {
-      *top.K = K;
-      *top.rho = sh.nRho[0];
-    }
-    return;
-  }
+  // deflation rotations on the rows of Qin (row-parallel); the secular roots, z from the roots, vectors
+  if (tid < DC_SEC) dc_rotate(sh, Qin, LD, m, tid);
   const int smax = (m + (1 << dd) - 1) >> dd;   // the widest node of this level
-  // narrow merges: one lane per root; wide ones: four lanes share each root's sums
-  if (smax <= DC_ONE_LANE) dc_roots<1>(sh, m, tid);
-  else dc_roots<4>(sh, m, tid);
-  // the K x K eigenvector matrices: items (row r, column t) inside the node blocks
-  for (int it = tid; it < m * smax; it += DC_NT) {
-    const int r = it / smax, t = it % smax;
-    const int lo = sh.nlo[r];
-    if (lo < 0) continue;
-    const int K = sh.nK[lo], i = r - lo;
-    if (i >= K || t >= K) continue;
-    const double u = sh.zh[lo + i] / ((sh.dK[lo + i] - sh.dK[sh.org[lo + t]]) - sh.tau[lo + t]) * sh.rn[lo + t];
-    U[(lo + t) + (size_t)(lo + sh.upos[lo + i]) * m] = u;   // row p = upos of the K x K matrix, stored transposed
-  }
-  if (tid < m) {
-    sh.nmd[tid] = 0;
-    sh.nmz[tid] = 0;
-  }
-  __syncthreads();
-  // Qout = Qin[:, kept] U, deflated columns copied.  Levels of narrow merges: one output per item.
-  if (smax < DC_BIG) {
-    for (int it = tid; it < m * smax; it += DC_NT) {
-      const int r = it / smax, t = it % smax;
-      const int lo = sh.nlo[r];
-      if (lo < 0) continue;
-      int lo2, hi;
-      dc_node(r, dd, m, lo2, hi);
-      if (t >= hi - lo) continue;
-      const int K = sh.nK[lo], c = lo + t;
-      double acc;
-      if (t < K) {
-        acc = 0.0;
-        for (int p = 0; p < K; ++p) acc += Qin[r + (size_t)sh.kcp[lo + p] * m] * U[c + (size_t)(lo + p) * m];
-      } else {
-        acc = Qin[r + (size_t)sh.dcol[c] * m];
-      }
-      Qout[r + (size_t)c * m] = acc;
-    }
-    __syncthreads();
-    return;
-  }
-  // wide merges: 16 x 16 output tiles on the FP64 matrix cores, one wavefront per tile, operands
-  // straight from L2
+  constexpr int T = NM / L;
+  if (smax <= L) dc_roots<L, 1>(sh, U, LU, m, tid);
+  else if (2 * smax <= NM) dc_roots<L, (T + 1) / 2>(sh, U, LU, m, tid);
+  else dc_roots<L, T>(sh, U, LU, m, tid);
+  // Qout = Qin[:, kept] U, deflated columns copied: 16 x 16 output tiles on the FP64 matrix cores, one wavefront per
+  // tile
   const int wave = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
   int base = 0;
   const int nn = 1 << dd;
   for (int k = 0; k < nn; ++k) {
     int lo = 0, hi = m;
+    bool leaf = false;
     for (int l = dd - 1; l >= 0; --l) {
+      if (hi - lo <= 2) leaf = true;
       const int mid = lo + ((hi - lo) >> 1);
       if ((k >> l) & 1) lo = mid;
       else hi = mid;
     }
     const int s = hi - lo;
-    if (s < 2) continue;   // no merge node here (uniform)
+    if (leaf || s <= 2) continue;   // no merge node here (uniform)
     const int K = sh.nK[lo], mid = lo + (s >> 1);
     const int rt = (s + 15) >> 4, ct = (K + 15) >> 4, ntile = rt * ct;
-    for (int tl = wave - base; tl < ntile; tl += DC_NT / 64) {
+    for (int tl = wave - base % (DC_NT / 64); tl < ntile; tl += DC_NT / 64) {
       if (tl < 0) continue;
       const int r0 = lo + 16 * (tl % rt), t0 = 16 * (tl / rt);
       // rows of the top half meet only top-half and rotated columns, the bottom half the others
@@ -854,90 +838,178 @@ __device__ void dc_level(DcShared& sh, const double* __restrict__ ev, int m, int
       // stored, and the k-steps beyond p1 are zeroed through b
       const int rac = min(ra, hi - 1), tbc = min(tb, K - 1);
       d4 acc = {0.0, 0.0, 0.0, 0.0};
-      // eight k-steps per pass: the column indices first (one LDS wait), then all sixteen operand loads in
+      // four k-steps per pass: the column indices first (one LDS wait), then all eight operand loads in
       // flight before the first product
-      for (int p = p0; p < p1; p += 32) {
-        int kk[8];
+      for (int p = p0; p < p1; p += 16) {
+        int kk[4];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) kk[u] = sh.kcp[lo + min(p + 4 * u + lk, p1 - 1)];
-        double a[8], b[8];
+        for (int u = 0; u < 4; ++u) kk[u] = sh.kcp[lo + min(p + 4 * u + lk, p1 - 1)];
+        double a[4], b[4];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          a[u] = Qin[rac + (size_t)kk[u] * m];
-          b[u] = U[(lo + tbc) + (size_t)(lo + min(p + 4 * u + lk, p1 - 1)) * m];
+        for (int u = 0; u < 4; ++u) {
+          a[u] = Qin[rac + (size_t)kk[u] * LD];
+          b[u] = U[(lo + tbc) + (size_t)(lo + min(p + 4 * u + lk, p1 - 1)) * LU];
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
+        for (int u = 0; u < 4; ++u)
           acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], p + 4 * u + lk < p1 ? b[u] : 0.0, acc, 0, 0, 0);
       }
       // output lane layout of the 16 x 16 x 4 FP64 product: register q holds row lk + 4 q, column li
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int r = r0 + lk + 4 * q;
-        if (r < hi && tb < K) Qout[r + (size_t)(lo + tb) * m] = acc[q];
+        if (r < hi && tb < K) Qout[r + (size_t)(lo + tb) * LO] = acc[q];
       }
     }
     base += ntile;
     const int nd = s - K;
     for (int e = tid; e < nd * s; e += DC_NT) {
       const int r = lo + e % s, t = K + e / s;
-      Qout[r + (size_t)(lo + t) * m] = Qin[r + (size_t)sh.dcol[lo + t] * m];
+      Qout[r + (size_t)(lo + t) * LO] = Qin[r + (size_t)sh.dcol[lo + t] * LD];
     }
   }
   __syncthreads();
 }
 
-// tridiagonal (d, e) -> eigenvalues lam (unsorted); the eigenvectors are Qb M, with the top merge's matrix M
-// stored transposed in U (m x m each); Qa: m x m scratch
-__global__ __launch_bounds__(DC_NT) void dc_kernel(const double* __restrict__ d, const double* __restrict__ e, int m,
-                                                   double* __restrict__ Qa, double* __restrict__ Qb,
-                                                   double* __restrict__ U, DcTop top, double* __restrict__ lam_out,
-                                                   const int* __restrict__ gate) {
+// One half of the tridiagonal (d, e), rows [0, m / 2) or [m / 2, m) by block, torn off the other: its eigenvalues into lam
+// and its eigenvectors into its columns of Qb (zero outside its rows).  NM: rows of a half at most; up to DC_QL of them
+// the eigenvector matrices of the levels stay in LDS, above that they alternate between Qa and Qb.
+constexpr int DC_QL = 72;
+template <int L, int NM>
+__global__ __launch_bounds__(DC_NT) void dc_kernel(const double* __restrict__ d, const double* __restrict__ e, int mtot,
+                                                   double* __restrict__ Qag, double* __restrict__ Qbg,
+                                                   double* __restrict__ lam_out, const int* __restrict__ gate) {
   if (gate && *gate == 0) return;
-  __shared__ DcShared sh;
+  constexpr bool QL = NM <= DC_QL;
+  // pitch 16 mod 32 doubles: the columns of an operand read start in alternate halves of the banks
+  constexpr int LQ = NM + (48 - NM % 32) % 32;
+  __shared__ DcShared<NM> sh;
+  __shared__ double Us[NM * LQ];
+  __shared__ double Q0[QL ? NM * LQ : 1], Q1[QL ? NM * LQ : 1];
   const int tid = threadIdx.x;
+  const int base = blockIdx.x ? mtot >> 1 : 0, m = (blockIdx.x ? mtot : mtot >> 1) - base;
+  if (m < 1) return;
+  // |T|: a wavefront's maximum of the bits of |d|, |e|
+  if (tid < 64) {
+    double x = 0.0;
+    for (int i = tid; i < mtot; i += 64) x = fmax(x, fmax(fabs(d[i]), i + 1 < mtot ? fabs(e[i]) : 0.0));
+    for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o));
+    if (tid == 0) sh.floor = 1e-40 * x;
+  }
+  d += base;
+  e += base;
+  double* Zg = Qbg + base + (size_t)base * mtot;   // this half's block of Qb
   const int depth = dc_depth(m);
-  // the levels alternate between the buffers; the top merge reads Qb (as does dc_final_kernel when m = 1)
-  const bool odd = depth > 0 && ((depth - 1) & 1);
-  double* Qin = odd ? Qa : Qb;
-  double* Qout = odd ? Qb : Qa;
-  // Qin = I, Qout = 0; the row and column of each element advance without a division per element
+  // zeros outside the block
   {
-    const int rstep = DC_NT % m, cstep = DC_NT / m;
-    int r = tid % m, c = tid / m;
-    for (int idx = tid; idx < m * m; idx += DC_NT) {
-      Qin[idx] = r == c ? 1.0 : 0.0;
-      Qout[idx] = 0.0;
-      r += rstep;
-      c += cstep;
-      if (r >= m) {
-        r -= m;
-        ++c;
+    const int rows = mtot - m, r0 = blockIdx.x ? 0 : m;
+    for (int idx = tid; idx < rows * m; idx += DC_NT) Qbg[r0 + idx % rows + (size_t)(base + idx / rows) * mtot] = 0.0;
+  }
+  // the levels alternate between two matrices, both starting as the leaves' vectors; the last one writes Zg (in LDS) or
+  // ends there (in global memory)
+  constexpr int LDC = LQ;
+  const int LD = QL ? LDC : mtot;
+  double* const Ya = Qag + base + (size_t)base * mtot;
+  auto mat = [&](int par) -> double* {
+    if constexpr (QL) return par ? Q1 : Q0;
+    else return ((depth ^ par) & 1) ? Ya : Zg;   // level 0 (of depth levels) reads mat(0)
+  };
+  for (int idx = tid; idx < m * m; idx += DC_NT) {
+    const int r = idx % m, c = idx / m;
+    const double v = r == c ? 1.0 : 0.0;
+    mat(0)[r + (size_t)c * LD] = v;
+    if (depth > 0) mat(1)[r + (size_t)c * LD] = v;
+  }
+  __syncthreads();
+  // leaves of one or two rows; every boundary between leaves is a tear, d_i -= |e_i| on both sides of it
+  if (tid < m) {
+    int lo = 0, hi = m;
+    while (hi - lo > 2) {
+      const int mid = lo + ((hi - lo) >> 1);
+      if (tid < mid) hi = mid;
+      else lo = mid;
+    }
+    if (tid == lo) {
+      double a = d[lo] - (base + lo > 0 ? fabs(e[lo - 1]) : 0.0);
+      if (hi - lo == 2) {
+        const double b = e[lo], c = d[lo + 1] - (base + lo + 2 < mtot ? fabs(e[lo + 1]) : 0.0);
+        double l0 = a, l1 = c;
+        if (b != 0.0) {   // one Jacobi rotation
+          const double ze = (c - a) / (2.0 * b), t = copysign(1.0, ze) / (fabs(ze) + sqrt(1.0 + ze * ze));
+          const double cs = 1.0 / sqrt(1.0 + t * t), sn = cs * t;
+          l0 = a - t * b;
+          l1 = c + t * b;
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            double* Q = mat(k);
+            if (k && depth == 0) break;
+            Q[lo + (size_t)lo * LD] = cs;
+            Q[lo + 1 + (size_t)lo * LD] = -sn;
+            Q[lo + (size_t)(lo + 1) * LD] = sn;
+            Q[lo + 1 + (size_t)(lo + 1) * LD] = cs;
+          }
+        }
+        sh.lam[lo] = l0;
+        sh.lam[lo + 1] = l1;
+      } else {
+        if (base + lo + 1 < mtot) a -= fabs(e[lo]);
+        sh.lam[lo] = a;
       }
     }
-  }
-  // leaves: every boundary is a tear, d_i -= |e_(i-1)| + |e_i|
-  if (tid < m) {
-    double v = d[tid];
-    if (tid > 0) v -= fabs(e[tid - 1]);
-    if (tid < m - 1) v -= fabs(e[tid]);
-    sh.lam[tid] = v;
     sh.nmd[tid] = 0;
     sh.nmz[tid] = 0;
   }
   __syncthreads();
-  for (int dd = depth - 1; dd >= 0; --dd) {
-    dc_level(sh, e, m, dd, Qin, Qout, U, top, lam_out, tid);
-    if (dd == 0) break;
-    double* t = Qin;
-    Qin = Qout;
-    Qout = t;
+  for (int l = 0; l < depth; ++l) {
+    const int dd = depth - 1 - l;
+    double* Qout = QL && dd == 0 ? Zg : mat((l + 1) & 1);
+    dc_level<L>(sh, e, m, dd, mat(l & 1), LD, Qout, QL && dd == 0 ? mtot : LD, Us, LQ, tid);
   }
-  if (depth == 0 && tid == 0) {   // m = 1: Qb = 1, one deflated column
-    *top.K = 0;
-    top.dcol[0] = 0;
-    lam_out[0] = sh.lam[0];
+  if (QL && depth == 0 && tid < m * m) Zg[tid % m + (size_t)(tid / m) * mtot] = mat(0)[tid % m + (tid / m) * LD];
+  if (tid < m) lam_out[base + tid] = sh.lam[tid];
+}
+
+// the deflation of the top merge of the two halves (eigenvalues lam, eigenvectors Qb)
+__global__ __launch_bounds__(DC_NT) void dc_top_kernel(const double* __restrict__ e, int m, double* __restrict__ Qb, DcTop top,
+                                                       double* __restrict__ lam, const int* __restrict__ gate) {
+  if (gate && *gate == 0) return;
+  __shared__ DcShared<JACOBI_MAX> sh;
+  const int tid = threadIdx.x;
+  if (m == 1) {   // Qb = 1, one deflated column
+    if (tid == 0) {
+      *top.K = 0;
+      top.dcol[0] = 0;
+    }
+    return;
+  }
+  if (tid == 0) sh.floor = 0.0;   // the node is the whole matrix
+  if (tid < m) {
+    sh.lam[tid] = lam[tid];
+    sh.nmd[tid] = 0;
+    sh.nmz[tid] = 0;
+  }
+  __syncthreads();
+  dc_gather(sh, e, m, 0, Qb, m, tid);
+  __syncthreads();
+  if (tid < 64) dc_scan_wave(sh, e, 0, m, tid);
+  __syncthreads();
+  dc_rotate(sh, Qb, m, m, tid);
+  const int K = sh.nK[0];
+  if (tid < m) {
+    if (tid < K) {
+      top.dK[tid] = sh.dK[tid];
+      top.zK[tid] = sh.zK[tid];
+      top.z2[tid] = sh.z2[tid];
+      top.kc[tid] = sh.kc[tid];
+    } else {
+      top.dcol[tid] = sh.dcol[tid];
+      lam[tid] = sh.dvl[tid];
+    }
+  }
+  if (tid == 0) {
+    *top.K = K;
+    *top.rho = sh.nRho[0];
   }
 }
 
@@ -957,7 +1029,7 @@ __global__ __launch_bounds__(64) void dc_sec_kernel(DcTop top, double* __restric
   __syncthreads();
   int o;
   double t;
-  dc_secular<64>(dk, z2, K, j, lane, o, t);
+  dc_secular<64, JACOBI_MAX / 64>(dk, z2, K, j, lane, o, t);
   if (lane == 0) {
     top.org[j] = o;
     top.tau[j] = t;
@@ -976,7 +1048,7 @@ __global__ __launch_bounds__(64) void dc_zh_kernel(DcTop top, const int* __restr
   for (int jj = lane; jj < K; jj += 64) {
     const double lmd = (top.dK[top.org[jj]] - di) + top.tau[jj];
     const double den = jj == K - 1 ? rho : (jj < i ? top.dK[jj] - di : top.dK[jj + 1] - di);
-    p *= lmd / den;
+    p *= div_nr(lmd, den);
   }
   p = prodL<64>(p);
   if (lane == 0) top.zh[i] = copysign(sqrt(fmax(p, 0.0)), top.zK[i]);
@@ -1007,7 +1079,7 @@ __global__ __launch_bounds__(64) void dc_final_kernel(const double* __restrict__
   double sq = 0.0;
   if (kept)
     for (int i = lk; i < K; i += 4) {
-      const double u = zh[i] / ((dk[i] - dorg) - tt);
+      const double u = div_nr(zh[i], (dk[i] - dorg) - tt);
       sq += u * u;
     }
   sq += __shfl_xor(sq, 16);
@@ -1022,7 +1094,7 @@ __global__ __launch_bounds__(64) void dc_final_kernel(const double* __restrict__
     for (int u = 0; u < 16; ++u) {
       const int i = min(p + 4 * u + lk, K - 1);
       a[u] = Z[rac + (size_t)kc[i] * m];
-      b[u] = zh[i] / ((dk[i] - dorg) - tt) * rn;
+      b[u] = div_nr(zh[i], (dk[i] - dorg) - tt) * rn;
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1172,9 +1244,9 @@ void trd_launch(const double* H, int ldh, int m, double* d, double* e, double* V
   TNAD_HIP_TRY(hipGetLastError());
 }
 
-// the work buffer: Vh, Qa, Qb, U (m x m each), d, e, tau, lambda (m each), the reflector block products
+// the work buffer: Vh, Qa, Qb (m x m each), d, e, tau, lambda (m each), the reflector block products
 struct DcWork {
-  double *Vh, *Qa, *Qb, *U, *dv, *ev, *tau, *lam, *gram;
+  double *Vh, *Qa, *Qb, *dv, *ev, *tau, *lam, *gram;
   DcTop top;
 };
 
@@ -1184,8 +1256,7 @@ DcWork dc_work(double* w, int m) {
   d.Vh = w;
   d.Qa = d.Vh + mm;
   d.Qb = d.Qa + mm;
-  d.U = d.Qb + mm;
-  d.dv = d.U + mm;
+  d.dv = d.Qb + mm;
   d.ev = d.dv + m;
   d.tau = d.ev + m;
   d.lam = d.tau + m;
@@ -1211,7 +1282,12 @@ int dc_gram_blocks(int m) { return m > 2 ? ((m - 2 + 2 * BK_Q - 1) / (2 * BK_Q))
 // the divide and conquer: the merge tree below the top merge in one workgroup, the top merge's roots and z
 // over the whole chip
 void dc_solve(const DcWork& w, int m, const int* gate, hipStream_t s) {
-  hipLaunchKernelGGL(dc_kernel, dim3(1), dim3(DC_NT), 0, s, w.dv, w.ev, m, w.Qa, w.Qb, w.U, w.top, w.lam, gate);
+  const int half = (m + 1) / 2;
+  if (half <= 48) hipLaunchKernelGGL((dc_kernel<16, 48>), dim3(2), dim3(DC_NT), 0, s, w.dv, w.ev, m, w.Qa, w.Qb, w.lam, gate);
+  else if (half <= DC_QL) hipLaunchKernelGGL((dc_kernel<8, DC_QL>), dim3(2), dim3(DC_NT), 0, s, w.dv, w.ev, m, w.Qa, w.Qb, w.lam, gate);
+  else hipLaunchKernelGGL((dc_kernel<8, 96>), dim3(2), dim3(DC_NT), 0, s, w.dv, w.ev, m, w.Qa, w.Qb, w.lam, gate);
+  TNAD_HIP_TRY(hipGetLastError());
+  hipLaunchKernelGGL(dc_top_kernel, dim3(1), dim3(DC_NT), 0, s, w.ev, m, w.Qb, w.top, w.lam, gate);
   TNAD_HIP_TRY(hipGetLastError());
   if (m > 1) {
     hipLaunchKernelGGL(dc_sec_kernel, dim3(m), dim3(64), 0, s, w.top, w.lam, gate);
@@ -1237,7 +1313,7 @@ void dc_vectors(const DcWork& w, int m, const int* gate, hipStream_t s) {
 
 }  // namespace
 
-size_t syev_dc_work_doubles(int m) { return 4 * (size_t)m * m + 13 * (size_t)m + 56; }
+size_t syev_dc_work_doubles(int m) { return 3 * (size_t)m * m + 13 * (size_t)m + 56; }
 
 void syev_dc(const double* H, int ldh, int m, double* evals, double* V, double* work, hipStream_t s,
              const int* gate) {
