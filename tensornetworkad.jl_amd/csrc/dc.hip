@@ -28,10 +28,11 @@
 //    that K x K matrix (deflated columns are copied), on the matrix cores.
 //    A level is a chain of latencies, not of work: at m = 96, in one workgroup from single rows up, 325 k cycles, 127 k of
 //    them in the roots (four lanes per root, terms reread from LDS in every iteration) and 80 k in products of narrow
-//    merges, one output per thread.  Eight or sixteen lanes per root hold their terms in registers and add by DPP; the
-//    vectors are formed where their norms are; every product goes to the matrix cores; up to 72 rows per half the
-//    eigenvector matrices stay in LDS.  Divide and conquer with its top merge's roots, us at m = 48 / 80 / 96 / 128 / 192:
-//    105 / 141 / 162 / 185 / 310 before, 59 / 90 / 93 / 99 / 182 now.
+//    merges, one output per thread.  Eight lanes per root hold their terms in registers (as many slots as the level needs)
+//    and add by DPP (four or sixteen lanes: the same to 3 us more); the vectors are formed where their norms are;
+//    every product goes to the matrix cores, a wavefront per 16 x 16 tile; up to 72 rows per half the eigenvector matrices
+//    stay in LDS.  Divide and conquer with its top merge's roots, us at m = 48 / 80 / 96 / 128 / 192:
+//    105 / 141 / 162 / 185 / 310 before, 51 / 73 / 75 / 82 / 134 now.
 //  * dc_top_kernel, dc_sec_kernel, dc_zh_kernel : the merge of the two halves as far as its roots; it stops short of its
 //    product: it leaves the children's eigenvectors Z in Qb and its kept poles, roots and recomputed z, since
 //    H (Z M) = (H Z) M lets the product with the merge matrix M run over the whole chip.
@@ -60,7 +61,25 @@ struct TrdShared {
   double p[2][JACOBI_MAX];     // tau A v
   double colb[JACOBI_MAX];     // the same for the last step of a column block (column j + 1 in the next block)
   double tv[2];                // tau
+  double pp[2][TD_NT / 64];    // per wavefront: its rows' share of p . v
 };
+
+// 1 / x from the hardware estimate and two Newton steps (x finite and nonzero)
+__device__ __forceinline__ double rcp_nr(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(r, fma(-x, r, 1.0), r);
+  return fma(r, fma(-x, r, 1.0), r);
+}
+
+// sqrt(x) and 1 / sqrt(x) from the hardware estimate, refined to the accuracy of the square root (x normal and positive)
+__device__ __forceinline__ double sqrt_nr(double x, double& rs) {
+  double y = __builtin_amdgcn_rsq(x);
+  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  rs = y;
+  const double q = x * y;
+  return fma(fma(-q, q, x), 0.5 * y, q);
+}
 
 // the value of x in lane k (k uniform)
 __device__ __forceinline__ double lane_of(double x, int k) {
@@ -89,10 +108,12 @@ __device__ __forceinline__ void trd_reflect(const double (&c)[3], int j, int m, 
   const double al = sl == 0 ? a0 : (sl == 1 ? a1 : a2);
   double be = al, tv = 0.0, sc = 0.0;
   if (sg > 1e-300) {   // below, beta d leaves the range of a double (a rank-one matrix gets there by rounding noise of noise)
-    const double nr = sqrt(al * al + sg);
+    // refined estimates in place of the square root and the division: they are a chain that every wavefront waits for
+    double rs;
+    const double nr = sqrt_nr(al * al + sg, rs);
     be = al >= 0.0 ? -nr : nr;
-    const double d = al - be;             // |d| >= |al|: no cancellation
-    const double inv = 1.0 / (be * d);    // tau = (beta - alpha) / beta = -d^2 inv, 1 / d = beta inv
+    const double d = al - be;                // |d| >= |al|: no cancellation
+    const double inv = rcp_nr(be * d);       // tau = (beta - alpha) / beta = -d^2 inv, 1 / d = beta inv
     tv = -d * d * inv;
     sc = be * inv;
   }
@@ -159,6 +180,16 @@ __device__ __forceinline__ void trd_block(double (&A)[RA][RB], int m, TrdShared&
 #pragma unroll
       for (int a = A0; a < RA; ++a) ps[a] += dpp_d<0x142, 0xA>(ps[a]);
     }
+    // the rows' share of p . v (v is zero on finished rows), summed over the wavefront's four rows of lanes
+    double vr[RA], pq = 0.0;
+#pragma unroll
+    for (int a = A0; a < RA; ++a) {
+      vr[a] = vv[ty + TD_GY * a];
+      pq = fma(ps[a], vr[a], pq);
+    }
+    pq += dpp_d<0x142, 0xA>(pq);
+    pq += dpp_d<0x143, 0x8>(pq);
+    if (lane == 63) sh.pp[buf][tid >> 6] = tv * pq;
 #pragma unroll
     for (int a = A0; a < RA; ++a) {
       if (TD_GY * a + TD_GY - 1 <= j) continue;
@@ -182,9 +213,9 @@ __device__ __forceinline__ void trd_block(double (&A)[RA][RB], int m, TrdShared&
     }
     __syncthreads();
     // w = p - (tau / 2) (p . v) v ;  A -= v w^T + w v^T
-    double pw = 0.0;
-    for (int r = j + 1 + lane; r < m; r += 64) pw += pv[r] * vv[r];
-    pw = wave_sum(pw);
+    const double* pp = sh.pp[buf];
+    static_assert(TD_NT / 64 == 8, "eight shares");
+    const double pw = ((pp[0] + pp[1]) + (pp[2] + pp[3])) + ((pp[4] + pp[5]) + (pp[6] + pp[7]));
     const double kc = 0.5 * tv * pw;
     if (next && tid < 64) {   // column j + 1 after the update (v[j+1] = 1), then the next reflector
       const double* cn = j + 1 < j0 + TD_GX ? sh.col[buf] : sh.colb;
@@ -200,11 +231,10 @@ __device__ __forceinline__ void trd_block(double (&A)[RA][RB], int m, TrdShared&
     }
     // the thread's rows of v and w, then the update column by column (p is written this step only for
     // rows in unskipped blocks: columns at or left of j take w = 0)
-    double vr[RA], wr[RA];
+    double wr[RA];
 #pragma unroll
     for (int a = A0; a < RA; ++a) {
       const int r = ty + TD_GY * a;
-      vr[a] = vv[r];
       wr[a] = TD_GY * a + TD_GY - 1 <= j ? 0.0 : pv[r] - kc * vr[a];
     }
 #pragma unroll
@@ -349,13 +379,6 @@ __device__ __forceinline__ double prodL(double x) {
   if constexpr (L >= 8) x *= dpp_d<0x141>(x);
   if constexpr (L >= 16) x *= dpp_d<0x140>(x);
   return x;
-}
-
-// 1 / x from the hardware estimate and two Newton steps (x finite and nonzero)
-__device__ __forceinline__ double rcp_nr(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(r, fma(-x, r, 1.0), r);
-  return fma(r, fma(-x, r, 1.0), r);
 }
 
 // a / b to the accuracy of a division (b finite and nonzero)
@@ -804,69 +827,59 @@ __device__ __forceinline__ void dc_level(DcShared<NM>& sh, const double* __restr
   // deflation rotations on the rows of Qin (row-parallel); the secular roots, z from the roots, vectors
   if (tid < DC_SEC) dc_rotate(sh, Qin, LD, m, tid);
   const int smax = (m + (1 << dd) - 1) >> dd;   // the widest node of this level
-  constexpr int T = NM / L;
+  constexpr int T = NM / L, TH = (T + 1) / 2;
   if (smax <= L) dc_roots<L, 1>(sh, U, LU, m, tid);
-  else if (2 * smax <= NM) dc_roots<L, (T + 1) / 2>(sh, U, LU, m, tid);
+  else if (smax <= 2 * L) dc_roots<L, 2>(sh, U, LU, m, tid);
+  else if (T <= 3 || smax <= 3 * L) dc_roots<L, 3>(sh, U, LU, m, tid);
+  else if (smax <= TH * L) dc_roots<L, TH>(sh, U, LU, m, tid);
   else dc_roots<L, T>(sh, U, LU, m, tid);
   // Qout = Qin[:, kept] U, deflated columns copied: 16 x 16 output tiles on the FP64 matrix cores, one wavefront per
-  // tile
+  // tile, the same number of tiles for every node of the level
   const int wave = tid >> 6, lane = tid & 63, li = lane & 15, lk = lane >> 4;
-  int base = 0;
-  const int nn = 1 << dd;
-  for (int k = 0; k < nn; ++k) {
+  const int tn = (smax + 15) >> 4, items = (tn * tn) << dd;
+  for (int it = wave; it < items; it += DC_NT / 64) {
+    const int k = it / (tn * tn), tl = it - k * tn * tn;
     int lo = 0, hi = m;
-    bool leaf = false;
     for (int l = dd - 1; l >= 0; --l) {
-      if (hi - lo <= 2) leaf = true;
       const int mid = lo + ((hi - lo) >> 1);
       if ((k >> l) & 1) lo = mid;
       else hi = mid;
     }
-    const int s = hi - lo;
-    if (leaf || s <= 2) continue;   // no merge node here (uniform)
+    const int s = hi - lo, r0 = lo + 16 * (tl % tn), t0 = 16 * (tl / tn);
+    if (s <= 2 || r0 >= hi || t0 >= s) continue;   // a leaf, or no such tile in this node (uniform)
     const int K = sh.nK[lo], mid = lo + (s >> 1);
-    const int rt = (s + 15) >> 4, ct = (K + 15) >> 4, ntile = rt * ct;
-    for (int tl = wave - base % (DC_NT / 64); tl < ntile; tl += DC_NT / 64) {
-      if (tl < 0) continue;
-      const int r0 = lo + 16 * (tl % rt), t0 = 16 * (tl / rt);
-      // rows of the top half meet only top-half and rotated columns, the bottom half the others
-      const int p0 = r0 >= mid ? sh.nT1[lo] : 0;
-      const int p1 = r0 + 15 < mid ? sh.nT12[lo] : K;
-      const int ra = r0 + li;   // A-fragment row of this lane (A[li][lk])
-      const int tb = t0 + li;   // B-fragment column of this lane (B[lk][li])
-      // clamped addresses, no branches: rows and columns beyond the node only feed outputs that are not
-      // stored, and the k-steps beyond p1 are zeroed through b
-      const int rac = min(ra, hi - 1), tbc = min(tb, K - 1);
-      d4 acc = {0.0, 0.0, 0.0, 0.0};
-      // four k-steps per pass: the column indices first (one LDS wait), then all eight operand loads in
-      // flight before the first product
-      for (int p = p0; p < p1; p += 16) {
-        int kk[4];
+    // rows of the top half meet only top-half and rotated columns, the bottom half the others
+    const int p0 = r0 >= mid ? sh.nT1[lo] : 0;
+    const int p1 = t0 >= K ? 0 : (r0 + 15 < mid ? sh.nT12[lo] : K);
+    const int ra = r0 + li;   // A-fragment row of this lane (A[li][lk])
+    const int tb = t0 + li;   // B-fragment column of this lane (B[lk][li])
+    // clamped addresses, no branches: rows and columns beyond the node only feed outputs that are not
+    // stored, and the k-steps beyond p1 are zeroed through b
+    const int rac = min(ra, hi - 1), tbc = min(tb, K - 1);
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+    // four k-steps per pass: the column indices first (one LDS wait), then all eight operand loads in
+    // flight before the first product
+    for (int p = p0; p < p1; p += 16) {
+      int kk[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) kk[u] = sh.kcp[lo + min(p + 4 * u + lk, p1 - 1)];
-        double a[4], b[4];
+      for (int u = 0; u < 4; ++u) kk[u] = sh.kcp[lo + min(p + 4 * u + lk, p1 - 1)];
+      double a[4], b[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          a[u] = Qin[rac + (size_t)kk[u] * LD];
-          b[u] = U[(lo + tbc) + (size_t)(lo + min(p + 4 * u + lk, p1 - 1)) * LU];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], p + 4 * u + lk < p1 ? b[u] : 0.0, acc, 0, 0, 0);
+      for (int u = 0; u < 4; ++u) {
+        a[u] = Qin[rac + (size_t)kk[u] * LD];
+        b[u] = U[(lo + tbc) + (size_t)(lo + min(p + 4 * u + lk, p1 - 1)) * LU];
       }
-      // output lane layout of the 16 x 16 x 4 FP64 product: register q holds row lk + 4 q, column li
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int r = r0 + lk + 4 * q;
-        if (r < hi && tb < K) Qout[r + (size_t)(lo + tb) * LO] = acc[q];
-      }
+      for (int u = 0; u < 4; ++u)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], p + 4 * u + lk < p1 ? b[u] : 0.0, acc, 0, 0, 0);
     }
-    base += ntile;
-    const int nd = s - K;
-    for (int e = tid; e < nd * s; e += DC_NT) {
-      const int r = lo + e % s, t = K + e / s;
-      Qout[r + (size_t)(lo + t) * LO] = Qin[r + (size_t)sh.dcol[lo + t] * LD];
+    // output lane layout of the 16 x 16 x 4 FP64 product: register q holds row lk + 4 q, column li
+    const int src = tb >= K && tb < s ? sh.dcol[lo + tb] : 0;   // a deflated column is copied
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = r0 + lk + 4 * q;
+      if (r < hi && tb < s) Qout[r + (size_t)(lo + tb) * LO] = tb < K ? acc[q] : Qin[r + (size_t)src * LD];
     }
   }
   __syncthreads();
@@ -1234,7 +1247,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 }
 
 // Instances for m up to 48, 96, 144, 192 (us at m = 20 / 48 / 80 / 128 with the last one for all: 48 / 102 / 159 / 229;
-// with these: 25 / 54 / 105 / 191)
+// with these: 24 / 52 / 98 / 189)
 void trd_launch(const double* H, int ldh, int m, double* d, double* e, double* Vh, double* tau, const int* gate,
                 hipStream_t s) {
   if (m <= 48) hipLaunchKernelGGL((trd_kernel<2, 3>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, gate);
@@ -1283,7 +1296,7 @@ int dc_gram_blocks(int m) { return m > 2 ? ((m - 2 + 2 * BK_Q - 1) / (2 * BK_Q))
 // over the whole chip
 void dc_solve(const DcWork& w, int m, const int* gate, hipStream_t s) {
   const int half = (m + 1) / 2;
-  if (half <= 48) hipLaunchKernelGGL((dc_kernel<16, 48>), dim3(2), dim3(DC_NT), 0, s, w.dv, w.ev, m, w.Qa, w.Qb, w.lam, gate);
+  if (half <= 48) hipLaunchKernelGGL((dc_kernel<8, 48>), dim3(2), dim3(DC_NT), 0, s, w.dv, w.ev, m, w.Qa, w.Qb, w.lam, gate);
   else if (half <= DC_QL) hipLaunchKernelGGL((dc_kernel<8, DC_QL>), dim3(2), dim3(DC_NT), 0, s, w.dv, w.ev, m, w.Qa, w.Qb, w.lam, gate);
   else hipLaunchKernelGGL((dc_kernel<8, 96>), dim3(2), dim3(DC_NT), 0, s, w.dv, w.ev, m, w.Qa, w.Qb, w.lam, gate);
   TNAD_HIP_TRY(hipGetLastError());
