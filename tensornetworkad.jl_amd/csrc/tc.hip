@@ -662,109 +662,101 @@ __global__ __launch_bounds__(64 * SLAB_W) void tc_slab_kernel(TcDesc d, const do
 }
 
 // ---------------------------------------------------------------------------
-// Complex FP64 kernel for small outputs: both planes of both operands staged together, 32 x 32 output tile per
-// workgroup, each of the 4 waves one 16 x 16 block with three accumulators (Ar Br, Ai Bi, Ar Bi + Ai Br), K-tile 16,
-// double-buffered LDS (49 KB).  A complex contraction of the sizes the complex path runs (corner matrix up to
-// 96 x 96) is bound by launch and latency, not by its products: as four real launches, two of them reading back
-// the output, it took 4 x 5.3 us.
+// Complex FP64 contraction in one launch, the planes of both operands as tc_slab_kernel reads them: 16 x 16 output tile per
+// workgroup, each of the 8 waves its own share of K with four accumulators (Ar Br, Ai Bi, Ar Bi, Ai Br), added over the
+// waves in LDS.  A complex contraction of the sizes the complex path runs (corner matrix up to 96 x 96) is bound by launch
+// and latency, not by its products: four real launches of 5.3 us, two of them reading back the output, then one with LDS
+// tiles and a barrier per 16 of K, 8.4 us on average over a chi = 12 gradient; this one 4.2.
 // ---------------------------------------------------------------------------
-constexpr int ZT = 32, ZBK = 16;
-__global__ __launch_bounds__(NT) void ztc_kernel(TcDesc d, const double* __restrict__ A, long long pA, double sa,
-                                                 const double* __restrict__ B, long long pB, double sb,
-                                                 double* __restrict__ C, long long pC) {
-  constexpr int PAD = 16, NR = ZT * ZBK / NT;   // loads per thread, operand and plane per K-tile (2)
-  __shared__ double As[2][2][ZBK][ZT + PAD];    // [buffer][plane]
-  __shared__ double Bs[2][2][ZBK][ZT + PAD];
+template <int AM, int BMD>
+__global__ __launch_bounds__(64 * SLAB_W) void ztc_kernel(TcDesc d, const double* __restrict__ A, long long pA, double sa,
+                                                          const double* __restrict__ B, long long pB, double sb,
+                                                          double* __restrict__ C, long long pC) {
+  constexpr int W = SLAB_W;
+  typedef SlabOperand<1, AM> OpA;
+  typedef SlabOperand<1, BMD> OpB;
+  constexpr int RP = 4 * 68;   // as in tc_slab_kernel
+  constexpr int WL = 2 * (OpA::LDS + OpB::LDS);
+  __shared__ __attribute__((aligned(16))) double sh[W * (WL > 4 * RP ? WL : 4 * RP)];
   const int M = d.M0 * d.M1, N = d.N0 * d.N1, K = d.K0 * d.K1;
-  const int tile_m = blockIdx.x * ZT, tile_n = blockIdx.y * ZT;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave & 1, wn = wave >> 1;
-  const bool a_mfast = (d.am0 == 1 && d.M0 > 1) || d.ak0 != 1;
-  const bool b_nfast = (d.bn0 == 1 && d.N0 > 1) || d.bk0 != 1;
-  int a_mi[NR], a_ki[NR], b_ni[NR], b_ki[NR];
-  long long a_off[NR], b_off[NR];
-  bool a_ok[NR], b_ok[NR];
-  KPos a_kp[NR], b_kp[NR];
-  const long long a_dk = d.ak1 - (long long)d.K0 * d.ak0, b_dk = d.bk1 - (long long)d.K0 * d.bk0;
+  const int tile_m = blockIdx.x * 16, tile_n = blockIdx.y * 16;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  OpA a[2];
+  OpB b[2];
 #pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    if (a_mfast) { a_mi[r] = t % ZT; a_ki[r] = t / ZT + (NT / ZT) * r; }
-    else         { a_ki[r] = t % ZBK; a_mi[r] = t / ZBK + (NT / ZBK) * r; }
-    if (b_nfast) { b_ni[r] = t % ZT; b_ki[r] = t / ZT + (NT / ZT) * r; }
-    else         { b_ki[r] = t % ZBK; b_ni[r] = t / ZBK + (NT / ZBK) * r; }
-    const int m = tile_m + a_mi[r], n = tile_n + b_ni[r];
-    a_ok[r] = m < M;
-    b_ok[r] = n < N;
-    a_off[r] = a_ok[r] ? off2(m, d.M0, d.fm, d.am0, d.am1) : 0;
-    b_off[r] = b_ok[r] ? off2(n, d.N0, d.fn, d.bn0, d.bn1) : 0;
-    a_kp[r].init(a_ki[r], d.K0, d.fk, d.ak0, d.ak1);
-    b_kp[r].init(b_ki[r], d.K0, d.fk, d.bk0, d.bk1);
+  for (int p = 0; p < 2; ++p) {
+    a[p].init(A + p * pA, tile_m, M, d.M0, d.fm, d.am0, d.am1, d.ak0, d.ak1, lane);
+    b[p].init(B + p * pB, tile_n, N, d.N0, d.fn, d.bn0, d.bn1, d.bk0, d.bk1, lane);
   }
-  double ra[2][NR], rb[2][NR];
-  auto gload = [&](int k0) {
+  double* wl = sh + wave * WL;
+  d4 acc[2][2] = {{{0, 0, 0, 0}, {0, 0, 0, 0}}, {{0, 0, 0, 0}, {0, 0, 0, 0}}};   // [plane of A][plane of B]
+  double xa[2][1][4], xb[2][1][4];
+  auto mul = [&] {
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      ra[0][r] = ra[1][r] = rb[0][r] = rb[1][r] = 0.0;
-      if (a_ok[r] && k0 + a_ki[r] < K) {
-        const long long o = a_off[r] + a_kp[r].off;
-        ra[0][r] = A[o];
-        ra[1][r] = sa * A[o + pA];
-      }
-      if (b_ok[r] && k0 + b_ki[r] < K) {
-        const long long o = b_off[r] + b_kp[r].off;
-        rb[0][r] = B[o];
-        rb[1][r] = sb * B[o + pB];
-      }
-      a_kp[r].advance(ZBK, d.K0, d.ak0, a_dk);
-      b_kp[r].advance(ZBK, d.K0, d.bk0, b_dk);
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[p][q] = MfmaOp<double>::run(xa[p][0][e], xb[q][0][e], acc[p][q]);
+  };
+  const int Kw = K & ~15;
+  int kb = 16 * wave;
+  auto load = [&](int k) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      a[p].load(k, lane, d);
+      b[p].load(k, lane, d);
     }
   };
-  auto stage = [&](int buf) {
+  if (kb < Kw) load(kb);
+  for (; kb < Kw; kb += 16 * W) {
 #pragma unroll
-    for (int r = 0; r < NR; ++r)
+    for (int p = 0; p < 2; ++p) {
+      a[p].operand(xa[p], wl + p * OpA::LDS, lane);
+      b[p].operand(xb[p], wl + 2 * OpA::LDS + p * OpB::LDS, lane);
+    }
+    if (kb + 16 * W < Kw) load(kb + 16 * W);
+    mul();
+  }
+  if (kb == Kw && Kw < K) {   // the wave whose turn it is takes the remainder
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        As[buf][q][a_ki[r]][a_mi[r]] = ra[q][r];
-        Bs[buf][q][b_ki[r]][b_ni[r]] = rb[q][r];
+    for (int p = 0; p < 2; ++p) {
+      a[p].load_tail(kb, lane, d, K);
+      b[p].load_tail(kb, lane, d, K);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        xa[p][0][e] = a[p].v[0][e];
+        xb[p][0][e] = b[p].v[0][e];
       }
-  };
-  d4 rr = {0, 0, 0, 0}, ii = {0, 0, 0, 0}, ri = {0, 0, 0, 0};
-  gload(0);
-  stage(0);
-  if (ZBK < K) gload(ZBK);
+    }
+    mul();
+  }
+  if (WL > 0) __syncthreads();   // the partial tiles take the place of the transposition rows
+  double* red = sh + wave * 4 * RP;
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[(2 * p + q) * RP + 68 * r + 17 * (lane >> 4) + (lane & 15)] = acc[p][q][r];
   __syncthreads();
-  int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += ZBK, buf ^= 1) {
+  // threads 0..255 the real plane, the others the imaginary one
+  const int e = threadIdx.x & 255, ml = e & 15, nl = e >> 4, im = threadIdx.x >> 8;
+  const int m = tile_m + ml, n = tile_n + nl;
+  if (m >= M || n >= N) return;
+  const double* p0 = sh + (im ? RP : 0) + 68 * (ml >> 2) + 17 * (ml & 3) + nl;   // Ar Br or Ar Bi
+  const double* p1 = p0 + (im ? RP : 3 * RP);                                    // Ai Bi or Ai Br
+  double u = p0[0], w = p1[0];
 #pragma unroll
-    for (int kk = 0; kk < ZBK; kk += 4) {
-      const int row = kk + (lane >> 4), ca = wm * 16 + (lane & 15), cb = wn * 16 + (lane & 15);
-      const double ar = As[buf][0][row][ca], ai = As[buf][1][row][ca], br = Bs[buf][0][row][cb], bi = Bs[buf][1][row][cb];
-      rr = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, rr, 0, 0, 0);
-      ii = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bi, ii, 0, 0, 0);
-      ri = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, ri, 0, 0, 0);
-      ri = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, ri, 0, 0, 0);
-    }
-    if (k0 + ZBK < K) {
-      stage(buf ^ 1);
-      if (k0 + 2 * ZBK < K) gload(k0 + 2 * ZBK);
-    }
-    __syncthreads();
+  for (int k = 1; k < W; ++k) {
+    u += p0[k * 4 * RP];
+    w += p1[k * 4 * RP];
   }
-  const int n = tile_n + wn * 16 + (lane & 15);
-  if (n >= N) return;
-  const long long noff = off2(n, d.N0, d.fn, d.cn0, d.cn1);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int m = tile_m + wm * 16 + MfmaOp<double>::row(lane, r);
-    if (m >= M) continue;
-    const long long o = noff + off2(m, d.M0, d.fm, d.cm0, d.cm1);
-    double vr = d.alpha * (rr[r] - ii[r]), vi = d.alpha * ri[r];
-    if (d.beta != 0.0) {
-      vr += d.beta * C[o];
-      vi += d.beta * C[o + pC];
-    }
-    C[o] = vr;
-    C[o + pC] = vi;
-  }
+  double v = d.alpha * (im ? sb * u + sa * w : u - sa * sb * w);
+  C += im ? pC : 0;
+  const long long o = off2(m, d.M0, d.fm, d.cm0, d.cm1) + off2(n, d.N0, d.fn, d.cn0, d.cn1);
+  if (d.beta != 0.0) v += d.beta * C[o];
+  C[o] = v;
 }
 
 // split-K reduction: C = alpha * sum_s W[s] + beta * C over the strided output (slices summed in
@@ -1342,15 +1334,18 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
   }
 }
 
-// The complex kernel up to ZTC_TILES 32 x 32 tiles and K up to ZTC_K; four real launches above, where the 64 x 64 tiles, the
-// 16-byte loads and the split along K of tc_launch pay.
-constexpr long long ZTC_TILES = 1024, ZTC_K = 512;
+// The complex kernel up to ZTC_TILES 16 x 16 tiles and ZTC_K of K; four real launches above, where tc_launch has larger tiles
+// and the split along the grid.
+constexpr long long ZTC_TILES = 4096, ZTC_K = 8192;
 void ztc_launch(Ctx* c, const TcDesc& d, const double* A, size_t planeA, bool conjA, const double* B, size_t planeB,
                 bool conjB, double* C, size_t planeC, hipStream_t s) {
   const double sa = conjA ? -1.0 : 1.0, sb = conjB ? -1.0 : 1.0;
   const long long M = (long long)d.M0 * d.M1, N = (long long)d.N0 * d.N1, K = (long long)d.K0 * d.K1;
-  const long long tiles = ((M + ZT - 1) / ZT) * ((N + ZT - 1) / ZT);
-  if (d.batch != 1 || tiles > ZTC_TILES || K > ZTC_K || M <= 0 || N <= 0 || K <= 0) {
+  const long long tiles = (M + 15) / 16 * ((N + 15) / 16);
+  const bool empty = M <= 0 || N <= 0 || K <= 0;
+  const size_t ea = empty ? 0 : extent_bytes(d.M0, d.am0, d.M1, d.am1, d.K0, d.ak0, d.K1, d.ak1, 1, 0, 8),
+               eb = empty ? 0 : extent_bytes(d.K0, d.bk0, d.K1, d.bk1, d.N0, d.bn0, d.N1, d.bn1, 1, 0, 8);
+  if (empty || d.batch != 1 || tiles > ZTC_TILES || K > ZTC_K || ea >= (1ull << 32) || eb >= (1ull << 32)) {
     // (Ar + i sa Ai)(Br + i sb Bi) = (Ar Br - sa sb Ai Bi) + i (sb Ar Bi + sa Ai Br)
     const double *Ai = A + planeA, *Bi = B + planeB;
     double* Ci = C + planeC;
@@ -1365,9 +1360,7 @@ void ztc_launch(Ctx* c, const TcDesc& d, const double* A, size_t planeA, bool co
     tc_launch(c, Prec::F64, x, Ai, B, Ci, s);
     return;
   }
-  const size_t ea = extent_bytes(d.M0, d.am0, d.M1, d.am1, d.K0, d.ak0, d.K1, d.ak1, 1, 0, 8),
-               eb = extent_bytes(d.K0, d.bk0, d.K1, d.bk1, d.N0, d.bn0, d.N1, d.bn1, 1, 0, 8),
-               ec = extent_bytes(d.M0, d.cm0, d.M1, d.cm1, d.N0, d.cn0, d.N1, d.cn1, 1, 0, 8);
+  const size_t ec = extent_bytes(d.M0, d.cm0, d.M1, d.cm1, d.N0, d.cn0, d.N1, d.cn1, 1, 0, 8);
   c->check_range(A, planeA * 8 + ea, "ztc A");
   c->check_range(B, planeB * 8 + eb, "ztc B");
   c->check_range(C, planeC * 8 + ec, "ztc C");
@@ -1375,8 +1368,13 @@ void ztc_launch(Ctx* c, const TcDesc& d, const double* A, size_t planeA, bool co
   x.fm = FDiv((unsigned)d.M0);
   x.fn = FDiv((unsigned)d.N0);
   x.fk = FDiv((unsigned)d.K0);
-  hipLaunchKernelGGL(ztc_kernel, dim3((unsigned)((M + ZT - 1) / ZT), (unsigned)((N + ZT - 1) / ZT)), dim3(NT), 0, s, x, A,
-                     (long long)planeA, sa, B, (long long)planeB, sb, C, (long long)planeC);
+  const dim3 grid((unsigned)((M + 15) / 16), (unsigned)((N + 15) / 16)), block(64 * SLAB_W);
+  const int am = slab_mode(d, d.M0, d.am0, d.ak0, false), bm = slab_mode(d, d.N0, d.bn0, d.bk0, false);
+  const long long qA = (long long)planeA, qB = (long long)planeB, qC = (long long)planeC;
+  if (am == 2 && bm == 2) hipLaunchKernelGGL((ztc_kernel<2, 2>), grid, block, 0, s, x, A, qA, sa, B, qB, sb, C, qC);
+  else if (am == 2) hipLaunchKernelGGL((ztc_kernel<2, 0>), grid, block, 0, s, x, A, qA, sa, B, qB, sb, C, qC);
+  else if (bm == 2) hipLaunchKernelGGL((ztc_kernel<0, 2>), grid, block, 0, s, x, A, qA, sa, B, qB, sb, C, qC);
+  else hipLaunchKernelGGL((ztc_kernel<0, 0>), grid, block, 0, s, x, A, qA, sa, B, qB, sb, C, qC);
   TNAD_HIP_TRY(hipGetLastError());
 }
 
