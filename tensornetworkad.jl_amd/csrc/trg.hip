@@ -69,16 +69,12 @@ __global__ void permute4_back_kernel(const double* __restrict__ gin, int d0, int
   }
 }
 
-// one block: max |x| and its first index
-__global__ void maxabs_kernel(const double* __restrict__ x, size_t n, double* out_val, int* out_idx) {
+// max |x|, its first index and the entry there.  maxabs_part_kernel: each block's maximum (val) and index over its strided
+// share; maxabs_kernel (one block) over the parts, out = {max, index, entry}.  One block over a whole tensor waits for
+// memory: 64 us on average over the steps of a chi = 32 run (32^4 entries at the end), now 7 with both launches.
+__device__ __forceinline__ void maxabs_block(double& best, int& idx) {   // over the block, valid in thread 0
   __shared__ double bv[16];
   __shared__ int bi[16];
-  double best = -1.0;
-  int idx = 0x7fffffff;
-  for (size_t e = threadIdx.x; e < n; e += blockDim.x) {
-    double v = fabs(x[e]);
-    if (v > best) { best = v; idx = (int)e; }
-  }
   for (int o = 32; o > 0; o >>= 1) {
     double ob = __shfl_down(best, o);
     int oi = __shfl_down(idx, o);
@@ -86,13 +82,38 @@ __global__ void maxabs_kernel(const double* __restrict__ x, size_t n, double* ou
   }
   if ((threadIdx.x & 63) == 0) { bv[threadIdx.x >> 6] = best; bi[threadIdx.x >> 6] = idx; }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double b = bv[0];
-    int ii = bi[0];
+  if (threadIdx.x == 0)
     for (int w = 1; w < (int)(blockDim.x >> 6); ++w)
-      if (bv[w] > b || (bv[w] == b && bi[w] < ii)) { b = bv[w]; ii = bi[w]; }
-    *out_val = b;
-    *out_idx = ii;
+      if (bv[w] > best || (bv[w] == best && bi[w] < idx)) { best = bv[w]; idx = bi[w]; }
+}
+
+constexpr int MAXABS_PARTS = 256;
+__global__ __launch_bounds__(1024) void maxabs_part_kernel(const double* __restrict__ x, size_t n, double* __restrict__ val,
+                                                           int* __restrict__ at) {
+  double best = -1.0;
+  int idx = 0x7fffffff;
+  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x) {
+    double v = fabs(x[e]);
+    if (v > best) { best = v; idx = (int)e; }
+  }
+  maxabs_block(best, idx);
+  if (threadIdx.x == 0) {
+    val[blockIdx.x] = best;
+    at[blockIdx.x] = idx;
+  }
+}
+
+__global__ __launch_bounds__(MAXABS_PARTS) void maxabs_kernel(const double* __restrict__ x, const double* __restrict__ val,
+                                                              const int* __restrict__ at, int parts,
+                                                              double* __restrict__ out) {
+  const int t = threadIdx.x;
+  double best = t < parts ? val[t] : -1.0;
+  int idx = t < parts ? at[t] : 0x7fffffff;
+  maxabs_block(best, idx);
+  if (t == 0) {
+    out[0] = best;
+    out[1] = (double)idx;
+    out[2] = best >= 0.0 ? x[idx] : 0.0;   // (no entry when every one is a NaN)
   }
 }
 
@@ -487,7 +508,7 @@ void trg_run(Ctx* c, const double* a_host, int q, int chi, int niter, double tol
   copy_in(c, a.ptr, a_host, (size_t)q * q * q * q * 8);
   std::vector<std::unique_ptr<TrgIter>> tape;
   double lnz = 0.0;
-  DevBuf mv(c, 16), mi(c, 16);
+  DevBuf mv(c, (MAXABS_PARTS + 3) * 8), mi(c, MAXABS_PARTS * sizeof(int));   // parts, then {max, index, entry}
   // the splits of one size are alike from one iteration to the next, and the two of an iteration too
   EigPlan plan;
   size_t plan_size = 0;
@@ -496,25 +517,27 @@ void trg_run(Ctx* c, const double* a_host, int q, int chi, int niter, double tol
     std::unique_ptr<TrgIter> T(new TrgIter());
     T->du = du; T->dr = dr;
     // maxval = maximum(abs.(a)); a /= maxval; lnZ += 2^(1-n) log(maxval)     (src/trg.jl:16-18)
-    hipLaunchKernelGGL(maxabs_kernel, dim3(1), dim3(1024), 0, s, a.as<double>(), na, mv.as<double>(), mi.as<int>());
+    const int parts = (int)std::min<size_t>(MAXABS_PARTS, (na + 1023) / 1024);
+    hipLaunchKernelGGL(maxabs_part_kernel, dim3(parts), dim3(1024), 0, s, a.as<double>(), na, mv.as<double>(), mi.as<int>());
+    hipLaunchKernelGGL(maxabs_kernel, dim3(1), dim3(MAXABS_PARTS), 0, s, a.as<double>(), mv.as<double>(), mi.as<int>(), parts,
+                       mv.as<double>() + MAXABS_PARTS);
     TNAD_HIP_TRY(hipGetLastError());
-    double hv = 0.0;
-    int hi = 0;
-    c->read_async(&hv, mv.ptr, 8);
-    c->read_async(&hi, mi.ptr, sizeof(int));
+    double top[3] = {0.0, 0.0, 0.0};
+    c->read_async(top, mv.as<double>() + MAXABS_PARTS, sizeof top);
     c->sync();
+    const double hv = top[0];
     if (!(hv > 0.0)) throw Error(TNAD_ERR_NAN, "trg: tensor vanished or is not finite");
-    if (grad) {
-      T->a_in = DevBuf(c, na * 8);
-      k_copy(a.as<double>(), T->a_in.as<double>(), na, s);
-      double v = 0.0;
-      c->read_async(&v, a.as<double>() + hi, 8);
-      c->sync();
-      T->sgn = v < 0 ? -1.0 : 1.0;
-    }
     T->maxval = hv;
-    T->idx = hi;
-    k_axpby(1.0 / hv, a.as<double>(), 0.0, a.as<double>(), na, s);
+    T->idx = (int)top[1];
+    T->sgn = top[2] < 0 ? -1.0 : 1.0;
+    if (grad) {   // the tape keeps the tensor as it came
+      DevBuf scaled(c, na * 8);
+      k_axpby(1.0 / hv, a.as<double>(), 0.0, scaled.as<double>(), na, s);
+      T->a_in = std::move(a);
+      a = std::move(scaled);
+    } else {
+      k_axpby(1.0 / hv, a.as<double>(), 0.0, a.as<double>(), na, s);
+    }
     lnz += std::pow(2.0, 1 - it) * std::log(hv);
     // dr_ul = ein"urdl -> drul"(a) ; ld_ru = ein"urdl -> ldru"(a)       (src/trg.jl:20-21)
     DevBuf p1(c, na * 8), p2(c, na * 8);
