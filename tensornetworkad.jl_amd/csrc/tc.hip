@@ -11,8 +11,9 @@
 // Tiling: 64x64 output tile per 256-thread workgroup (4 waves in 2x2), each
 // wave owns a 32x32 sub-tile made of 2x2 MFMA 16x16 blocks.  Operands are
 // staged through LDS with a register prefetch of the next K-tile.
-// Split-K: a contraction with few output tiles and a long K (the Gram and
-// projection products of the eigensolver, the bulk cotangent of the adjoint)
+// FP64 with few output tiles (most of the eigensolver's and the adjoint's
+// products): tc_slab_kernel, K split over the waves of a workgroup.
+// Split-K along the grid: what remains with few output tiles and a long K
 // would leave most of the 256 CUs idle, so tc_launch cuts K into slices along
 // grid z; every slice writes its partial tile to a workspace and a second
 // kernel sums the slices in a fixed order (deterministic) and applies
@@ -51,7 +52,7 @@ constexpr int BM = 64, BN = 64, NT = 256;
 // grids of fewer than 256 workgroups, which wait on global-load latency once per K-tile
 constexpr int TC_BK = 16, TC_BK_DEEP = 32, TC_DEEP_BELOW = 256;
 constexpr int TC_BIG_MIN_WG = 1024;  // 128 x 128 tiles only at 4+ workgroups per CU (slower at 1 per CU)
-constexpr int TC_SMALL_BELOW = 128;  // 32 x 32 tiles below this many 64 x 64 workgroups
+constexpr int TC_SMALL_BELOW = 128;  // FP32: 32 x 32 tiles below this many 64 x 64 workgroups
 
 __device__ __forceinline__ int fdiv(int x, const FDiv& f) { return (int)((__umulhi((unsigned)x, f.mul) + (unsigned)x) >> f.sh); }
 
@@ -289,7 +290,7 @@ __global__ __launch_bounds__(NT, PF == 2 ? (sizeof(T) == 8 ? 3 : 4) : 1) void tc
 // index has unit stride, else k), so a thread issues V times fewer loads and no per-element address
 // arithmetic; the K-tile never straddles a K0 run (K0 a multiple of BK, or a single K sub-index) and K
 // is a multiple of BK, so the K loop carries no bounds tests.  TILE x TILE output tile (64, K-tile 16;
-// or 32, K-tile 32, for grids too small to fill the chip with 64 x 64 tiles), 4 waves in 2 x 2,
+// or, in FP32, 32, K-tile 32, for grids too small to fill the chip with 64 x 64 tiles), 4 waves in 2 x 2,
 // double-buffered LDS (one barrier per K-tile), the next K-tile's vectors in flight in registers while
 // the current one is multiplied.
 // ---------------------------------------------------------------------------
