@@ -49,6 +49,11 @@ __global__ void coldot_kernel(const double* __restrict__ X, const double* __rest
   }
 }
 
+// out = a - b
+__global__ void sub_kernel(const double* __restrict__ a, const double* __restrict__ b, size_t n, double* __restrict__ out) {
+  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x) out[e] = a[e] - b[e];
+}
+
 // isig_j = 1 / sig_j, or 0 for a kept value at the rounding level of the largest
 // (sig_j <= 1e-28 sig_0, i.e. s_j <= 1e-14 s_0): such a column has no resolvable
 // complement (the reference's Lorentzian gives F = 0 between equal zeros) and is skipped.
@@ -227,11 +232,10 @@ int resolvent_pcg(Ctx* c, int rows, int r, int k, const double* W, const double*
   precond(bb.as<double>(), x, 0, r);                    // x0 = M^-1 P b
   coldot(bb.as<double>(), x, bz);                       // b.M^-1 b (stopping scale)
   op(x, q.as<double>(), 0, r);
-  k_copy(bb.as<double>(), res.as<double>(), nb_, s);
-  k_axpby(-1.0, q.as<double>(), 1.0, res.as<double>(), nb_, s);   // r0 = P b - A x0
-  precond(res.as<double>(), z.as<double>(), 0, r);
-  k_copy(z.as<double>(), p.as<double>(), nb_, s);
-  coldot(res.as<double>(), z.as<double>(), rz);
+  hipLaunchKernelGGL(sub_kernel, dim3(nb(nb_)), dim3(NT), 0, s, bb.as<double>(), q.as<double>(), nb_, res.as<double>());
+  TNAD_HIP_TRY(hipGetLastError());                      // r0 = P b - A x0
+  precond(res.as<double>(), p.as<double>(), 0, r);
+  coldot(res.as<double>(), p.as<double>(), rz);
 
   // Columns start active; a column stops when r.M^-1 r <= max(tol^2 b.M^-1 b, 1e-30 |b_full|^2 / sig)
   // (the second term measures against the whole right-hand side, so a complement part at the rounding

@@ -236,13 +236,6 @@ __global__ void unsplit_kernel(const double* __restrict__ W, int m, int mp, int 
   }
 }
 
-// X[:, j] *= s[j]
-__global__ void scale_cols_by_kernel(double* __restrict__ X, int rows, int cols, const double* __restrict__ sv) {
-  size_t tot = (size_t)rows * cols;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < tot; e += (size_t)gridDim.x * blockDim.x)
-    X[e] *= sv[e / rows];
-}
-
 // R (K x K) of svd_back (src/trg.jl:72-106) restricted to the K computed singular triplets,
 // cotangents dU, dV on the first kk columns (gu = U^T dU, gv = V^T dV, K x kk), dS on kk:
 //   i,j < kk : (F_ij gu_ij + F_ji gu_ji) s_j + s_i (F_ij gv_ij + F_ji gv_ji) + delta_ij dS_j
@@ -331,16 +324,16 @@ struct SvdTape {
 };
 
 // singular triplets of M from the top eigenpairs of [[0, M], [M^T, 0]]
-static void svd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, int dmax, double tol, double* u_out,
+// (t: the m x mp matrix, taken over by the tape)
+static void svd_split(Ctx* c, DevBuf&& t, int d1, int d2, int d3, int d4, int dmax, double tol, double* u_out,
                       double* v_out, SvdTape& tp, EigPlan* plan = nullptr) {
   hipStream_t s = c->stream;
   const int m = d1 * d2, mp = d3 * d4, N = m + mp;
   const int len = std::min(m, mp);
   tp.d1 = d1; tp.d2 = d2; tp.d3 = d3; tp.d4 = d4; tp.m = m; tp.mp = mp; tp.N = N;
-  tp.M = DevBuf(c, (size_t)m * mp * 8);
-  k_copy(t, tp.M.as<double>(), (size_t)m * mp, s);
+  tp.M = std::move(t);
   DevBuf B(c, (size_t)N * N * 8);
-  hipLaunchKernelGGL(augment_kernel, dim3(nb((size_t)N * N)), dim3(NT), 0, s, t, m, mp, B.as<double>());
+  hipLaunchKernelGGL(augment_kernel, dim3(nb((size_t)N * N)), dim3(NT), 0, s, tp.M.as<double>(), m, mp, B.as<double>());
   TNAD_HIP_TRY(hipGetLastError());
   const int want = std::min(N, 2 * std::min(dmax, len) + 2);
   int keig = (N <= JACOBI_MAX) ? N : std::min(JACOBI_MAX, std::max(want + 24, 2 * want));
@@ -372,7 +365,7 @@ static void svd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, i
   tp.sq = DevBuf(c, (size_t)std::max(k, Kc) * 8);
   tp.U = DevBuf(c, (size_t)m * Kc * 8);
   tp.V = DevBuf(c, (size_t)mp * Kc * 8);
-  k_fill(tp.sq.as<double>(), (size_t)std::max(k, Kc), 0.0, s);
+  if (K < std::max(k, Kc)) k_fill(tp.sq.as<double>(), (size_t)std::max(k, Kc), 0.0, s);
   if (K > 0) {
     c->write_async(cols.ptr, pos.data(), (size_t)K * sizeof(int));
     hipLaunchKernelGGL(split_vectors_kernel, dim3(K), dim3(NT), 0, s, X.as<double>(), theta.as<double>(), N, m,
@@ -397,15 +390,16 @@ static void svd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, i
     }
   }
   // u = U[:, 1:k] sqrt(s), v = sqrt(s) V[:, 1:k]^T; columns j >= K are zero
-  k_fill(u_out, (size_t)m * k, 0.0, s);
-  k_fill(v_out, (size_t)k * mp, 0.0, s);
   const int kv = std::min(k, K);
+  if (kv < k) {
+    k_fill(u_out, (size_t)m * k, 0.0, s);
+    k_fill(v_out, (size_t)k * mp, 0.0, s);
+  }
   if (kv > 0) {
     hipLaunchKernelGGL(scale_split_kernel, dim3(nb((size_t)(m + mp) * kv)), dim3(NT), 0, s, tp.U.as<double>(),
                        tp.V.as<double>(), tp.sq.as<double>(), m, mp, kv, u_out, v_out, k);
     TNAD_HIP_TRY(hipGetLastError());
   }
-  c->sync();
 }
 
 // svd_back (src/trg.jl:72-106) for u = U sqrt(s), v = sqrt(s) V^T: cotangents of u (m x k) and
@@ -421,8 +415,10 @@ static void svd_split_back(Ctx* c, const SvdTape& tp, const double* ubar, const 
   hipStream_t s = c->stream;
   const int m = tp.m, mp = tp.mp, k = tp.k, K = tp.K;
   const int kk = std::min(k, K);            // kept columns carrying a resolved singular triplet
-  k_fill(tbar, (size_t)m * mp, 0.0, s);
-  if (kk == 0) return;
+  if (kk == 0) {
+    k_fill(tbar, (size_t)m * mp, 0.0, s);
+    return;
+  }
   const double* U = tp.U.as<double>();
   const double* V = tp.V.as<double>();
   // dU = ubar sqrt(s), dV = vbar^T sqrt(s), dS = (ubar . U + vbar . V) / (2 sqrt(s))
@@ -454,10 +450,7 @@ static void svd_split_back(Ctx* c, const SvdTape& tp, const double* ubar, const 
   if (m > kk) {
     // left: b = s dU + M dV ; G = M M^T
     DevBuf bl(c, (size_t)m * kk * 8), X(c, (size_t)m * kk * 8);
-    k_copy(dU.as<double>(), bl.as<double>(), (size_t)m * kk, s);
-    hipLaunchKernelGGL(scale_cols_by_kernel, dim3(nb((size_t)m * kk)), dim3(NT), 0, s, bl.as<double>(), m, kk,
-                       tp.sv.as<double>());
-    TNAD_HIP_TRY(hipGetLastError());
+    k_scale_cols_to(dU.as<double>(), m, kk, tp.sv.as<double>(), bl.as<double>(), s);
     tc_launch(c, Prec::F64, gemm_desc('N', 'N', m, kk, mp, m, mp, m, 1.0, 1.0), M, dV.as<double>(), bl.as<double>(), s);
     auto applyMMt = [&](const double* Vb, double* out, int nc) {
       tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp, nc, m, m, m, mp), M, Vb, T1.as<double>(), s);
@@ -470,10 +463,7 @@ static void svd_split_back(Ctx* c, const SvdTape& tp, const double* ubar, const 
   if (mp > kk) {
     // right: b' = M^T dU + s dV ; G = M^T M
     DevBuf br(c, (size_t)mp * kk * 8), Y(c, (size_t)mp * kk * 8);
-    k_copy(dV.as<double>(), br.as<double>(), (size_t)mp * kk, s);
-    hipLaunchKernelGGL(scale_cols_by_kernel, dim3(nb((size_t)mp * kk)), dim3(NT), 0, s, br.as<double>(), mp, kk,
-                       tp.sv.as<double>());
-    TNAD_HIP_TRY(hipGetLastError());
+    k_scale_cols_to(dV.as<double>(), mp, kk, tp.sv.as<double>(), br.as<double>(), s);
     tc_launch(c, Prec::F64, gemm_desc('T', 'N', mp, kk, m, m, m, mp, 1.0, 1.0), M, dU.as<double>(), br.as<double>(), s);
     auto applyMtM = [&](const double* Vb, double* out, int nc) {
       tc_launch(c, Prec::F64, gemm_desc('N', 'N', m, nc, mp, m, mp, m), M, Vb, T1.as<double>(), s);
@@ -554,8 +544,8 @@ void trg_run(Ctx* c, const double* a_host, int q, int chi, int niter, double tol
     T->ru_t = DevBuf(c, (size_t)kmax2 * dr * du * 8 + 8);
     if (plan_size != na) plan = EigPlan{};
     plan_size = na;
-    svd_split(c, p1.as<double>(), du, dr, du, dr, chi, tol, T->dr_t.as<double>(), T->ul_t.as<double>(), T->s1, &plan);
-    svd_split(c, p2.as<double>(), dr, du, dr, du, chi, tol, T->ld_t.as<double>(), T->ru_t.as<double>(), T->s2, &plan);
+    svd_split(c, std::move(p1), du, dr, du, dr, chi, tol, T->dr_t.as<double>(), T->ul_t.as<double>(), T->s1, &plan);
+    svd_split(c, std::move(p2), dr, du, dr, du, chi, tol, T->ld_t.as<double>(), T->ru_t.as<double>(), T->s2, &plan);
     const int k1 = T->s1.k, k2 = T->s2.k;
     T->k1 = k1; T->k2 = k2;
     // a = ein"npu,por,dom,lmn -> urdl"(dr, ld, ul, ru)                   (src/trg.jl:25)
@@ -659,7 +649,7 @@ void trg_svd_run(Ctx* c, const double* t, int d1, int d2, int d3, int d4, int dm
   DevBuf bt(c, (size_t)m * mp * 8), bu(c, (size_t)m * kmax * 8 + 8), bv(c, (size_t)kmax * mp * 8 + 8);
   copy_in(c, bt.ptr, t, (size_t)m * mp * 8);
   SvdTape tp;
-  svd_split(c, bt.as<double>(), d1, d2, d3, d4, dmax, tol, bu.as<double>(), bv.as<double>(), tp);
+  svd_split(c, std::move(bt), d1, d2, d3, d4, dmax, tol, bu.as<double>(), bv.as<double>(), tp);
   const int k = tp.k;
   // outputs are written with the caller's capacity kmax: u (m x kmax), v (kmax x mp)
   std::vector<double> hu((size_t)m * k), hv((size_t)k * mp);
@@ -688,7 +678,7 @@ void trg_svd_back_run(Ctx* c, const double* t, int d1, int d2, int d3, int d4, i
   DevBuf bt(c, (size_t)m * mp * 8), bu(c, (size_t)m * kmax * 8 + 8), bv(c, (size_t)kmax * mp * 8 + 8);
   copy_in(c, bt.ptr, t, (size_t)m * mp * 8);
   SvdTape tp;
-  svd_split(c, bt.as<double>(), d1, d2, d3, d4, dmax, tol, bu.as<double>(), bv.as<double>(), tp);
+  svd_split(c, std::move(bt), d1, d2, d3, d4, dmax, tol, bu.as<double>(), bv.as<double>(), tp);
   if (tp.k != k) throw Error(TNAD_ERR_SHAPE, "trg_svd_back: k is not the forward's kept count");
   DevBuf bub(c, (size_t)m * k * 8), bvb(c, (size_t)k * mp * 8), btb(c, (size_t)m * mp * 8);
   copy_in(c, bub.ptr, ubar, (size_t)m * k * 8);
