@@ -594,7 +594,7 @@ __global__ __launch_bounds__(64 * CH_W) void chol_inv_kernel(const double* __res
   }
   __syncthreads();
 #pragma unroll
-  for (int s = 0; s < CH_S; ++s)
+  for (int s = 0; s < CH_S; ++s) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int row = CH_B * pk[s] + q + 4 * k, col = CH_B * (pi[s] < 0 ? 0 : pi[s]) + r;
@@ -602,6 +602,8 @@ __global__ __launch_bounds__(64 * CH_W) void chol_inv_kernel(const double* __res
       acc[s][k] = (row < m && col < m) ? (acc[s][k] * sh.sc[row] * sh.sc[col] + (row == col ? shift : 0.0))
                                        : (row == col ? 1e300 : 0.0);
     }
+    if (!pairs) break;   // as in the loads: the other slots of these wavefronts hold no pair
+  }
 
   if (wave == 0) {
     double pmin = HUGE_VAL;
