@@ -132,7 +132,7 @@ __global__ void canon_sign_kernel(double* __restrict__ X, double* __restrict__ Y
     int ii = bi[0];
     for (int w = 1; w < 4; ++w)
       if (bv[w] > b || (bv[w] == b && bi[w] < ii)) { b = bv[w]; ii = bi[w]; }
-    sgn = X[ii + (long long)j * n] < 0 ? -1.0 : 1.0;
+    sgn = ii < n && X[ii + (long long)j * n] < 0 ? -1.0 : 1.0;   // (no such entry in a column of NaNs)
   }
   __syncthreads();
   if (sgn < 0) {
@@ -519,12 +519,16 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
     const bool exact = flag != 0;   // the exact solver ran (forced, or the selective Rayleigh-Ritz declined)
     n_exact += exact;
     double mx = 0.0;
-    for (int j = 0; j < want; ++j) mx = std::max(mx, hres[j]);
+    bool nan = false;   // (the maximum passes over a NaN)
+    for (int j = 0; j < want; ++j) {
+      mx = std::max(mx, hres[j]);
+      nan |= hres[j] != hres[j];
+    }
     rel = mx / std::max(std::fabs(hth[0]), 1e-300);
     if (dbg)
       std::fprintf(stderr, "[tnad eig] n=%d k=%d want=%d it=%d rel_resid=%.3e theta0=%.6e rr=%s(%d)\n", n, k, want,
                    it, rel, hth[0], exact ? "exact" : "select", exact_forced ? -1 : flag);
-    if (!(rel == rel)) throw Error(TNAD_ERR_NAN, "eigensolver: NaN in Ritz residual");
+    if (nan || !(rel == rel)) throw Error(TNAD_ERR_NAN, "eigensolver: NaN in Ritz residual");
     // residual ratio per product: observed between two Rayleigh-Ritz steps, else the guard's edge over the
     // last kept value
     rate = std::fabs(hth[k - 1]) / std::max(std::fabs(hth[want - 1]), 1e-300);

@@ -1,0 +1,28 @@
+"""Inputs that are not numbers end in an error, in the kernels that look for a largest entry too: a column or a tensor of
+NaNs has none."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("where", ["entry", "row", "all", "inf"])
+@pytest.mark.parametrize("n,want,k", [(200, 8, 16), (333, 37, 83)])
+def test_symeig_truncated_nonfinite(ctx, n, want, k, where):
+    import tnad
+    print(f"case: symeig truncated {where} n={n} want={want} k={k}", flush=True)
+    A = np.random.default_rng(n).standard_normal((n, n))
+    A = np.asfortranarray(A + A.T)
+    if where == "entry":
+        A[5, 5] = np.nan
+    elif where == "row":
+        A[5, :] = A[:, 5] = np.nan
+    else:
+        A[:] = np.nan if where == "all" else np.inf
+    ev, X, got = np.zeros(k), np.zeros((n, k), order="F"), C.c_int(0)
+    with pytest.raises(tnad.TnadError) as e:
+        ctx.check(ctx.lib.tnad_symeig(ctx.h, C.c_void_p(A.ctypes.data), n, want, k, C.c_void_p(ev.ctypes.data),
+                                      C.c_void_p(X.ctypes.data), C.byref(got)))
+    assert "NaN" in str(e.value)
