@@ -80,9 +80,9 @@ __global__ void zmaxabs_kernel(const double* __restrict__ x, size_t n, double* o
     int ii = bi[0];
     for (int w = 1; w < (int)(blockDim.x >> 6); ++w)
       if (bv[w] > b || (bv[w] == b && bi[w] < ii)) { b = bv[w]; ii = bi[w]; }
-    out_val[0] = sqrt(b);
-    out_val[1] = x[ii];
-    out_val[2] = x[n + ii];
+    out_val[0] = sqrt(b);   // (NaN when every entry is one: no entry to look at)
+    out_val[1] = b >= 0.0 ? x[ii] : 0.0;
+    out_val[2] = b >= 0.0 ? x[n + ii] : 0.0;
     *out_idx = ii;
   }
 }

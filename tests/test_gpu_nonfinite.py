@@ -26,3 +26,16 @@ def test_symeig_truncated_nonfinite(ctx, n, want, k, where):
         ctx.check(ctx.lib.tnad_symeig(ctx.h, C.c_void_p(A.ctypes.data), n, want, k, C.c_void_p(ev.ctypes.data),
                                       C.c_void_p(X.ctypes.data), C.byref(got)))
     assert "NaN" in str(e.value)
+
+
+@pytest.mark.parametrize("where", ["entry", "all"])
+@pytest.mark.parametrize("dtype", [float, complex])
+def test_trg_nan(ctx, dtype, where):
+    import tnad
+    print(f"case: trg {dtype.__name__} {where}", flush=True)
+    a = np.ones((2, 2, 2, 2), dtype=dtype)
+    a[0, 1, 0, 1] = np.nan
+    if where == "all":
+        a[:] = np.nan
+    with pytest.raises(tnad.TnadError):
+        tnad.trg_and_grad(a, 4, 3, ctx=ctx)
