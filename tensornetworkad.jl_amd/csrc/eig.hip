@@ -14,6 +14,8 @@
 //    triangular inverse, register-resident, for CholeskyQR orthonormalisation.
 #include "tnad_internal.h"
 
+#include <cfloat>
+
 namespace tnad {
 namespace {
 
@@ -435,13 +437,14 @@ __global__ __launch_bounds__(JS_NT) void jacobi_sort_kernel(const double* __rest
   __shared__ int cnt_w[JS_NT / 64], row_w[JS_NT / 64];
   __shared__ double best_w[JS_NT / 64];
   const int i = blockIdx.x, t = threadIdx.x;
-  const double li = diag[i], ai = fabs(li);
+  // (a NaN counts as the largest value, so the ranks are a permutation and every pair is written whatever the input)
+  const double li = diag[i], ai = fmin(fabs(li), DBL_MAX);
   const double* vi = Vu + (long long)i * m;
   int cnt = 0;
   double best = -1.0;
   int brow = m;
   for (int j = t; j < m; j += JS_NT) {
-    const double aj = fabs(diag[j]);
+    const double aj = fmin(fabs(diag[j]), DBL_MAX);
     cnt += (aj > ai) || (aj == ai && j < i);
     const double v = fabs(vi[j]);
     if (v > best) { best = v; brow = j; }

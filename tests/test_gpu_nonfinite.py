@@ -39,3 +39,16 @@ def test_trg_nan(ctx, dtype, where):
         a[:] = np.nan
     with pytest.raises(tnad.TnadError):
         tnad.trg_and_grad(a, 4, 3, ctx=ctx)
+
+
+@pytest.mark.parametrize("n", [1, 8, 97, 192])
+def test_symeig_full_nan(ctx, n):
+    # every eigenpair is written (a NaN has no rank among the values), so nothing of an earlier call shows
+    print(f"case: symeig full NaN n={n}", flush=True)
+    A = np.full((n, n), np.nan, order="F")
+    ev, U, count = np.zeros(n), np.zeros((n, n), order="F"), C.c_int(0)
+    ctx.check(ctx.lib.tnad_symeig(ctx.h, C.c_void_p(A.ctypes.data), n, n, n, C.c_void_p(ev.ctypes.data),
+                                  C.c_void_p(U.ctypes.data), C.byref(count)))
+    assert np.isnan(ev).all()
+    if n > 1:
+        assert np.isnan(U).all()
