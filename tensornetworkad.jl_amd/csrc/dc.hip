@@ -107,7 +107,9 @@ __device__ __forceinline__ void trd_reflect(const double (&c)[3], int j, int m, 
   const double a0 = lane_of(c[0], jr & 63), a1 = lane_of(c[1], jr & 63), a2 = lane_of(c[2], jr & 63);
   const double al = sl == 0 ? a0 : (sl == 1 ? a1 : a2);
   double be = al, tv = 0.0, sc = 0.0;
-  if (sg > 1e-300) {   // below, beta d leaves the range of a double (a rank-one matrix gets there by rounding noise of noise)
+  // below, beta d leaves the range of a double (a rank-one matrix gets there by rounding noise of noise); the largest entry
+  // of the matrix is at least 1 here (trd_kernel), so a column below 1e-150 is nothing beside it
+  if (sg > 1e-300) {
     // refined estimates in place of the square root and the division: they are a chain that every wavefront waits for
     double rs;
     const double nr = sqrt_nr(al * al + sg, rs);
@@ -259,15 +261,17 @@ __device__ __forceinline__ void trd_blocks(double (&A)[RA][RB], int m, TrdShared
   if constexpr (BJ + 1 < RB) trd_blocks<RA, RB, BJ + 1>(A, m, sh, tx, ty, lane, tid, Vh, tauo, eo);
 }
 
-// H (m x m, ld ldh; the upper triangle is read) -> diagonal dout (m), off-diagonal eout (m - 1),
-// reflectors Vh (m x m, column j = v_j) and tauo (m - 2).  RA x RB: elements per thread, the smallest of the
+// H (m x m, ld ldh; the upper triangle is read) -> of H / scale the diagonal dout (m), off-diagonal eout (m - 1),
+// reflectors Vh (m x m, column j = v_j) and tauo (m - 2).  scale: the power of two that brings the largest entry
+// into [1, 2), exact to divide by.  Squares of entries and of gaps are formed here and in the divide and conquer, and
+// without it a matrix of norm 1e-133 lost eigenvectors with values 1e-14 of the largest, one of 1e-150 all of them.  RA x RB: elements per thread, the smallest of the
 // instances in trd_launch that covers m: the padding of a larger one is multiplied and updated like the rest (the
 // values are the same for each).
 template <int RA, int RB>
 __global__ __launch_bounds__(TD_NT) void trd_kernel(const double* __restrict__ H, int ldh, int m,
                                                     double* __restrict__ dout, double* __restrict__ eout,
                                                     double* __restrict__ Vh, double* __restrict__ tauo,
-                                                    const int* __restrict__ gate) {
+                                                    double* __restrict__ scale, const int* __restrict__ gate) {
   if (gate && *gate == 0) return;
   __shared__ TrdShared sh;
   const int tid = threadIdx.x, ty = tid / TD_GX, tx = tid % TD_GX, lane = tid & 63;
@@ -281,6 +285,22 @@ __global__ __launch_bounds__(TD_NT) void trd_kernel(const double* __restrict__ H
       const double x = H[in ? min(r, c) + (size_t)max(r, c) * ldh : 0];   // branch-free, clamped address
       A[a][b] = in ? x : 0.0;
     }
+  double mx = 0.0;
+#pragma unroll
+  for (int a = 0; a < RA; ++a)
+#pragma unroll
+    for (int b = 0; b < RB; ++b) mx = fmax(mx, fabs(A[a][b]));
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
+  if (lane == 0) sh.pp[0][tid >> 6] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < TD_NT / 64; ++w) mx = fmax(mx, sh.pp[0][w]);
+  const int ex = mx > 0.0 && mx <= DBL_MAX ? ilogb(mx) : 0;   // (zero and non-finite matrices as they are)
+  if (tid == 0) *scale = ldexp(1.0, ex);
+#pragma unroll
+  for (int a = 0; a < RA; ++a)
+#pragma unroll
+    for (int b = 0; b < RB; ++b) A[a][b] = ldexp(A[a][b], -ex);
   if (m > 2) {   // the first reflector, from column 0 (published, then formed by wavefront 0)
     if (tx == 0) {
 #pragma unroll
@@ -1248,18 +1268,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 
 // Instances for m up to 48, 96, 144, 192 (us at m = 20 / 48 / 80 / 128 with the last one for all: 48 / 102 / 159 / 229;
 // with these: 24 / 52 / 98 / 189)
-void trd_launch(const double* H, int ldh, int m, double* d, double* e, double* Vh, double* tau, const int* gate,
-                hipStream_t s) {
-  if (m <= 48) hipLaunchKernelGGL((trd_kernel<2, 3>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, gate);
-  else if (m <= 96) hipLaunchKernelGGL((trd_kernel<3, 6>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, gate);
-  else if (m <= 144) hipLaunchKernelGGL((trd_kernel<5, 9>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, gate);
-  else hipLaunchKernelGGL((trd_kernel<6, 12>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, gate);
+void trd_launch(const double* H, int ldh, int m, double* d, double* e, double* Vh, double* tau, double* scale,
+                const int* gate, hipStream_t s) {
+  if (m <= 48) hipLaunchKernelGGL((trd_kernel<2, 3>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, scale, gate);
+  else if (m <= 96) hipLaunchKernelGGL((trd_kernel<3, 6>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, scale, gate);
+  else if (m <= 144) hipLaunchKernelGGL((trd_kernel<5, 9>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, scale, gate);
+  else hipLaunchKernelGGL((trd_kernel<6, 12>), dim3(1), dim3(TD_NT), 0, s, H, ldh, m, d, e, Vh, tau, scale, gate);
   TNAD_HIP_TRY(hipGetLastError());
 }
 
-// the work buffer: Vh, Qa, Qb (m x m each), d, e, tau, lambda (m each), the reflector block products
+// the work buffer: Vh, Qa, Qb (m x m each), d, e, tau, lambda (m each), the reflector block products, the scale
 struct DcWork {
-  double *Vh, *Qa, *Qb, *dv, *ev, *tau, *lam, *gram;
+  double *Vh, *Qa, *Qb, *dv, *ev, *tau, *lam, *gram, *scale;
   DcTop top;
 };
 
@@ -1274,6 +1294,7 @@ DcWork dc_work(double* w, int m) {
   d.tau = d.ev + m;
   d.lam = d.tau + m;
   d.gram = d.lam + m;   // 6 per block of four reflectors, the count padded to 32: at most 1.5 m + 44
+  d.scale = d.gram + 2 * (size_t)m + 47;
   double* t = d.gram + 2 * (size_t)m + 48;   // the top merge: 5 m doubles, rho, then 3 m + 1 ints
   d.top.dK = t;
   d.top.zK = t + m;
@@ -1332,10 +1353,10 @@ void syev_dc(const double* H, int ldh, int m, double* evals, double* V, double* 
              const int* gate) {
   if (m < 1 || m > JACOBI_MAX) throw Error(TNAD_ERR_ARG, "syev_dc: size out of range");
   const DcWork w = dc_work(work, m);
-  trd_launch(H, ldh, m, w.dv, w.ev, w.Vh, w.tau, gate, s);
+  trd_launch(H, ldh, m, w.dv, w.ev, w.Vh, w.tau, w.scale, gate, s);
   dc_solve(w, m, gate, s);
   dc_vectors(w, m, gate, s);
-  sort_eigenpairs(w.lam, w.Qa, m, evals, V, gate, s);
+  sort_eigenpairs(w.lam, w.Qa, m, evals, V, gate, s, w.scale);
 }
 
 void syev_dc_time(const double* H, int m, int reps, double* work, hipStream_t s, float ms[3]) {
@@ -1348,12 +1369,12 @@ void syev_dc_time(const double* H, int m, int reps, double* work, hipStream_t s,
   float acc[3] = {0.f, 0.f, 0.f};
   for (int r = 0; r <= reps; ++r) {   // the first run warms up
     TNAD_HIP_TRY(hipEventRecord(e[0], s));
-    trd_launch(H, m, m, w.dv, w.ev, w.Vh, w.tau, nullptr, s);
+    trd_launch(H, m, m, w.dv, w.ev, w.Vh, w.tau, w.scale, nullptr, s);
     TNAD_HIP_TRY(hipEventRecord(e[1], s));
     dc_solve(w, m, nullptr, s);
     TNAD_HIP_TRY(hipEventRecord(e[2], s));
     dc_vectors(w, m, nullptr, s);
-    sort_eigenpairs(w.lam, w.Qa, m, evals, V, nullptr, s);
+    sort_eigenpairs(w.lam, w.Qa, m, evals, V, nullptr, s, w.scale);
     TNAD_HIP_TRY(hipEventRecord(e[3], s));
     TNAD_HIP_TRY(hipEventSynchronize(e[3]));
     if (r == 0) continue;

@@ -427,12 +427,14 @@ __global__ __launch_bounds__(64 * JA_WAVES) void jacobi_apply_kernel(const doubl
 }
 
 // sort by |lambda| descending (stable), sign convention: largest |component| of each vector positive
-// (the first such component when several tie).  One workgroup per (unsorted) eigenpair.
+// (the first such component when several tie).  One workgroup per (unsorted) eigenpair.  scale (nullable): the
+// eigenvalues' common factor.
 constexpr int JS_NT = 256;
 __global__ __launch_bounds__(JS_NT) void jacobi_sort_kernel(const double* __restrict__ diag,
                                                             const double* __restrict__ Vu, int m,
                                                             double* __restrict__ evals, double* __restrict__ V,
-                                                            const int* __restrict__ gate) {
+                                                            const int* __restrict__ gate,
+                                                            const double* __restrict__ scale) {
   if (gate && *gate == 0) return;
   __shared__ int cnt_w[JS_NT / 64], row_w[JS_NT / 64];
   __shared__ double best_w[JS_NT / 64];
@@ -465,7 +467,7 @@ __global__ __launch_bounds__(JS_NT) void jacobi_sort_kernel(const double* __rest
     if (best_w[w] > bb || (best_w[w] == bb && row_w[w] < br)) { bb = best_w[w]; br = row_w[w]; }
   }
   const double sgn = (br < m && vi[br] < 0) ? -1.0 : 1.0;
-  if (t == 0) evals[rank] = li;
+  if (t == 0) evals[rank] = scale ? li * *scale : li;
   for (int row = t; row < m; row += JS_NT) V[row + (long long)rank * m] = sgn * vi[row];
 }
 
@@ -962,8 +964,8 @@ __global__ __launch_bounds__(EIG_NT) void ritz_select_kernel(const double* __res
 }  // namespace
 
 void sort_eigenpairs(const double* lam, const double* Vu, int m, double* evals, double* V, const int* gate,
-                     hipStream_t s) {
-  hipLaunchKernelGGL(jacobi_sort_kernel, dim3(m), dim3(JS_NT), 0, s, lam, Vu, m, evals, V, gate);
+                     hipStream_t s, const double* scale) {
+  hipLaunchKernelGGL(jacobi_sort_kernel, dim3(m), dim3(JS_NT), 0, s, lam, Vu, m, evals, V, gate, scale);
   TNAD_HIP_TRY(hipGetLastError());
 }
 
@@ -1003,7 +1005,8 @@ void jacobi_eig_ws(const double* H, int ldh, int m, double* evals, double* V, do
   hipLaunchKernelGGL(jacobi_apply_kernel, dim3((m + JA_WAVES - 1) / JA_WAVES), dim3(64 * JA_WAVES), 0, s, rot,
                      rounds, m, Vu, gate);
   TNAD_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(jacobi_sort_kernel, dim3(m), dim3(JS_NT), 0, s, diag, Vu, m, evals, V, gate);
+  hipLaunchKernelGGL(jacobi_sort_kernel, dim3(m), dim3(JS_NT), 0, s, diag, Vu, m, evals, V, gate,
+                     (const double*)nullptr);
   TNAD_HIP_TRY(hipGetLastError());
 }
 

@@ -126,9 +126,9 @@ void syev_dc(const double* H, int ldh, int m, double* evals, double* V, double* 
 // back-transformation and sort.  work: syev_dc_work_doubles(m) + m * m + m doubles.  For roofline measurement.
 void syev_dc_time(const double* H, int m, int reps, double* work, hipStream_t s, float ms[3]);
 // eigenpairs (lam[i], column i of Vu, m x m) sorted by |lambda| descending into evals / V with the sign
-// convention of jacobi_eig_ws; skipped when *gate == 0
+// convention of jacobi_eig_ws, evals times *scale (nullable); skipped when *gate == 0
 void sort_eigenpairs(const double* lam, const double* Vu, int m, double* evals, double* V, const int* gate,
-                     hipStream_t s);
+                     hipStream_t s, const double* scale = nullptr);
 
 // Eigenpairs of a nearly diagonal symmetric m x m H for its first nh columns (pairs among the
 // others are not rotated), sorted by |lambda| descending: pairs with min(i, j) < nh coupled more
