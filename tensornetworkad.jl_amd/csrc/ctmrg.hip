@@ -107,6 +107,15 @@ __global__ void inv_sqrt2_coef_kernel(const double* __restrict__ G, const double
   F[q] = 0.375 * G2[q] - 1.25 * G[q] + (i == j ? 1.875 : 0.0);
 }
 
+// *out = max(*out, max |A_i|), as bits (the order of non-negative doubles is that of their bits; NaNs are passed over)
+__global__ void max_bits_kernel(const double* __restrict__ A, size_t n, unsigned long long* __restrict__ out) {
+  double m = 0.0;
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+    m = fmax(m, fabs(A[i]));
+  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_down(m, o));
+  if ((threadIdx.x & 63) == 0) atomicMax(out, (unsigned long long)__double_as_longlong(m));
+}
+
 // make the largest-|.| entry of every column positive (first occurrence wins);
 // the same sign is applied to the companion block Y (A*X) when given.
 __global__ void canon_sign_kernel(double* __restrict__ X, double* __restrict__ Y, int n) {
@@ -302,7 +311,9 @@ static void dbg_finite(Ctx* c, const char* what, const double* dev, size_t n) {
 // ==========================================================================
 // light: one pass is enough (the block goes through another product and orthonormalisation before a
 // Rayleigh-Ritz step looks at it, so only its span and a deviation well below 1 matter): X^T X is not formed
-static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& w, unsigned seed, bool light = false) {
+// range (nullable): set, and nothing done to Y, when the first pass finds a squared column norm outside 1e-200 .. 1e200
+static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& w, unsigned seed, bool light = false,
+                           bool* range = nullptr) {
   hipStream_t s = c->stream;
   // (the columns' scale is taken out of the Gram matrix by the Cholesky kernel: Y itself is only normalised,
   // with a random refill of null columns, when a pass fails)
@@ -362,6 +373,10 @@ static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& 
     c->sync();
     int info = (int)hs[1];
     const double dev = std::sqrt(hs[2]);
+    if (round == 0 && info == -1 && range) {
+      *range = true;
+      return;
+    }
     if (std::getenv("TNAD_DEBUG_EIG"))
       std::fprintf(stderr, "[tnad eig] plain Cholesky info=%d min pivot=%.3e |X^T X - I|_F=%.3e\n", info, hs[0], dev);
     if (info == 0 && hs[0] > 1e-6 && dev <= 1e-2) {
@@ -428,6 +443,20 @@ static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& 
   // passes alternate X -> Y -> X: the orthonormal block ends in X (Y is scratch)
 }
 
+// the power of two that brings the largest entry of A into [1, 2) when that lies outside 2^-300 .. 2^300, else 1
+static double unit_scale(Ctx* c, const double* A, size_t nn, EigWork& w) {
+  double* top = w.scal.as<double>() + 8;
+  k_fill(top, 1, 0.0, c->stream);
+  hipLaunchKernelGGL(max_bits_kernel, dim3(256), dim3(NT), 0, c->stream, A, nn, reinterpret_cast<unsigned long long*>(top));
+  TNAD_HIP_TRY(hipGetLastError());
+  double mx = 0.0;
+  c->read_async(&mx, top, sizeof(double));
+  c->sync();
+  if (!(mx > 0.0) || !std::isfinite(mx)) return 1.0;
+  const int ex = std::ilogb(mx);
+  return std::abs(ex) > 300 ? std::ldexp(1.0, -std::max(-1020, std::min(ex, 1020))) : 1.0;
+}
+
 EigWork::EigWork(Ctx* c, int n, int k)
     : Y(c, (size_t)n * k * 8), Xr(c, (size_t)n * k * 8), Yr(c, (size_t)n * k * 8), H(c, (size_t)k * k * 8),
       W(c, (size_t)k * k * 8), Vw(c, syev_dc_work_doubles(k) * 8), G(c, (size_t)k * k * 8), Rinv(c, (size_t)k * k * 8),
@@ -452,8 +481,11 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
   EigWork w(c, n, k);
   // starting block: the previous step's Ritz vectors, or a random one (its columns' norms lie within a few per
   // cent of each other, and only its span counts: it needs no orthonormalisation)
-  if (X0) k_copy(X0, X, (size_t)n * k, s);
-  else k_random_matrix(X, (size_t)n * k, 0x1234567u, s);
+  auto start_block = [&] {
+    if (X0) k_copy(X0, X, (size_t)n * k, s);
+    else k_random_matrix(X, (size_t)n * k, 0x1234567u, s);
+  };
+  start_block();
   if (maxit < 2) {   // the Rayleigh-Ritz step comes at once: it needs an orthonormal block
     k_copy(X, w.Y.as<double>(), (size_t)n * k, s);
     orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x9e3779b9u);
@@ -482,11 +514,25 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
   next_rr = std::min(next_rr, std::max(maxit, 1));
   double rel = 0.0, best = HUGE_VAL, best_mark = HUGE_VAL, prev_rel = HUGE_VAL, rate = 0.0;
   bool force_exact = false;
+  // The Gram matrices hold squares, so a matrix far from order one (below 1e-100, above 1e100: the first product's columns
+  // tell) is taken times a power of two, exactly, from there on: Y = scale A X, and theta and A X divided by it at the end.
+  double scale = 1.0;
   while (true) {
-    tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, n, n, n, n), A, X, w.Y.as<double>(), s);   // Y = A X
+    tc_launch(c, Prec::F64, gemm_desc('N', 'N', n, k, n, n, n, n, scale), A, X, w.Y.as<double>(), s);   // Y = A X
     ++it;
     if (it < next_rr) {
-      orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, it + 1 < next_rr);
+      bool range = false;
+      const bool light = it + 1 < next_rr;
+      orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, light, it == 1 && scale == 1.0 ? &range : nullptr);
+      if (range) {
+        scale = unit_scale(c, A, (size_t)n * n, w);
+        if (scale != 1.0) {
+          start_block();
+          it = 0;
+        } else {   // only null columns
+          orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, light);
+        }
+      }
       continue;
     }
     // Rayleigh-Ritz: H = X^T Y ; H = W diag(theta) W^T ; Xr = X W ; Yr = Y W.  One product after the last
@@ -550,7 +596,12 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
   }
   if (plan) { plan->products = it; plan->resid = rel; plan->rate = rate; }
   k_copy(w.Xr.as<double>(), X, (size_t)n * k, s);
-  k_copy(w.Yr.as<double>(), AX, (size_t)n * k, s);
+  if (scale == 1.0) {
+    k_copy(w.Yr.as<double>(), AX, (size_t)n * k, s);
+  } else {
+    k_axpby(1.0 / scale, w.Yr.as<double>(), 0.0, AX, (size_t)n * k, s);
+    k_axpby(1.0 / scale, theta, 0.0, theta, k, s);
+  }
   hipLaunchKernelGGL(canon_sign_kernel, dim3(k), dim3(NT), 0, s, X, AX, n);
   TNAD_HIP_TRY(hipGetLastError());
   if (st) { st->iters = it; st->k = k; st->resid = rel; st->exact = n_exact; }

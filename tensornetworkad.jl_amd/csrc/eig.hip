@@ -500,6 +500,9 @@ constexpr int CH_W = 16;                        // wavefronts
 constexpr int CH_P = 12;                        // of them with pairs (not on SIMD 0)
 constexpr int CH_S = (CH_NB * (CH_NB + 1) / 2 + CH_P - 1) / CH_P;   // pairs per wavefront
 static_assert(CH_NB * CH_B == JACOBI_MAX, "Cholesky tiling");
+// Largest scale factor 1 / sqrt(G_ii) of a unit-diagonal factorisation (and the smallest, inverted): products of two
+// columns 1e-50 below such a norm still are normal numbers
+constexpr double CH_SC = 1e100;
 typedef double chd4 __attribute__((ext_vector_type(4)));
 
 struct CholShared {
@@ -641,11 +644,14 @@ __global__ __launch_bounds__(64 * CH_W) void chol_inv_kernel(const double* __res
     __syncthreads();   // the last row block of B is published
     if (piv)
       for (int i = lane; i < m; i += 64) piv[i] = sh.pv[i];
+    bool off = false;   // a column norm out of range (or zero, or NaN)
+    for (int i = lane; i < m; i += 64) off |= !(sh.sc[i] <= CH_SC && sh.sc[i] * CH_SC >= 1.0);
+    const bool any_off = __ballot(off) != 0;
     if (lane == 0) {
       if (info) *info = bad;
       if (pmin_out) {   // the smallest pivot and the breakdown column, for one host transfer
         pmin_out[0] = pmin;
-        pmin_out[1] = (double)bad;
+        pmin_out[1] = any_off ? -1.0 : (double)bad;
       }
     }
     return;

@@ -143,7 +143,8 @@ void ritz_select(const double* H, int ldh, int m, int nh, double thresh, double*
 // (upper triangular, column-major) so that X = Y * Rinv with Rinv = L^-T.
 // piv (nullable, m doubles) receives the Cholesky pivots diag(L); pmin (nullable, two device doubles) the
 // smallest of them and the first non-positive one's column (1-based, 0: none).  unit: G is scaled to unit
-// diagonal first (before the shift) and Rinv scaled back, so that Y's columns need no normalisation.
+// diagonal first (before the shift) and Rinv scaled back, so that Y's columns need no normalisation; a column
+// number of -1 then says that a diagonal entry of G lies outside 1e-200 .. 1e200.
 void chol_inv(const double* G, int m, double shift, double* Rinv, int* info, double* piv, hipStream_t s,
               double* pmin = nullptr, bool unit = false);
 

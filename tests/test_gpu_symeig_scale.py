@@ -31,3 +31,24 @@ def test_full_spectrum_scales(ctx, n, kind, power):
     evs, Us = _symeig(ctx, np.ldexp(A, power), n, n)
     assert np.array_equal(evs, np.ldexp(ev, power))
     assert np.array_equal(Us, U)
+
+
+@pytest.mark.parametrize("power", [-500, -440, -350, 350, 500])
+@pytest.mark.parametrize("kind", ["graded", "slow"])
+@pytest.mark.parametrize("n,want,k", [(200, 8, 17), (333, 37, 83)])
+def test_truncated_scales(ctx, n, want, k, kind, power):
+    print(f"case: symeig truncated n={n} want={want} k={k} {kind} 2^{power}", flush=True)
+    Q, _ = np.linalg.qr(np.random.default_rng(n).standard_normal((n, n)))
+    i = np.arange(n)
+    A = (Q * (10.0 ** (-9.0 * i / want) if kind == "graded" else 1.0 / (1.0 + i) ** 2)) @ Q.T
+    A = A + A.T
+    ev, X = _symeig(ctx, A, want, k)
+    evs, Xs = _symeig(ctx, np.ldexp(A, power), want, k)
+    assert np.array_equal(evs, np.ldexp(ev, power))
+    assert np.array_equal(Xs, X)
+
+
+def test_truncated_zero(ctx):
+    ev, X = _symeig(ctx, np.zeros((200, 200)), 8, 17)
+    assert np.array_equal(ev, np.zeros(17))
+    assert np.abs(X.T @ X - np.eye(17)).max() < 1e-11
