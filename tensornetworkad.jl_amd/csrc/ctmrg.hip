@@ -594,7 +594,13 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
     TNAD_HIP_TRY(hipGetLastError());
     orthonormalize(c, w.Y.as<double>(), n, k, X, w, 0x51ed2701u + it, it + 1 < next_rr);
   }
-  if (plan) { plan->products = it; plan->resid = rel; plan->rate = rate; }
+  // A solve that ended above tol stopped falling (or hit maxit): the products past its best residual bought nothing, so
+  // the next one looks where this one's residual last halved, and adds none for the tolerance it cannot reach.
+  if (plan) {
+    plan->products = rel <= tol ? it : best_it;
+    plan->resid = rel <= tol ? rel : tol;
+    plan->rate = rate;
+  }
   k_copy(w.Xr.as<double>(), X, (size_t)n * k, s);
   if (scale == 1.0) {
     k_copy(w.Yr.as<double>(), AX, (size_t)n * k, s);
