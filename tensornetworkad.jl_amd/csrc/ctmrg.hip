@@ -587,8 +587,9 @@ int topk_eig(Ctx* c, const double* A, int n, int want, int k, const double* X0, 
     // stagnation at the rounding level: no halving of the best residual in 8 iterations
     if (rel < best) { if (rel < 0.5 * best_mark) { best_mark = rel; best_it = it; } best = rel; }
     if (best < 1e3 * tol && it - best_it >= 8) break;
-    const int ahead = (int)std::ceil(std::log(tol / rel) / std::log(rate));
-    next_rr = std::min(maxit, it + std::max(1, std::min(ahead, 16)));
+    // (bounded before the conversion: the quotient is infinite when tol / rel underflows)
+    const int ahead = (int)std::ceil(std::max(1.0, std::min(std::log(tol / rel) / std::log(rate), 16.0)));
+    next_rr = std::min(maxit, it + ahead);
     hipLaunchKernelGGL(ritz_scale_kernel, dim3(k), dim3(256), 0, s, w.Xr.as<double>(), w.Yr.as<double>(), theta, n,
                        w.Y.as<double>());
     TNAD_HIP_TRY(hipGetLastError());
