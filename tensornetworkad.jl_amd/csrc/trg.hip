@@ -135,11 +135,12 @@ __global__ void augment_kernel(const double* __restrict__ M, int m, int mp, doub
 // to 1e-13 from the subspace iteration, which lengthens u and shortens v by as much.  Normalising the halves separately
 // takes it out, and theta over the product of the halves' norms is the singular value (they are 1/sqrt 2 each without
 // it).  Also writes s_j and sqrt(s_j).  A column whose halves are far from equal (an unconverged guard pair) is only scaled.
+// T: copies of the first nt columns of U, then of V (nt = 0: none).
 __global__ __launch_bounds__(NT) void split_vectors_kernel(const double* __restrict__ X,
                                                                 const double* __restrict__ theta, int N, int m,
                                                                 const int* __restrict__ cols, double* __restrict__ U,
                                                                 double* __restrict__ V, double* __restrict__ sv,
-                                                                double* __restrict__ sq) {
+                                                                double* __restrict__ sq, int nt, double* __restrict__ T) {
   __shared__ double red[2][NT / 64];
   const int j = blockIdx.x, mp = N - m;
   const double* x = X + (size_t)N * cols[j];
@@ -172,8 +173,10 @@ __global__ __launch_bounds__(NT) void split_vectors_kernel(const double* __restr
     s *= 0.5 * fu * fv;
   }
   for (int r = threadIdx.x; r < N; r += NT) {
-    if (r < m) U[r + (size_t)m * j] = fu * x[r];
-    else V[(r - m) + (size_t)mp * j] = fv * x[r];
+    const double y = (r < m ? fu : fv) * x[r];
+    if (r < m) U[r + (size_t)m * j] = y;
+    else V[(r - m) + (size_t)mp * j] = y;
+    if (j < nt) T[r < m ? r + (size_t)m * j : (size_t)m * nt + (r - m) + (size_t)mp * j] = y;
   }
   if (threadIdx.x == 0) {
     sv[j] = s;
@@ -319,9 +322,41 @@ __global__ void svd_cotangent_kernel(const double* __restrict__ ubar, const doub
 struct SvdTape {
   int d1 = 0, d2 = 0, d3 = 0, d4 = 0, m = 0, mp = 0, N = 0, k = 0, K = 0;
   DevBuf M;                    // the m x mp matrix being split
-  DevBuf U, V, sv, sq;         // the K computed singular triplets (U m x K, V mp x K), s and sqrt(s)
+  DevBuf UV, sv, sq;           // the K computed singular triplets (U m x K, then V mp x K), s and sqrt(s)
   std::vector<double> hs;
+  double* U() const { return UV.as<double>(); }
+  double* V() const { return U() + (size_t)m * std::max(K, 1); }
 };
+
+// Small kept values also mix with each other's partners, by eps s_0 / (s_i + s_j): u and v as wholes then lose their
+// orthogonality, which the adjoint relies on.  Newton-Schulz steps X <- X (3 I - X^T X) / 2 bring the kv kept columns of U and
+// V back to it; T holds copies of them.  A step leaves 3/4 of the square of the deviation.
+static void orthonormalize_halves(Ctx* c, const SvdTape& tp, int kv, int steps, double* T) {
+  hipStream_t s = c->stream;
+  const int m = tp.m, mp = tp.mp, nbat = m == mp ? 2 : 1;   // equal halves: one launch for both
+  DevBuf G(c, 2 * (size_t)kv * kv * 8);
+  for (int it = 0; it < steps; ++it)
+    for (int half = 0; half < 3 - nbat; ++half) {
+      double* Q = half ? tp.V() : tp.U();
+      double* Tq = T + (half ? (size_t)m * kv : 0);
+      const int rows = half ? mp : m;
+      if (it > 0) {
+        k_copy(Q, Tq, (size_t)rows * kv, s);
+        if (nbat == 2) k_copy(tp.V(), T + (size_t)m * kv, (size_t)mp * kv, s);
+      }
+      TcDesc g = gemm_desc('T', 'N', kv, kv, rows, rows, rows, kv);
+      g.batch = nbat;
+      g.abat = g.bbat = (long long)m * kv;
+      g.cbat = (long long)kv * kv;
+      tc_launch(c, Prec::F64, g, Tq, Tq, G.as<double>(), s);
+      TcDesc x = gemm_desc('N', 'N', rows, kv, kv, rows, kv, rows, -0.5, 1.5);
+      x.batch = nbat;
+      x.abat = (long long)m * kv;
+      x.bbat = (long long)kv * kv;
+      x.cbat = (long long)m * std::max(tp.K, 1);
+      tc_launch(c, Prec::F64, x, Tq, G.as<double>(), Q, s);
+    }
+}
 
 // singular triplets of M from the top eigenpairs of [[0, M], [M^T, 0]]
 // (t: the m x mp matrix, taken over by the tape)
@@ -363,31 +398,22 @@ static void svd_split(Ctx* c, DevBuf&& t, int d1, int d2, int d3, int d4, int dm
   DevBuf cols(c, (size_t)Kc * sizeof(int) + 16);
   tp.sv = DevBuf(c, (size_t)Kc * 8);
   tp.sq = DevBuf(c, (size_t)std::max(k, Kc) * 8);
-  tp.U = DevBuf(c, (size_t)m * Kc * 8);
-  tp.V = DevBuf(c, (size_t)mp * Kc * 8);
+  tp.UV = DevBuf(c, (size_t)(m + mp) * Kc * 8);
   if (K < std::max(k, Kc)) k_fill(tp.sq.as<double>(), (size_t)std::max(k, Kc), 0.0, s);
   if (K > 0) {
+    // Deviations of U^T U and V^T V measured before the correction (truncated splits of 144 .. 576 rows, full ones of 64): at
+    // most 1e-16 s_0 / s for the smallest kept s.  No step above 1e-2 of s_0 (1e-14), one down to 1e-6 (1e-10), two below.
+    const int kv = std::min(k, K);
+    const double least = tp.hs[kv - 1] / tp.hs[0];
+    const int steps = least < 1e-6 ? 2 : least < 1e-2 ? 1 : 0;
+    DevBuf T;
+    if (steps > 0) T = DevBuf(c, (size_t)(m + mp) * kv * 8);
     c->write_async(cols.ptr, pos.data(), (size_t)K * sizeof(int));
     hipLaunchKernelGGL(split_vectors_kernel, dim3(K), dim3(NT), 0, s, X.as<double>(), theta.as<double>(), N, m,
-                       cols.as<int>(), tp.U.as<double>(), tp.V.as<double>(), tp.sv.as<double>(), tp.sq.as<double>());
+                       cols.as<int>(), tp.U(), tp.V(), tp.sv.as<double>(), tp.sq.as<double>(), steps > 0 ? kv : 0,
+                       T.as<double>());
     TNAD_HIP_TRY(hipGetLastError());
-    // Small kept values also mix with each other's partners, by eps s_0 / (s_i + s_j): u and v as wholes then lose their
-    // orthogonality, which the adjoint relies on.  Two Newton-Schulz steps X <- X (3 I - X^T X) / 2 bring the kept
-    // columns back to it.
-    const int kv = std::min(k, K);
-    if (kv > 0 && tp.hs[kv - 1] < 1e-6 * tp.hs[0]) {
-      DevBuf G(c, (size_t)kv * kv * 8), T(c, (size_t)std::max(m, mp) * kv * 8);
-      for (int half = 0; half < 2; ++half) {
-        double* Q = half ? tp.V.as<double>() : tp.U.as<double>();
-        const int rows = half ? mp : m;
-        for (int it = 0; it < 2; ++it) {
-          tc_launch(c, Prec::F64, gemm_desc('T', 'N', kv, kv, rows, rows, rows, kv), Q, Q, G.as<double>(), s);
-          k_copy(Q, T.as<double>(), (size_t)rows * kv, s);
-          tc_launch(c, Prec::F64, gemm_desc('N', 'N', rows, kv, kv, rows, kv, rows, -0.5, 1.5), T.as<double>(),
-                    G.as<double>(), Q, s);
-        }
-      }
-    }
+    if (steps > 0) orthonormalize_halves(c, tp, kv, steps, T.as<double>());
   }
   // u = U[:, 1:k] sqrt(s), v = sqrt(s) V[:, 1:k]^T; columns j >= K are zero
   const int kv = std::min(k, K);
@@ -396,8 +422,8 @@ static void svd_split(Ctx* c, DevBuf&& t, int d1, int d2, int d3, int d4, int dm
     k_fill(v_out, (size_t)k * mp, 0.0, s);
   }
   if (kv > 0) {
-    hipLaunchKernelGGL(scale_split_kernel, dim3(nb((size_t)(m + mp) * kv)), dim3(NT), 0, s, tp.U.as<double>(),
-                       tp.V.as<double>(), tp.sq.as<double>(), m, mp, kv, u_out, v_out, k);
+    hipLaunchKernelGGL(scale_split_kernel, dim3(nb((size_t)(m + mp) * kv)), dim3(NT), 0, s, tp.U(),
+                       tp.V(), tp.sq.as<double>(), m, mp, kv, u_out, v_out, k);
     TNAD_HIP_TRY(hipGetLastError());
   }
 }
@@ -419,8 +445,8 @@ static void svd_split_back(Ctx* c, const SvdTape& tp, const double* ubar, const 
     k_fill(tbar, (size_t)m * mp, 0.0, s);
     return;
   }
-  const double* U = tp.U.as<double>();
-  const double* V = tp.V.as<double>();
+  const double* U = tp.U();
+  const double* V = tp.V();
   // dU = ubar sqrt(s), dV = vbar^T sqrt(s), dS = (ubar . U + vbar . V) / (2 sqrt(s))
   DevBuf dU(c, (size_t)m * kk * 8), dV(c, (size_t)mp * kk * 8), dS(c, (size_t)kk * 8), Wtmp(c, (size_t)(m + mp) * kk * 8);
   hipLaunchKernelGGL(svd_cotangent_kernel, dim3(kk), dim3(NT), 0, s, ubar, vbar, U, V, tp.sq.as<double>(), m, mp, k,
