@@ -134,8 +134,9 @@ __global__ void augment_kernel(const double* __restrict__ M, int m, int mp, doub
 // cols[j].  A pair carries a part eps s_0 / (2 s) of its (-s, [u; -v]) partner, eps being 1e-16 from the full spectrum and up
 // to 1e-13 from the subspace iteration, which lengthens u and shortens v by as much.  Normalising the halves separately
 // takes it out, and theta over the product of the halves' norms is the singular value (they are 1/sqrt 2 each without
-// it).  Also writes s_j and sqrt(s_j).  A column whose halves are far from equal (an unconverged guard pair) is only scaled.
-// T: copies of the first nt columns of U, then of V (nt = 0: none).
+// it).  Also writes s_j and sqrt(s_j).  A column whose halves are far from equal (a value at the rounding level) is only
+// scaled; no column is lengthened by sqrt 3 or more, which orthonormalize_halves relies on.  T: copies of the first nt
+// columns of U, then of V (nt = 0: none).
 __global__ __launch_bounds__(NT) void split_vectors_kernel(const double* __restrict__ X,
                                                                 const double* __restrict__ theta, int N, int m,
                                                                 const int* __restrict__ cols, double* __restrict__ U,
@@ -167,7 +168,7 @@ __global__ __launch_bounds__(NT) void split_vectors_kernel(const double* __restr
   nu = sqrt(nu);
   nv = sqrt(nv);
   double fu = 1.4142135623730951, fv = 1.4142135623730951, s = theta[cols[j]];
-  if (2.0 * nu * nv > 0.5) {
+  if (2.0 * nu * nv > 0.95) {   // halves of norm 0.586 .. 0.81: factors up to 1.71
     fu = 1.0 / nu;
     fv = 1.0 / nv;
     s *= 0.5 * fu * fv;
@@ -330,7 +331,9 @@ struct SvdTape {
 
 // Small kept values also mix with each other's partners, by eps s_0 / (s_i + s_j): u and v as wholes then lose their
 // orthogonality, which the adjoint relies on.  Newton-Schulz steps X <- X (3 I - X^T X) / 2 bring the kv kept columns of U and
-// V back to it; T holds copies of them.  A step leaves 3/4 of the square of the deviation.
+// V back to it; T holds copies of them.  A step leaves 3/4 of the square of the deviation, and where a
+// singular value of X is far from 1 it still moves it towards 1, as long as it is below sqrt 3: the columns are
+// orthonormal eigenvectors' halves, so that is what the longest factor (split_vectors_kernel) allows.
 static void orthonormalize_halves(Ctx* c, const SvdTape& tp, int kv, int steps, double* T) {
   hipStream_t s = c->stream;
   const int m = tp.m, mp = tp.mp, nbat = m == mp ? 2 : 1;   // equal halves: one launch for both
