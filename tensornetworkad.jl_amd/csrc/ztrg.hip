@@ -284,24 +284,63 @@ __global__ __launch_bounds__(256) void zeig_extract_any_kernel(const double* __r
   if (t == 0) *taken_out = taken_s;
 }
 
-// U[:, j] = sqrt(2) X[0:m, col_j], V[:, j] = sqrt(2) X[m:, col_j]   (X planar N x ldc columns)
-__global__ void zsplit_cols_kernel(const double* __restrict__ X, int N, size_t xplane, int m,
-                                   const int* __restrict__ cols, int K, double* __restrict__ U,
-                                   double* __restrict__ V) {
-  const int mp = N - m;
-  const size_t nU = (size_t)m * K, nV = (size_t)mp * K;
-  const double r2 = 1.4142135623730951;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < (size_t)N * K;
-       e += (size_t)gridDim.x * blockDim.x) {
-    const int r = e % N, j = e / N;
-    const size_t src = r + (size_t)N * cols[j];
-    if (r < m) {
-      U[r + (size_t)m * j] = r2 * X[src];
-      U[nU + r + (size_t)m * j] = r2 * X[xplane + src];
-    } else {
-      V[(r - m) + (size_t)mp * j] = r2 * X[src];
-      V[nV + (r - m) + (size_t)mp * j] = r2 * X[xplane + src];
+// Singular triplets from the complex eigenpairs (lam, [u; v] / sqrt 2) of the augmented matrix (X planar), one workgroup per
+// column cols[j], as split_vectors_kernel of the real path: u and v normalised by themselves, which takes out the part
+// eps s_0 / (2 s) of the (-s, [u; -v]) partner, the singular value lam over the product of their norms; halves far from
+// equal are scaled by sqrt 2, so no factor reaches sqrt 3.  T: copies of the first nt columns of U, then of V.
+__global__ __launch_bounds__(NT) void zsplit_vectors_kernel(const double* __restrict__ X, const double* __restrict__ lam, int N,
+                                                            size_t xplane, int m, const int* __restrict__ cols, int K,
+                                                            double* __restrict__ U, double* __restrict__ V,
+                                                            double* __restrict__ sv, double* __restrict__ sq, int nt,
+                                                            double* __restrict__ T) {
+  __shared__ double red[2][NT / 64];
+  const int j = blockIdx.x, mp = N - m;
+  const size_t nU = (size_t)m * K, nV = (size_t)mp * K, tU = (size_t)m * nt, tV = (size_t)mp * nt;
+  const double *xr = X + (size_t)N * cols[j], *xi = xr + xplane;
+  double a = 0.0, b = 0.0;
+  for (int r = threadIdx.x; r < N; r += NT) {
+    const double v = xr[r] * xr[r] + xi[r] * xi[r];
+    if (r < m) a += v;
+    else b += v;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_down(a, o);
+    b += __shfl_down(b, o);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = a;
+    red[1][threadIdx.x >> 6] = b;
+  }
+  __syncthreads();
+  double nu = 0.0, nv = 0.0;
+  for (int w = 0; w < NT / 64; ++w) {
+    nu += red[0][w];
+    nv += red[1][w];
+  }
+  nu = sqrt(nu);
+  nv = sqrt(nv);
+  double fu = 1.4142135623730951, fv = 1.4142135623730951, s = lam[cols[j]];
+  if (2.0 * nu * nv > 0.95) {
+    fu = 1.0 / nu;
+    fv = 1.0 / nv;
+    s *= 0.5 * fu * fv;
+  }
+  for (int r = threadIdx.x; r < N; r += NT) {
+    const bool top = r < m;
+    const double f = top ? fu : fv, yr = f * xr[r], yi = f * xi[r];
+    const size_t e = top ? r + (size_t)m * j : (r - m) + (size_t)mp * j;
+    double* Q = top ? U : V;
+    Q[e] = yr;
+    Q[(top ? nU : nV) + e] = yi;
+    if (j < nt) {
+      double* t = T + (top ? 0 : 2 * tU);
+      t[e] = yr;
+      t[(top ? tU : tV) + e] = yi;
     }
+  }
+  if (threadIdx.x == 0) {
+    sv[j] = s;
+    sq[j] = sqrt(s);
   }
 }
 
@@ -380,97 +419,14 @@ struct ZSvdTape {
   DevBuf U, V, sv, sq;          // K computed triplets: U planar m x K, V planar mp x K, s, sqrt(s)
 };
 
-static void zsvd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, int dmax, double tol, double* u_out,
-                       double* v_out, ZSvdTape& tp) {
+// The split from the eigenpairs of the augmented matrix (Xc planar with the planes xplane apart, lam, nc of them by |lambda|
+// descending): singular values = the positive eigenvalues above the rounding level.
+static void zsplit_triplets(Ctx* c, const double* Xc, size_t xplane, const double* lam, int nc, int dmax, double tol,
+                            double* u_out, double* v_out, ZSvdTape& tp) {
   hipStream_t s = c->stream;
-  const int m = d1 * d2, mp = d3 * d4, N = m + mp, len = std::min(m, mp);
-  tp.m = m; tp.mp = mp;
-  tp.M = DevBuf(c, 2 * (size_t)m * mp * 8);
-  k_copy(t, tp.M.as<double>(), 2 * (size_t)m * mp, s);
-  DevBuf B(c, 2 * (size_t)N * N * 8);
-  hipLaunchKernelGGL(zaug_kernel, dim3(nb((size_t)N * N)), dim3(NT), 0, s, t, m, mp, B.as<double>());
-  TNAD_HIP_TRY(hipGetLastError());
-  // complex eigenpairs of B by |lambda| descending: Xc (planar N x nc), lam (nc)
-  DevBuf Xc, lam;
-  int nc = 0;
-  if (2 * N <= JACOBI_MAX) {
-    nc = N;
-    Xc = DevBuf(c, 2 * (size_t)N * N * 8);
-    lam = DevBuf(c, (size_t)N * 8);
-    z_heig(c, B.as<double>(), N, Xc.as<double>(), lam.as<double>());
-  } else {
-    const int N2 = 2 * N;
-    const int want_c = std::min(N, 2 * std::min(dmax, len) + 2);
-    int want = std::min(N2, 2 * want_c);
-    int keig = std::min(JACOBI_MAX, std::max(want + 24, 2 * want));
-    keig = std::min(keig, N2);
-    want = std::min(want, keig);
-    DevBuf R(c, (size_t)N2 * N2 * 8), X(c, (size_t)N2 * keig * 8), AX(c, (size_t)N2 * keig * 8),
-        th(c, (size_t)keig * 8), ntk(c, 16);
-    hipLaunchKernelGGL(realify_rect_kernel, dim3(nb((size_t)N * N * 4)), dim3(NT), 0, s, B.as<double>(), N, N,
-                       R.as<double>());
-    TNAD_HIP_TRY(hipGetLastError());
-    keig = topk_eig(c, R.as<double>(), N2, want, keig, nullptr, 300, 1e-13, X.as<double>(), AX.as<double>(),
-                    th.as<double>(), nullptr);
-    const int max_take = std::min(keig, 192);
-    Xc = DevBuf(c, 2 * (size_t)N * max_take * 8);
-    lam = DevBuf(c, (size_t)max_take * 8);
-    const size_t lds = 2 * (size_t)N * 8;
-    if (lds > 64 * 1024) throw Error(TNAD_ERR_UNSUPPORTED, "complex trg: split above 4096 + 4096");
-    hipLaunchKernelGGL(zeig_extract_any_kernel, dim3(1), dim3(256), lds, s, X.as<double>(), th.as<double>(), N, keig,
-                       max_take, Xc.as<double>(), lam.as<double>(), ntk.as<int>());
-    TNAD_HIP_TRY(hipGetLastError());
-    c->read_async(&nc, ntk.ptr, sizeof(int));
-    c->sync();
-    // Xc's imaginary plane sits after N x max_take entries; compact the count to what was taken below
-    if (nc < 1) throw Error(TNAD_ERR_NAN, "complex trg: no eigenvectors");
-    // keep the planar layout of N x max_take (the split kernel takes the plane size)
-    tp.K = 0;
-    std::vector<double> hl(nc);
-    c->read_async(hl.data(), lam.ptr, (size_t)nc * 8);
-    c->sync();
-    const double zero_level = 1e-14 * std::fabs(hl[0]);
-    std::vector<int> pos;
-    std::vector<double> hs;
-    for (int i = 0; i < nc && (int)pos.size() < len; ++i)
-      if (hl[i] > zero_level) { pos.push_back(i); hs.push_back(hl[i]); }
-    const int K = (int)pos.size();
-    int above = 0;
-    for (int i = 0; i < K; ++i) above += hs[i] > tol;
-    const int k = std::min(std::min(above + 1, dmax), len);
-    tp.k = k;
-    tp.K = K;
-    const int Kc = std::max(K, 1);
-    DevBuf cols(c, (size_t)Kc * sizeof(int) + 16);
-    tp.sv = DevBuf(c, (size_t)Kc * 8);
-    tp.sq = DevBuf(c, (size_t)std::max(k, Kc) * 8);
-    tp.U = DevBuf(c, 2 * (size_t)m * Kc * 8);
-    tp.V = DevBuf(c, 2 * (size_t)mp * Kc * 8);
-    std::vector<double> hsq(Kc, 0.0);
-    for (int j = 0; j < K; ++j) hsq[j] = std::sqrt(hs[j]);
-    k_fill(tp.sq.as<double>(), (size_t)std::max(k, Kc), 0.0, s);
-    if (K > 0) {
-      c->write_async(cols.ptr, pos.data(), (size_t)K * sizeof(int));
-      c->write_async(tp.sv.ptr, hs.data(), (size_t)K * 8);
-      c->write_async(tp.sq.ptr, hsq.data(), (size_t)K * 8);
-      hipLaunchKernelGGL(zsplit_cols_kernel, dim3(nb((size_t)N * K)), dim3(NT), 0, s, Xc.as<double>(), N,
-                         (size_t)N * max_take, m, cols.as<int>(), K, tp.U.as<double>(), tp.V.as<double>());
-      TNAD_HIP_TRY(hipGetLastError());
-    }
-    k_fill(u_out, 2 * (size_t)m * k, 0.0, s);
-    k_fill(v_out, 2 * (size_t)k * mp, 0.0, s);
-    const int kv = std::min(k, K);
-    if (kv > 0) {
-      hipLaunchKernelGGL(zscale_split_kernel, dim3(nb((size_t)(m + mp) * kv)), dim3(NT), 0, s, tp.U.as<double>(),
-                         tp.V.as<double>(), tp.sq.as<double>(), m, mp, K, kv, k, u_out, v_out);
-      TNAD_HIP_TRY(hipGetLastError());
-    }
-    c->sync();
-    return;
-  }
-  // full spectrum (N <= 96)
+  const int m = tp.m, mp = tp.mp, N = m + mp, len = std::min(m, mp);
   std::vector<double> hl(nc);
-  c->read_async(hl.data(), lam.ptr, (size_t)nc * 8);
+  c->read_async(hl.data(), lam, (size_t)nc * 8);
   c->sync();
   const double zero_level = 1e-14 * std::fabs(hl[0]);
   std::vector<int> pos;
@@ -483,32 +439,94 @@ static void zsvd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, 
   const int k = std::min(std::min(above + 1, dmax), len);
   tp.k = k;
   tp.K = K;
-  const int Kc = std::max(K, 1);
+  const int Kc = std::max(K, 1), kv = std::min(k, K);
   DevBuf cols(c, (size_t)Kc * sizeof(int) + 16);
   tp.sv = DevBuf(c, (size_t)Kc * 8);
   tp.sq = DevBuf(c, (size_t)std::max(k, Kc) * 8);
   tp.U = DevBuf(c, 2 * (size_t)m * Kc * 8);
   tp.V = DevBuf(c, 2 * (size_t)mp * Kc * 8);
-  std::vector<double> hsq(Kc, 0.0);
-  for (int j = 0; j < K; ++j) hsq[j] = std::sqrt(hs[j]);
   k_fill(tp.sq.as<double>(), (size_t)std::max(k, Kc), 0.0, s);
   if (K > 0) {
+    // Newton-Schulz steps X <- X (3 I - X^H X) / 2 on the kept columns, as many as in the real path (svd_split)
+    const double least = hs[kv - 1] / hs[0];
+    const int steps = least < 1e-6 ? 2 : least < 1e-2 ? 1 : 0;
+    DevBuf T, G;
+    if (steps > 0) {
+      T = DevBuf(c, 2 * (size_t)N * kv * 8);
+      G = DevBuf(c, 2 * (size_t)kv * kv * 8);
+    }
     c->write_async(cols.ptr, pos.data(), (size_t)K * sizeof(int));
-    c->write_async(tp.sv.ptr, hs.data(), (size_t)K * 8);
-    c->write_async(tp.sq.ptr, hsq.data(), (size_t)K * 8);
-    hipLaunchKernelGGL(zsplit_cols_kernel, dim3(nb((size_t)N * K)), dim3(NT), 0, s, Xc.as<double>(), N,
-                       (size_t)N * N, m, cols.as<int>(), K, tp.U.as<double>(), tp.V.as<double>());
+    hipLaunchKernelGGL(zsplit_vectors_kernel, dim3(K), dim3(NT), 0, s, Xc, lam, N, xplane, m, cols.as<int>(), K,
+                       tp.U.as<double>(), tp.V.as<double>(), tp.sv.as<double>(), tp.sq.as<double>(), steps > 0 ? kv : 0,
+                       T.as<double>());
     TNAD_HIP_TRY(hipGetLastError());
+    for (int it = 0; it < steps; ++it)
+      for (int half = 0; half < 2; ++half) {
+        const int rows = half ? mp : m;
+        const size_t nT = (size_t)rows * kv, nQ = (size_t)rows * K, nG = (size_t)kv * kv;
+        double* Q = half ? tp.V.as<double>() : tp.U.as<double>();
+        double* Tq = T.as<double>() + (half ? 2 * (size_t)m * kv : 0);
+        if (it > 0) {
+          k_copy(Q, Tq, nT, s);
+          k_copy(Q + nQ, Tq + nT, nT, s);
+        }
+        const TView vQ = cm("rj", {rows, kv});
+        zein_v(c, cm("ri", {rows, kv}), Tq, nT, true, vQ, Tq, nT, false, cm("ij", {kv, kv}), G.as<double>(), nG);
+        zein_v(c, cm("ri", {rows, kv}), Tq, nT, false, cm("ij", {kv, kv}), G.as<double>(), nG, false, vQ, Q, nQ, -0.5, 1.5);
+      }
   }
   k_fill(u_out, 2 * (size_t)m * k, 0.0, s);
   k_fill(v_out, 2 * (size_t)k * mp, 0.0, s);
-  const int kv = std::min(k, K);
   if (kv > 0) {
     hipLaunchKernelGGL(zscale_split_kernel, dim3(nb((size_t)(m + mp) * kv)), dim3(NT), 0, s, tp.U.as<double>(),
                        tp.V.as<double>(), tp.sq.as<double>(), m, mp, K, kv, k, u_out, v_out);
     TNAD_HIP_TRY(hipGetLastError());
   }
   c->sync();
+}
+
+static void zsvd_split(Ctx* c, const double* t, int d1, int d2, int d3, int d4, int dmax, double tol, double* u_out,
+                       double* v_out, ZSvdTape& tp) {
+  hipStream_t s = c->stream;
+  const int m = d1 * d2, mp = d3 * d4, N = m + mp, len = std::min(m, mp);
+  tp.m = m; tp.mp = mp;
+  tp.M = DevBuf(c, 2 * (size_t)m * mp * 8);
+  k_copy(t, tp.M.as<double>(), 2 * (size_t)m * mp, s);
+  DevBuf B(c, 2 * (size_t)N * N * 8);
+  hipLaunchKernelGGL(zaug_kernel, dim3(nb((size_t)N * N)), dim3(NT), 0, s, t, m, mp, B.as<double>());
+  TNAD_HIP_TRY(hipGetLastError());
+  // complex eigenpairs of B by |lambda| descending: Xc (planar), lam
+  if (2 * N <= JACOBI_MAX) {   // full spectrum (N <= 96)
+    DevBuf Xc(c, 2 * (size_t)N * N * 8), lam(c, (size_t)N * 8);
+    z_heig(c, B.as<double>(), N, Xc.as<double>(), lam.as<double>());
+    zsplit_triplets(c, Xc.as<double>(), (size_t)N * N, lam.as<double>(), N, dmax, tol, u_out, v_out, tp);
+    return;
+  }
+  const int N2 = 2 * N;
+  const int want_c = std::min(N, 2 * std::min(dmax, len) + 2);
+  int want = std::min(N2, 2 * want_c);
+  int keig = std::min(JACOBI_MAX, std::max(want + 24, 2 * want));
+  keig = std::min(keig, N2);
+  want = std::min(want, keig);
+  DevBuf R(c, (size_t)N2 * N2 * 8), X(c, (size_t)N2 * keig * 8), AX(c, (size_t)N2 * keig * 8), th(c, (size_t)keig * 8),
+      ntk(c, 16);
+  hipLaunchKernelGGL(realify_rect_kernel, dim3(nb((size_t)N * N * 4)), dim3(NT), 0, s, B.as<double>(), N, N,
+                     R.as<double>());
+  TNAD_HIP_TRY(hipGetLastError());
+  keig = topk_eig(c, R.as<double>(), N2, want, keig, nullptr, 300, 1e-13, X.as<double>(), AX.as<double>(),
+                  th.as<double>(), nullptr);
+  const int max_take = std::min(keig, 192);
+  DevBuf Xc(c, 2 * (size_t)N * max_take * 8), lam(c, (size_t)max_take * 8);
+  const size_t lds = 2 * (size_t)N * 8;
+  if (lds > 64 * 1024) throw Error(TNAD_ERR_UNSUPPORTED, "complex trg: split above 4096 + 4096");
+  hipLaunchKernelGGL(zeig_extract_any_kernel, dim3(1), dim3(256), lds, s, X.as<double>(), th.as<double>(), N, keig,
+                     max_take, Xc.as<double>(), lam.as<double>(), ntk.as<int>());
+  TNAD_HIP_TRY(hipGetLastError());
+  int nc = 0;
+  c->read_async(&nc, ntk.ptr, sizeof(int));
+  c->sync();
+  if (nc < 1) throw Error(TNAD_ERR_NAN, "complex trg: no eigenvectors");
+  zsplit_triplets(c, Xc.as<double>(), (size_t)N * max_take, lam.as<double>(), nc, dmax, tol, u_out, v_out, tp);
 }
 
 // svd_back (src/trg.jl:72-106) for u = U sqrt(s), v = sqrt(s) V^H: the kept pairs by the reference's complex
