@@ -525,10 +525,8 @@ __device__ __forceinline__ double rsqrt_refined(double d) {
 }
 
 // the value of lane N of each group of 16 lanes, in every lane of the group (DPP row_newbcast; one 64-bit move)
-extern "C" __device__ long tnad_update_dpp_i64(long old, long src, int ctrl, int row_mask, int bank_mask,
-                                               bool bound_ctrl) __asm("llvm.amdgcn.update.dpp.i64");
 template <int N> __device__ __forceinline__ double row_lane(double x) {
-  return __longlong_as_double(tnad_update_dpp_i64(0, __double_as_longlong(x), 0x150 + N, 0xF, 0xF, true));
+  return __builtin_amdgcn_update_dpp(0.0, x, 0x150 + N, 0xF, 0xF, true);
 }
 
 // a[C] -= l l_C for C = C0 .. 15
