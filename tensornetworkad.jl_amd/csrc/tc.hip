@@ -1337,32 +1337,18 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
   }
 }
 
-// The complex kernel up to ZTC_TILES 16 x 16 tiles and ZTC_K of K; four real launches above, where tc_launch has larger tiles
-// and the split along the grid.
-constexpr long long ZTC_TILES = 4096, ZTC_K = 8192;
 void ztc_launch(Ctx* c, const TcDesc& d, const double* A, size_t planeA, bool conjA, const double* B, size_t planeB,
                 bool conjB, double* C, size_t planeC, hipStream_t s) {
   const double sa = conjA ? -1.0 : 1.0, sb = conjB ? -1.0 : 1.0;
   const long long M = (long long)d.M0 * d.M1, N = (long long)d.N0 * d.N1, K = (long long)d.K0 * d.K1;
-  const long long tiles = (M + 15) / 16 * ((N + 15) / 16);
-  const bool empty = M <= 0 || N <= 0 || K <= 0;
-  const size_t ea = empty ? 0 : extent_bytes(d.M0, d.am0, d.M1, d.am1, d.K0, d.ak0, d.K1, d.ak1, 1, 0, 8),
-               eb = empty ? 0 : extent_bytes(d.K0, d.bk0, d.K1, d.bk1, d.N0, d.bn0, d.N1, d.bn1, 1, 0, 8);
-  if (empty || d.batch != 1 || tiles > ZTC_TILES || K > ZTC_K || ea >= (1ull << 32) || eb >= (1ull << 32)) {
-    // (Ar + i sa Ai)(Br + i sb Bi) = (Ar Br - sa sb Ai Bi) + i (sb Ar Bi + sa Ai Br)
-    const double *Ai = A + planeA, *Bi = B + planeB;
-    double* Ci = C + planeC;
-    TcDesc x = d;
-    tc_launch(c, Prec::F64, x, A, B, C, s);
-    x.alpha = d.alpha * sb;
-    tc_launch(c, Prec::F64, x, A, Bi, Ci, s);
-    x.beta = 1.0;
-    x.alpha = -d.alpha * sa * sb;
-    tc_launch(c, Prec::F64, x, Ai, Bi, C, s);
-    x.alpha = d.alpha * sa;
-    tc_launch(c, Prec::F64, x, Ai, B, Ci, s);
-    return;
-  }
+  if (M <= 0 || N <= 0) return;
+  if (K <= 0) throw Error(TNAD_ERR_ARG, "ztc_launch: empty contraction index");
+  if (M > (1LL << 30) || N > 16LL * 65535 || K > (1LL << 30) || d.batch != 1)
+    throw Error(TNAD_ERR_ARG, "ztc_launch: extents out of range");
+  const size_t ea = extent_bytes(d.M0, d.am0, d.M1, d.am1, d.K0, d.ak0, d.K1, d.ak1, 1, 0, 8),
+               eb = extent_bytes(d.K0, d.bk0, d.K1, d.bk1, d.N0, d.bn0, d.N1, d.bn1, 1, 0, 8);
+  // (operands are addressed with 32-bit byte offsets; the complex path's largest, 1024 x 1024, has 8 MB planes)
+  if (ea >= (1ull << 32) || eb >= (1ull << 32)) throw Error(TNAD_ERR_UNSUPPORTED, "ztc_launch: operand of 4 GB or more");
   const size_t ec = extent_bytes(d.M0, d.cm0, d.M1, d.cm1, d.N0, d.cn0, d.N1, d.cn1, 1, 0, 8);
   c->check_range(A, planeA * 8 + ea, "ztc A");
   c->check_range(B, planeB * 8 + eb, "ztc B");

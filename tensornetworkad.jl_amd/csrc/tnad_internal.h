@@ -88,7 +88,7 @@ struct Ctx;
 // blocks before the launch (a size or precision mismatch throws instead of faulting).
 void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, void* C, hipStream_t s);
 // The same on complex FP64 operands in planar form (imaginary plane planeA / planeB / planeC elements after the real
-// one), either operand conjugated: one launch of a complex kernel for small outputs, four real launches above.
+// one), either operand conjugated, in one launch.
 void ztc_launch(Ctx* c, const TcDesc& d, const double* A, size_t planeA, bool conjA, const double* B, size_t planeB,
                 bool conjB, double* C, size_t planeC, hipStream_t s);
 

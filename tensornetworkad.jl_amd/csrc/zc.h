@@ -1,5 +1,5 @@
 // ComplexF64 path (zc.hip): planar complex device buffers (real plane, then imaginary plane), complex
-// contractions as four real strided contractions, the Hermitian eigensolver through the real embedding,
+// contractions, the Hermitian eigensolver through the real embedding,
 // and the complex CTMRG energy with its reverse sweep.
 #pragma once
 #include <map>

@@ -5,12 +5,12 @@
 // the imaginary plane (both column-major).  The C ABI takes and returns Julia's interleaved ComplexF64
 // arrays; the entry points convert at the boundary.
 //
-// Contractions: every complex einsum is four real strided MFMA contractions (tc) on the planes, with
+// Contractions: every complex einsum is one launch (ztc_launch) of four real MFMA products on the planes, with
 // the conjugation of either operand folded into the signs.
 //
 // Hermitian eigenproblems (n <= 96): the real symmetric embedding R = [[Re H, -Im H], [Im H, Re H]]
 // (2n x 2n) has every eigenvalue of H twice, with eigenvectors [Re x; Im x] and [-Im x; Re x] for each
-// eigenvector x of H.  The FP64 Jacobi solver decomposes R; complex vectors are read off its
+// eigenvector x of H.  The FP64 divide and conquer decomposes R; complex vectors are read off its
 // eigenvectors in order of |lambda| with two passes of classical Gram-Schmidt (the partner of each pair
 // is i times a vector already taken and is dropped), then each vector's phase is fixed by the rule
 // below.  The reference's SVD of a complex Hermitian matrix (src/ctmrg.jl:136) leaves these phases to
