@@ -319,9 +319,10 @@ static void orthonormalize(Ctx* c, double* Y, int n, int k, double* X, EigWork& 
   // with a random refill of null columns, when a pass fails)
   // A well-conditioned block takes plain CholeskyQR passes: one when the result is orthonormal to
   // working precision (|X^T X - I|_F <= 1e-12, the usual case once the iteration converges), else a
-  // second: X (X^T X)^{-1/2} to second order when |X^T X - I|_F <= 1e-5, CholeskyQR2 above.  That holds when the
-  // Cholesky pivots of the Gram matrix stay above 1e-6 (unit columns: condition number below u^-1/2) and the
-  // first pass leaves a deviation below 1e-2.  The first pass and the test run before
+  // second: X (X^T X)^{-1/2} to second order when |X^T X - I|_F <= 1e-5, CholeskyQR2 above.  A pass counts when the
+  // Cholesky pivots of the Gram matrix (unit columns) stay above 1e-6, and, unless it is a light one, when it leaves a
+  // deviation below 1e-2: pivots alone bound no condition number, but a light block meets another product and a
+  // measured pass before anything is read off it.  The first pass and the test run before
   // the host looks at the pivots, so that one round trip serves both.  A block that fails (condition
   // number up to ~1e10: the first product with a random block) takes one shifted CholeskyQR pass, which
   // keeps its small directions (to an accuracy of u over their relative size, all that the iteration needs of

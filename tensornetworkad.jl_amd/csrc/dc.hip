@@ -376,14 +376,15 @@ __device__ __forceinline__ int dc_depth(int m) {
   return d;
 }
 
-// sums / products over the L aligned lanes that share a root (butterflies: the same bits in all of them)
+// sums / products over the L aligned lanes that share a root, 8 or the wavefront (butterflies: the same bits in all of
+// them)
 template <int L>
 __device__ __forceinline__ double sumL(double x) {
+  static_assert(L == 8 || L == 64, "8 lanes or all");
   if constexpr (L == 64) return wave_sum(x);
   x += dpp_d<0xB1>(x);
   x += dpp_d<0x4E>(x);
-  if constexpr (L >= 8) x += dpp_d<0x141>(x);
-  if constexpr (L >= 16) x += dpp_d<0x140>(x);
+  x += dpp_d<0x141>(x);
   return x;
 }
 
@@ -396,8 +397,7 @@ __device__ __forceinline__ double prodL(double x) {
   }
   x *= dpp_d<0xB1>(x);
   x *= dpp_d<0x4E>(x);
-  if constexpr (L >= 8) x *= dpp_d<0x141>(x);
-  if constexpr (L >= 16) x *= dpp_d<0x140>(x);
+  x *= dpp_d<0x141>(x);
   return x;
 }
 
@@ -850,7 +850,7 @@ __device__ __forceinline__ void dc_level(DcShared<NM>& sh, const double* __restr
   constexpr int T = NM / L, TH = (T + 1) / 2;
   if (smax <= L) dc_roots<L, 1>(sh, U, LU, m, tid);
   else if (smax <= 2 * L) dc_roots<L, 2>(sh, U, LU, m, tid);
-  else if (T <= 3 || smax <= 3 * L) dc_roots<L, 3>(sh, U, LU, m, tid);
+  else if (smax <= 3 * L) dc_roots<L, 3>(sh, U, LU, m, tid);
   else if (smax <= TH * L) dc_roots<L, TH>(sh, U, LU, m, tid);
   else dc_roots<L, T>(sh, U, LU, m, tid);
   // Qout = Qin[:, kept] U, deflated columns copied: 16 x 16 output tiles on the FP64 matrix cores, one wavefront per
@@ -1313,8 +1313,8 @@ DcWork dc_work(double* w, int m) {
 // blocks of four reflectors that trd_back_kernel reads (m - 2 padded to a multiple of 32)
 int dc_gram_blocks(int m) { return m > 2 ? ((m - 2 + 2 * BK_Q - 1) / (2 * BK_Q)) * (BK_Q / 2) : 0; }
 
-// the divide and conquer: the merge tree below the top merge in one workgroup, the top merge's roots and z
-// over the whole chip
+// the divide and conquer: the merge tree below the top merge in a workgroup per half, the top merge's deflation in one, its
+// roots and z over the whole chip
 void dc_solve(const DcWork& w, int m, const int* gate, hipStream_t s) {
   const int half = (m + 1) / 2;
   if (half <= 48) hipLaunchKernelGGL((dc_kernel<8, 48>), dim3(2), dim3(DC_NT), 0, s, w.dv, w.ev, m, w.Qa, w.Qb, w.lam, gate);
