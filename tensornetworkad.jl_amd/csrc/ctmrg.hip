@@ -84,7 +84,7 @@ __global__ __launch_bounds__(GD_NT) void gram_dev_kernel(const double* __restric
   double acc = 0.0;
   if (i < k)
 #pragma unroll 8
-    for (int j = jo; j < k; j += GD_NT / 256) {   // (eight loads in flight; one at a time took 10 us at k = 128, now 5)
+    for (int j = jo; j < k; j += GD_NT / 256) {   // (eight loads in flight; one at a time 14.6 us on average at k up to 192, now 6.4)
       const double v = G[i + (size_t)k * j] - (i == j ? 1.0 : 0.0);
       acc += v * v;
     }
