@@ -52,7 +52,7 @@ constexpr int BM = 64, BN = 64, NT = 256;
 // grids of fewer than 256 workgroups, which wait on global-load latency once per K-tile
 constexpr int TC_BK = 16, TC_BK_DEEP = 32, TC_DEEP_BELOW = 256;
 constexpr int TC_BIG_MIN_WG = 1024;  // 128 x 128 tiles only at 4+ workgroups per CU (slower at 1 per CU)
-constexpr int TC_SMALL_BELOW = 128;  // FP32: 32 x 32 tiles below this many 64 x 64 workgroups
+constexpr int TC_SMALL_BELOW = 128;  // 32 x 32 tiles below this many 64 x 64 workgroups
 
 __device__ __forceinline__ int fdiv(int x, const FDiv& f) { return (int)((__umulhi((unsigned)x, f.mul) + (unsigned)x) >> f.sh); }
 
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(NT, PF == 2 ? (sizeof(T) == 8 ? 3 : 4) : 1) void tc
 // index has unit stride, else k), so a thread issues V times fewer loads and no per-element address
 // arithmetic; the K-tile never straddles a K0 run (K0 a multiple of BK, or a single K sub-index) and K
 // is a multiple of BK, so the K loop carries no bounds tests.  TILE x TILE output tile (64, K-tile 16;
-// or, in FP32, 32, K-tile 32, for grids too small to fill the chip with 64 x 64 tiles), 4 waves in 2 x 2,
+// or 32, K-tile 32, for grids too small to fill the chip with 64 x 64 tiles), 4 waves in 2 x 2,
 // double-buffered LDS (one barrier per K-tile), the next K-tile's vectors in flight in registers while
 // the current one is multiplied.
 // ---------------------------------------------------------------------------
@@ -1152,6 +1152,32 @@ static int slab_mode(const TcDesc& d, int X0, long long x0, long long k0, bool e
   return even && x0 == 1 && X0 % 2 == 0 ? 1 : 0;
 }
 
+// How well tc_slab_kernel reads an operand: 2 along its rows or along even runs of the first K sub-index, 1 along odd runs
+// (8 bytes at a time), 0 with a line per element
+static int slab_reads(int X0, long long x0, int K0, int K1, long long k0) {
+  if (x0 == 1 && X0 > 1) return 2;
+  return k0 == 1 && K0 > 1 ? (K1 == 1 || K0 % 2 == 0 ? 2 : 1) : 0;
+}
+
+// d with its K sub-indices (their order is that of A's indices) in the order that the kernel reads better: the higher sum of
+// the operands' grades, at equal sums the better one for the larger operand.  2303 x 180 x (50 x 33), A along its rows and B
+// along the second sub-index: 99 us in the given order, 52 in the other; geometric mean of the calls so reordered, over a
+// sweep of random sizes and orders, 0.77.  Below K = 256 the loop is over before the order matters (the transposition
+// through LDS then costs 0.5 us).
+static TcDesc slab_k_order(const TcDesc& d) {
+  if (d.K1 == 1 || (long long)d.K0 * d.K1 < 256) return d;
+  TcDesc x = d;
+  std::swap(x.K0, x.K1);
+  std::swap(x.ak0, x.ak1);
+  std::swap(x.bk0, x.bk1);
+  auto grade = [](const TcDesc& t) {
+    const int a = slab_reads(t.M0, t.am0, t.K0, t.K1, t.ak0), b = slab_reads(t.N0, t.bn0, t.K0, t.K1, t.bk0);
+    const bool a_larger = (long long)t.M0 * t.M1 > (long long)t.N0 * t.N1;
+    return 8 * (a + b) + (a_larger ? a : b);
+  };
+  return grade(x) > grade(d) ? x : d;
+}
+
 template <int MB, int NB, int AM>
 static void launch_slab_b(int bm, dim3 grid, const TcDesc& d, const double* A, const double* B, double* C, hipStream_t s) {
   const dim3 block(64 * SLAB_W);
@@ -1174,11 +1200,20 @@ static void launch_slab(const TcDesc& d, const double* A, const double* B, doubl
 // kernel / those: 576 x 576 x 64 5.0 / 6.5, 1024 x 1024 x 64 10.1 / 8.9, 1024 x 1024 x 256 15.8 / 18.6, 4096 x 512 x 512 47
 // / 51, 2048 x 2048 x 256 57 / 49); for a longer K a few tiles leave the chip idle, which the split along the grid fills
 // (96 x 96 x 8192 28 / 32, 16 x 16 x 16384 46 / 41).  Operands are addressed with 32-bit byte offsets.
+// For fewer than 32 tiles a long K is left to that split earlier where the loads are slower (time here / there, geometric
+// mean over sweeps of random sizes and orders): both operands along their rows, 8 or 16 bytes per row and k, from K = 3072
+// (1.05, worst 1.42; at 1536 .. 3072 0.87, with 32 tiles or more 0.77); one along K and one in odd runs of K or strided,
+// from 1536 (0.96, worst 1.69; below 0.49, worst 1.07); where neither has even runs, from 1536 at any number of tiles
+// (1.04, worst 1.75).  One such operand with 32 tiles or more stays here (0.67), and so do even runs along K (0.59).
 static bool slab_applies(const TcDesc& d, size_t bytes_a, size_t bytes_b) {
   const long long M = (long long)d.M0 * d.M1, N = (long long)d.N0 * d.N1, K = (long long)d.K0 * d.K1;
   const long long n = (M + 31) / 32 * ((N + 31) / 32) * d.batch;
-  return (n <= 512 || (n <= 2048 && K >= 256)) && K <= 8192 && bytes_a < (1ull << 32) &&
-         bytes_b < (1ull << 32);
+  if (!((n <= 512 || (n <= 2048 && K >= 256)) && K <= 8192 && bytes_a < (1ull << 32) && bytes_b < (1ull << 32))) return false;
+  if (K < 1536) return true;
+  const int a = slab_reads(d.M0, d.am0, d.K0, d.K1, d.ak0), b = slab_reads(d.N0, d.bn0, d.K0, d.K1, d.bk0);
+  const bool along_k = ((d.am0 != 1 || d.M0 == 1) && d.ak0 == 1) || ((d.bn0 != 1 || d.N0 == 1) && d.bk0 == 1);
+  if (!along_k) return K < 3072 || n >= 32 || a + b < 4;
+  return a + b == 4 || (a + b > 1 && n >= 32);
 }
 
 // Its tile: the one with the least estimated time, rounds over the 256 CUs times the cost of a tile (measured with every
@@ -1237,10 +1272,16 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
   dd.fm = FDiv((unsigned)d.M0);
   dd.fn = FDiv((unsigned)d.N0);
   dd.fk = FDiv((unsigned)d.K0);
-  if (p == Prec::F64 && slab_applies(d, bytes_a, bytes_b)) {
-    slab(dd, (const double*)A, (const double*)B, (double*)C, s);
-    TNAD_HIP_TRY(hipGetLastError());
-    return;
+  if (p == Prec::F64) {
+    TcDesc ds = slab_k_order(d);
+    if (slab_applies(ds, bytes_a, bytes_b)) {
+      ds.fm = dd.fm;
+      ds.fn = dd.fn;
+      ds.fk = FDiv((unsigned)ds.K0);
+      slab(ds, (const double*)A, (const double*)B, (double*)C, s);
+      TNAD_HIP_TRY(hipGetLastError());
+      return;
+    }
   }
   const long long K = (long long)d.K0 * d.K1;
   const long long tiles64 = (long long)grid.x * grid.y;
@@ -1248,8 +1289,8 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
   // output of at most 16 tiles with K up to 4096 (the k x k Gram products of the eigensolver, cut along
   // K below as well; for longer K the 64 x 64 tile's higher MFMA rate per slice wins)
   const dim3 grid32((unsigned)((M + 31) / 32), (unsigned)((N + 31) / 32), (unsigned)d.batch);
-  // (FP64 calls of these sizes went to tc_slab_kernel above)
-  const bool small = p != Prec::F64 && (long long)grid.x * grid.y * grid.z < TC_SMALL_BELOW && grid32.y <= 65535 &&
+  // (in FP64 what tc_slab_kernel left)
+  const bool small = (long long)grid.x * grid.y * grid.z < TC_SMALL_BELOW && grid32.y <= 65535 &&
                      (K < 256 || (tiles64 <= 16 && K <= 4096));
   if (small) grid = grid32;
   // split-K when the output tiles cannot fill the chip and K is long: about 512 workgroups,
@@ -1283,7 +1324,8 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
   if (!tc_vec_disabled()) {
     if (p == Prec::F64)
       vec = vbig ? launch_vec<double, 128, 16>(dd, grid_big, A, B, C, W, s)
-                 : !big && launch_vec<double, 64, 16>(dd, grid, A, B, C, W, s);
+                 : small ? launch_vec<double, 32, 32>(dd, grid, A, B, C, W, s)
+                         : !big && launch_vec<double, 64, 16>(dd, grid, A, B, C, W, s);
     else if (p == Prec::F32)
       vec = vbig ? launch_vec<float, 128, 16>(dd, grid_big, A, B, C, W, s)
                  : small ? launch_vec<float, 32, 32>(dd, grid, A, B, C, W, s)
@@ -1293,7 +1335,10 @@ void tc_launch(Ctx* c, Prec p, const TcDesc& d, const void* A, const void* B, vo
   }
   if (!vec) switch (p) {
     case Prec::F64:
-      if (big)
+      if (small)
+        hipLaunchKernelGGL((tc_kernel<double, TC_BK, 32>), grid, dim3(NT), 0, s, dd, (const double*)A,
+                           (const double*)B, (double*)C, (double*)W);
+      else if (big)
         hipLaunchKernelGGL((tc_kernel<double, TC_BK, 128>), grid_big, dim3(NT), 0, s, dd, (const double*)A,
                            (const double*)B, (double*)C, (double*)W);
       else if (deep)
